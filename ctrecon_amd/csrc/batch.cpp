@@ -320,10 +320,10 @@ void cache_store(const ctr_batch& B, const std::string& key) {
 }
 
 int autotune(ctr_batch& B) {
-  bool all64 = true;
+  bool one_column = true;
   int maxZN = 0;
   for (auto& c : B.scans) {
-    all64 = all64 && c->P->d.DNV == 64;
+    one_column = one_column && fp_lanes_log2(c->P->d.DNV) == 6;
     maxZN = std::max(maxZN, c->P->d.ZN);
   }
   // schedules: (grid, strided); grid 0 = one workgroup per item
@@ -331,7 +331,7 @@ int autotune(ctr_batch& B) {
   float best = 1e30f;
   bool bcolw = false;
   int bgrid = 0, bstr = 0, rc;
-  for (int cw = all64 ? 1 : 0; cw >= 0; --cw) {
+  for (int cw = one_column ? 1 : 0; cw >= 0; --cw) {
     B.colw = cw;
     if ((rc = build(B))) return rc;
     for (const auto& sc : sched) {

@@ -61,6 +61,7 @@ struct Dims {
   float beta0, dbeta_g;  // fan angle of boundary 0 and mean boundary spacing (adjoint guess)
   float B0, dB;          // row boundary index of row 0 and mean spacing (adjoint guess)
   float dBmin;           // smallest row spacing of the FP32 boundary table
+  float dBmax;           // largest row height (dBz)
 };
 
 // Host copies used by host-side accounting (cone voxel counts).
@@ -78,15 +79,16 @@ struct FpArgs {
   const TV* vol;
   TO* out;
   const ViewP* views;
-  const float2* bnd;
   const double2* bnd64;
   const float4* cols;
   const float* Bz;
+  const float* dBz;
   const float* h2;
   const float* invdB;
   const float* maskf;
   const float2* mext;
   Dims d;
+  int lg;  // lanes per item (log2)
   int vb, vs;
   const float* b;
   const float* invRow;
@@ -142,6 +144,7 @@ struct Plan {
   double2* bnd64 = nullptr;    // [PN][DNU+1]  the same in FP64 (forward projector, transpose)
   float4* cols = nullptr;      // [PN][DNU]    (r0, r1, G, Q)
   float* Bz = nullptr;         // [DNV+1]      (bz_v - z0)/dz
+  float* dBz = nullptr;        // [DNV]        row heights (bz_(v+1) - bz_v)/dz
   float* h2 = nullptr;         // [DNV]        (zds_v - z0)^2
   float* invdB = nullptr;      // [DNV]        1/(Bz[v+1]-Bz[v])
   double2* rot64 = nullptr;    // [PN]         (cos, sin) of the regularised view angle, FP64
@@ -191,6 +194,10 @@ int ensure_bytes(void** p, size_t* have, size_t need, const char* what);
 // partials (2 fp_partial_blocks(P, chunk) doubles) and sums (kResidualSums doubles) as
 // scratch, on stream st; synchronous.  Allocates nothing for the direct method.
 constexpr int kResidualSums = 128;
+// Views per chunk of both residual entry points (the same chunks give the same sums): at
+// most 256, fewer where their partial sums would exceed kResidualScratch doubles.
+constexpr long long kResidualScratch = 1ll << 19;
+int residual_chunk(const Plan& P);
 int residual_run(Plan& P, const float* d_x, const float* d_prj, float* prj, int chunk,
                  double* partials, double* sums, hipStream_t st, double* out);
 
@@ -229,6 +236,7 @@ template <typename T>
 BpArgs<T> bp_args(const Plan& P, const T* prj, float* vol, int vb, int vs, int vc,
                   const float* invCol, uint16_t* shadow);
 int fp_blocks_per_view(const Plan& P, bool colw);
+int fp_lanes_log2(int DNV);
 // batched launches: grid = number of persistent workgroups (<= 0: one per work item),
 // strided = interleaved instead of contiguous item ranges
 template <typename T>

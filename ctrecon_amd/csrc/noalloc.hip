@@ -17,11 +17,8 @@ namespace {
 // The scratch: the per-workgroup partial sums of one view chunk (2 doubles per workgroup
 // of the fused forward projector), then kResidualSums doubles of per-chunk totals.  4 MiB;
 // every GPU the library runs on holds its own copy until the process ends.
-constexpr size_t kScratchDoubles = size_t(1) << 19;
+constexpr size_t kScratchDoubles = (size_t)kResidualScratch;
 static __device__ __align__(256) double scratch[kScratchDoubles];
-
-// The views of one chunk, as ctr_residual (the same chunks give the same sums, bit for bit).
-constexpr int kChunkViews = 256;
 
 // Device address of each GPU's copy of scratch, looked up once per device (with that
 // device current) on its first call; host code uses only these addresses, never the
@@ -59,15 +56,20 @@ int ctr_residual_noalloc(ctr_plan* plan, const float* d_x, const float* d_prj, d
                 "ctr_residual_noalloc: the direct method only (the integral-image method "
                 "builds its tables in plan memory)");
   CTR_HIP(hipSetDevice(P->device));
-  const int chunk = std::min(P->d.PN, kChunkViews);
-  const size_t parts = 2 * (size_t)fp_partial_blocks(*P, chunk);
-  if (parts + kResidualSums > kScratchDoubles)
+  // the detectors taken: 2 doubles per 256 rays of up to 256 views
+  const size_t most = 2 * (((size_t)P->d.DNU * P->d.DNV + 255) / 256) * std::min(P->d.PN, 256);
+  if (most + kResidualSums > kScratchDoubles)
     return fail(CTR_ERR_ARG,
-                "ctr_residual_noalloc: a chunk of " + std::to_string(chunk) + " views of " +
+                "ctr_residual_noalloc: " + std::to_string(std::min(P->d.PN, 256)) + " views of " +
                     std::to_string(P->d.DNU) + " x " + std::to_string(P->d.DNV) +
-                    " rays needs " + std::to_string(parts + kResidualSums) +
+                    " rays need " + std::to_string(most + kResidualSums) +
                     " doubles of scratch; the maximum is " + std::to_string(kScratchDoubles) +
                     " (4 MiB): use ctr_residual");
+  const int chunk = residual_chunk(*P);
+  const size_t parts = 2 * (size_t)fp_partial_blocks(*P, chunk);
+  if (parts + kResidualSums > kScratchDoubles)
+    return fail(CTR_ERR_ARG, "ctr_residual_noalloc: one view's partial sums exceed the 4 MiB "
+                             "scratch: use ctr_residual");
   double* s = nullptr;
   if (int rc = scratch_on(P->device, &s)) return rc;
   // every partial slot and every total is written before it is read: nothing to clear

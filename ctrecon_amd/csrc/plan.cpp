@@ -141,17 +141,20 @@ static int build_tables(const ctr_geometry* g, Plan& P, double half = 0.0) {
                             bz = boundaries(g->zds, DNV);
 
   // rows
-  std::vector<float> Bz(DNV + 1), h2(DNV), invdB(DNV);
+  std::vector<float> Bz(DNV + 1), dBz(DNV), h2(DNV), invdB(DNV);
   for (int v = 0; v <= DNV; ++v) Bz[v] = (float)((bz[v] - z0) / dz);
   for (int v = 0; v < DNV; ++v) {
     const double h = g->zds[v] - z0;
     h2[v] = (float)(h * h);
     invdB[v] = (float)(dz / (bz[v + 1] - bz[v]));
+    dBz[v] = (float)((bz[v + 1] - bz[v]) / dz);
   }
   d.B0 = Bz[0];
   d.dB = (float)((bz[DNV] - bz[0]) / dz / DNV);
   d.dBmin = Bz[1] - Bz[0];
   for (int v = 1; v < DNV; ++v) d.dBmin = std::min(d.dBmin, Bz[v + 1] - Bz[v]);
+
+  d.dBmax = *std::max_element(dBz.begin(), dBz.end());
 
   // fan angles of the column boundaries seen from the source (rotation invariant)
   const double sid = std::sqrt(x0 * x0 + y0 * y0);
@@ -310,6 +313,7 @@ static int build_tables(const ctr_geometry* g, Plan& P, double half = 0.0) {
   if ((rc = upload(&P.bnd64, bnd64))) return rc;
   if ((rc = upload(&P.cols, cols))) return rc;
   if ((rc = upload(&P.Bz, Bz))) return rc;
+  if ((rc = upload(&P.dBz, dBz))) return rc;
   if ((rc = upload(&P.h2, h2))) return rc;
   if ((rc = upload(&P.invdB, invdB))) return rc;
   if ((rc = upload(&P.mask, mask))) return rc;
@@ -329,6 +333,7 @@ static void free_plan(Plan* P) {
   (void)hipFree(P->bnd64);
   (void)hipFree(P->cols);
   (void)hipFree(P->Bz);
+  (void)hipFree(P->dBz);
   (void)hipFree(P->h2);
   (void)hipFree(P->invdB);
   (void)hipFree(P->mask);
@@ -490,6 +495,12 @@ struct DBuf {
   double* d() const { return (double*)p; }
   uint16_t* h() const { return (uint16_t*)p; }
 };
+
+int residual_chunk(const Plan& P) {
+  const int views = std::min(P.d.PN, 256);
+  const long long most = (kResidualScratch - kResidualSums) / 2 / fp_partial_blocks(P, 1);
+  return (int)std::max<long long>(1, std::min<long long>(views, most));
+}
 
 int residual_run(Plan& P, const float* d_x, const float* d_prj, float* prj, int chunk,
                  double* partials, double* sums, hipStream_t st, double* out) {
@@ -738,7 +749,7 @@ int ctr_residual(ctr_plan* plan, const float* d_x, const float* d_prj, double* o
   if (int rc0 = check_solver_method(*P)) return rc0;
   CTR_HIP(hipSetDevice(P->device));
   // chunk the views so the scratch stays modest
-  const int chunk = std::min(P->d.PN, 256);
+  const int chunk = residual_chunk(*P);
   int rc = ensure_scratch_prj(*P, chunk);
   if (rc) return rc;
   if ((rc = ensure_partials(*P, 2 * (size_t)fp_partial_blocks(*P, chunk) + 2))) return rc;
