@@ -77,10 +77,10 @@ struct ctr_batch {
   Mem bpItems[5], tuneBpItems[5];
   std::vector<int> bpTotal[5];
   int winZ = 0;    // tallest column of the windowed class
-  int winDNV = 0;  // most detector rows of a scan of the windowed class
+  int winRC = 0;   // row chunks of the windowed class (bp_row_chunks)
   bool colw = false;
-  // zg: z groups per lane for every scan (1..4), 0 for each scan's own ceil(ZN / 64), or
-  // kZgWindow for the windowed form (scans with columns taller than kWinMaxZ: their own)
+  // zg: z groups per lane (1..4; 0 and kZgWindow: each scan's own ceil(ZN / 64)) of the scans
+  // with columns taller than kWinMaxZ; every other scan runs the windowed form
   int fpGrid = 0, zg = 0, bpGrid = 0;  // grids: persistent workgroups, <= 0 one per item
   int fpStrided = 0, bpStrided = 0;
   hipStream_t st = nullptr;
@@ -102,7 +102,7 @@ constexpr int kZgWindow = 5;
 
 // back-projection class of a scan (0: windowed)
 int scan_zg(const ctr_batch& B, const Plan& P) {
-  if (B.zg == kZgWindow && P.d.ZN <= kWinMaxZ) return 0;
+  if (P.d.ZN <= kWinMaxZ) return 0;  // the windowed form, whatever zg
   return (B.zg > 0 && B.zg < kZgWindow) ? B.zg : std::min(4, (P.d.ZN + 63) / 64);
 }
 
@@ -118,15 +118,19 @@ int build_tables(ctr_batch& B) {
     B.bpTotal[c].assign(S, 0);
   }
   B.winZ = 0;
-  B.winDNV = 0;
+  bool staged = true;
+  B.winRC = 0;
   for (int i = 0; i < n; ++i) {
     const int c = scan_zg(B, *B.scans[i]->P);
     B.clsScans[c].push_back(i);
     if (c == 0) {
       B.winZ = std::max(B.winZ, B.scans[i]->P->d.ZN);
-      B.winDNV = std::max(B.winDNV, B.scans[i]->P->d.DNV);
+      const int rc = bp_row_chunks(B.scans[i]->P->d.DNU, B.scans[i]->P->d.DNV);
+      staged = staged && rc > 0;
+      B.winRC = std::max(B.winRC, rc);
     }
   }
+  if (!staged) B.winRC = 0;
   auto up = [&](Mem& m, const void* src, size_t bytes) -> int {
     if (m.p) {
       (void)hipFree(m.p);
@@ -203,7 +207,7 @@ int step_bp(ctr_batch& B, int s, bool tuning) {
     const Mem& mem = tuning ? B.tuneBpItems[cz] : B.bpItems[cz];
     const BpBatchItem<T>* items = (const BpBatchItem<T>*)mem.p + (size_t)s * m;
     int rc = cz == 0 ? launch_bp_batch_win<T>(items, (int)m, B.bpTotal[0][s], B.winZ,
-                                              B.winDNV, B.bpGrid, B.bpStrided, B.st)
+                                              B.winRC, B.bpGrid, B.bpStrided, B.st)
                      : launch_bp_batch<T>(items, (int)m, B.bpTotal[cz][s], cz, B.bpGrid,
                                           B.bpStrided, B.st);
     if (rc) return rc;
@@ -357,7 +361,8 @@ int autotune(ctr_batch& B) {
   bstr = 0;
   const int zgs[5] = {kZgWindow, 0, 1, 2, 4};  // 0: each scan's own ceil(ZN / 64)
   for (int zg : zgs) {
-    if (zg > 1 && 64 * (zg / 2) >= maxZN) break;  // more groups than any column needs
+    if (zg != kZgWindow && maxZN <= kWinMaxZ) break;  // no column runs in z groups
+    if (zg > 1 && 64 * (zg / 2) >= maxZN) break;      // more groups than any column needs
     B.zg = zg;
     if ((rc = build(B))) return rc;
     for (const auto& sc : sched) {

@@ -62,6 +62,9 @@ struct Dims {
   float B0, dB;          // row boundary index of row 0 and mean spacing (adjoint guess)
   float dBmin;           // smallest row spacing of the FP32 boundary table
   float dBmax;           // largest row height (dBz)
+  double B0_64, dB_64;   // row boundary 0 and the mean spacing, FP64
+  int even_rows;         // 1: every row boundary is B0 + v dB to within the FP32 rounding of
+                         // the given row positions
 };
 
 // Host copies used by host-side accounting (cone voxel counts).
@@ -246,10 +249,12 @@ template <typename T>
 int launch_bp_batch(const BpBatchItem<T>* items, int nscan, int total, int zg, int grid,
                     int strided, hipStream_t st);
 // windowed form: one work item per block of 4 columns over all z; zmax = tallest column,
-// maxDNV = most detector rows of a scan in the list
+// rc = the row chunks of its staged waves (bp_row_chunks; 0 when a scan needs the unstaged
+// form)
+int bp_row_chunks(int DNU, int DNV);
 template <typename T>
-int launch_bp_batch_win(const BpBatchItem<T>* items, int nscan, int total, int zmax,
-                        int maxDNV, int grid, int strided, hipStream_t st);
+int launch_bp_batch_win(const BpBatchItem<T>* items, int nscan, int total, int zmax, int rc,
+                        int grid, int strided, hipStream_t st);
 int launch_reduce_batch(const ReduceItem* items, int nscan, hipStream_t st);
 int launch_to_bf16(uint16_t* dst, const float* src, size_t n, hipStream_t st);
 // the solvers' dithered BF16 shadow of an iterate (to_bf16_dither)

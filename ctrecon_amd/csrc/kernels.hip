@@ -107,6 +107,7 @@ struct Overlap3 {
 };
 template <int NT>
 __device__ __forceinline__ Overlap3 overlap3(float t, float h) {
+#pragma clang fp contract(off)
   Overlap3 o;
   const float fr = __builtin_amdgcn_fractf(t);
   const float a = 1.f - fr;
@@ -170,8 +171,15 @@ __device__ __forceinline__ void z_run(const Buf<uint16_t>&, const uint16_t* vol,
 // Groups (fewer than 64 rows to a column) gather each cell's taps as one load per lane:
 // 64^3, 720 views of 256 x 16, 212 us one thread per ray with its own FP64 footprints,
 // 85 us with four columns per wave.
-template <bool FUSED, bool COLW, typename TV, typename TO>
+//
+// ONES: the projection of a volume of ones (the row sums of OS-SART), read from no volume.
+// A slice wholly inside the volume's z range adds its height times its cells' weights; the
+// others take the weights of the projection itself, so that a ray that grazes the volume by
+// a rounding error has a row sum that matches its projection (no contraction: the
+// instantiations must not round a footprint differently).
+template <bool FUSED, bool COLW, typename TV, typename TO, bool ONES = false>
 __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk, double* slot) {
+#pragma clang fp contract(off)
   const Dims& d = A.d;
   const int p = A.vb + k * A.vs;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -228,7 +236,7 @@ __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk
         const float wy = ((ij == 0) ? o.wj0 : (ij == o.nj - 1 ? o.wjl : 1.f)) * maskf[mo];
         float g = 0.f;
         for (int ik = 0; ik < nk; ++ik)
-          g = fmaf((ik == 0) ? wf : (ik == nk - 1 ? wl : 1.f), V[e + ik], g);
+          g = fmaf((ik == 0) ? wf : (ik == nk - 1 ? wl : 1.f), ONES ? 1.f : (float)V[e + ik], g);
         s = fmaf(wy, g, s);
         e += cS;
         mo += mC;
@@ -317,6 +325,7 @@ __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk
           if (!m) return;
           // the slice's z run of every cell, one element per lane (stored bits)
           auto fetch = [&](int j, uint32_t(&a)[NJ][NZ]) {
+            if constexpr (ONES) return;
             const int e = __builtin_amdgcn_readlane(q_e, j);
             // lanes past the last cell re-read it, so that they touch no further cache lines
             // (FP32, 512^2 x 256: 2.37 ms against 2.50 ms unclamped; the first 64 BF16 cells
@@ -336,11 +345,19 @@ __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk
             const int kb = __builtin_amdgcn_readlane(q_kb, j);
             float wy[4] = {q.y, q.z, q.w, 0.f};
             if constexpr (NJ == 4) wy[3] = rdl(wy3, j);
+            if constexpr (ONES && !EDGE) {
+              float W = wy[0];
+#pragma unroll
+              for (int ij = 1; ij < NJ; ++ij) W += wy[ij];
+              acc = fmaf(q.x * dBv, W, acc);
+              return;
+            }
 #pragma unroll
             for (int h = 0; h < NZ; ++h) {
-              float R = wy[0] * Buf<TV>::widen(a[0][h]);
+              float R = wy[0] * (ONES ? 1.f : Buf<TV>::widen(a[0][h]));
 #pragma unroll
-              for (int ij = 1; ij < NJ; ++ij) R = fmaf(wy[ij], Buf<TV>::widen(a[ij][h]), R);
+              for (int ij = 1; ij < NJ; ++ij)
+                R = fmaf(wy[ij], ONES ? 1.f : Buf<TV>::widen(a[ij][h]), R);
               if constexpr (EDGE)
                 R = (uint32_t)(kb + vp.azi + lane + 64 * h) < (uint32_t)d.ZN ? R : 0.f;
               zrun[lane + 64 * h] = R;
@@ -400,6 +417,10 @@ __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk
             const float4 q = rec[gbase + j];
             const int4 f = off[gbase + j];
             float t = fmaf(q.x, Bv, azf), h = q.x * dBv;
+            if constexpr (ONES && !EDGE) {
+              acc = fmaf(h, (q.y + q.z) + (q.w + __int_as_float(f.z)), acc);
+              continue;
+            }
             if constexpr (EDGE) {
               const float te = __builtin_elementwise_minimum(t + h, tmax);
               t = __builtin_elementwise_maximum(t, tmin);
@@ -414,7 +435,8 @@ __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk
             if (f.y == 0) e = 0;
 #pragma unroll
             for (int ij = 0; ij < NJ; ++ij) {
-              z_run<NT>(V, A.vol, e, a[ij]);
+              if constexpr (ONES) a[ij][0] = a[ij][1] = a[ij][2] = 1.f;
+              else z_run<NT>(V, A.vol, e, a[ij]);
               if (ij + 1 < f.y) e += cS;
             }
             float s = 0.f;
@@ -464,70 +486,6 @@ __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk
   if constexpr (FUSED) block_sum2(res, bsq, slot);
 }
 
-// The projection of a volume of ones (the row sums of OS-SART), read from no volume: the z
-// weights of a footprint sum to its clipped height zh - zl, so a slice adds
-// (zh - zl) * sum_j wy_j mask_j (the sum of fp_body in another rounding order).  One thread
-// per ray; COLW (DNV == 64): a wave is exactly one detector column, lane l evaluates the
-// in-plane part of slice ii0 + l, with the sum W of its cells' edge weights times mask
-// bytes, read back with readlane.
-template <bool COLW>
-__device__ __forceinline__ void fp_ones_body(const FpArgs<float, float>& A, int k, int ublk) {
-  const Dims& d = A.d;
-  const int p = A.vb + k * A.vs;
-  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int ray =
-      COLW ? (ublk * kWaves + wid) * 64 + (threadIdx.x & 63) : ublk * kBlock + threadIdx.x;
-  if (ray >= d.DNU * d.DNV) return;
-  const int u = COLW ? (ublk * kWaves + wid) : ray / d.DNV;
-  const int v = ray - u * d.DNV;
-  const ViewP vp = gload(A.views, p);
-  const double2 bl = gload(A.bnd64, (size_t)p * (d.DNU + 1) + u);
-  const double2 br = gload(A.bnd64, (size_t)p * (d.DNU + 1) + u + 1);
-  const float4 ct = gload(A.cols, (size_t)p * d.DNU + u);
-  const float Bv = gp(A.Bz)[v], Bv1 = gp(A.Bz)[v + 1];
-  const int NS = vp.xmarch ? d.XN : d.YN, NI = vp.xmarch ? d.YN : d.XN;
-  const int mS = vp.xmarch ? 1 : d.XN, mC = vp.xmarch ? d.XN : 1;
-  // z in cell-index units relative to azi (exact shifts of the volume's bounds)
-  const float zlo_b = -0.5f - (float)vp.azi, zhi_b = ((float)d.ZN - 0.5f) - (float)vp.azi;
-  const float2* me = A.mext + (vp.xmarch ? 0 : d.XN);
-  const CTR_GLOBAL float* maskf = gp(A.maskf);
-  float acc = 0.f;
-  auto weight = [&](const SliceIP& o, int ii) {
-    float W = 0.f;
-    for (int ij = 0; ij < o.nj; ++ij)
-      W = fmaf((ij == 0) ? o.wj0 : (ij == o.nj - 1 ? o.wjl : 1.f),
-               maskf[ii * mS + (o.j0 + ij) * mC], W);
-    return W;
-  };
-  auto add = [&](float r, float W, float inv) {
-    const float zl = fmaxf(fmaf(r, Bv, vp.azf), zlo_b), zh = fminf(fmaf(r, Bv1, vp.azf), zhi_b);
-    if (zl < zh) acc = fmaf((zh - zl) * W, inv, acc);
-  };
-  if constexpr (COLW) {
-    const int lane = threadIdx.x & 63;
-    for (int ii0 = 0; ii0 < NS; ii0 += 64) {
-      const int il = ii0 + lane;
-      float q_W = 0.f;
-      SliceIP si{};
-      const bool ok = il < NS && fp_inplane(bl, br, ct, gload(me, il), il, NI, si);
-      if (ok) q_W = weight(si, il);
-      uint64_t live = __ballot(ok);
-      while (live) {
-        const int j = __builtin_ctzll(live);
-        live &= live - 1;
-        add(rdl(si.r, j), rdl(q_W, j), rdl(si.inv, j));
-      }
-    }
-  } else {
-    for (int ii = 0; ii < NS; ++ii) {
-      SliceIP si;
-      if (fp_inplane(bl, br, ct, gload(me, ii), ii, NI, si)) add(si.r, weight(si, ii), si.inv);
-    }
-  }
-  const float K = ct.w * __builtin_amdgcn_sqrtf(ct.z + gp(A.h2)[v]) * gp(A.invdB)[v];
-  gp(A.out)[((size_t)k * d.DNU + u) * d.DNV + v] = acc * K;
-}
-
 template <bool FUSED, bool COLW, typename TV, typename TO>
 __global__ __launch_bounds__(kBlock) void fp_kernel(FpArgs<TV, TO> A, int bpv, int views) {
   const int hw = blockIdx.x;
@@ -539,11 +497,12 @@ __global__ __launch_bounds__(kBlock) void fp_kernel(FpArgs<TV, TO> A, int bpv, i
 
 // Forward projection of a volume of ones (A.vol unused).
 template <bool COLW>
-__global__ __launch_bounds__(kBlock) void fp_ones_kernel(FpArgs<float, float> A) {
-  const int hw = blockIdx.y * gridDim.x + blockIdx.x;
-  const int lb = xcd_logical_block(hw, gridDim.x * gridDim.y);
-  const int k = lb / gridDim.x;
-  fp_ones_body<COLW>(A, k, lb - k * gridDim.x);
+__global__ __launch_bounds__(kBlock) void fp_ones_kernel(FpArgs<float, float> A, int bpv,
+                                                         int views) {
+  const int lb = xcd_chunked_block(blockIdx.x);
+  const int k = lb / bpv;
+  if (k >= views) return;
+  fp_body<false, COLW, float, float, true>(A, k, lb - k * bpv, nullptr);
 }
 
 // Batched persistent forward projection: each workgroup takes one contiguous range of
@@ -635,6 +594,7 @@ __global__ __launch_bounds__(kBlock) void fp_batch1_kernel(const FpBatchItem<T>*
 // the row-shadow constants (rows of a voxel at dZ = Pz - sz: [dZ rlS + cA, dZ rlS + cB]).
 struct BpView {
   float rlS, cA, cB, sz, l2, cws, wu0, fh;
+  double rl;
   int u0, nu;
   bool uvis;
 };
@@ -657,6 +617,7 @@ __device__ __forceinline__ BpView bp_view(const BpArgs<T>& A, int p, double Px, 
   const double dX = Px - s64.x, dY = Py - s64.y;
   const double l2 = dX * dX + dY * dY;
   const double rl = rsqrt(l2);
+  r.rl = rl;
   const double alpha = asin_fan((s64.y * Px - s64.x * Py) * c64.inv_sid * rl);
   const double w = vp.wx ? dX : dY;
   const double dA = w * (rl * rl) * (c64.dx * 0.5);
@@ -777,53 +738,6 @@ __device__ __forceinline__ float bp_cell_sum(const Buf<T>& pp, int u0, int nu, f
   return s;
 }
 
-// Staged windowed back projector (DNV <= kStageRows): per wave, the current view's
-// combined rows (kStagePad floats: two rows of zeros past the last row for taps there),
-// then a table of 64 view records (kRecF floats each: row-shadow constants, cosVal
-// constants and the four column weights, written by lane l for view k0 + l).  kStageF
-// floats per wave, a multiple of 4 so every wave's table is 16-byte aligned.
-constexpr int kStageRows = 64;
-constexpr int kStagePad = kStageRows + 2;
-constexpr int kRowsF = kStagePad + 2;  // rows, then the record table 16-byte aligned
-constexpr int kRecF = 12;
-constexpr int kStageF = kRowsF + 64 * kRecF;
-// staged waves' column sums carry 64 floats past the column: a pass's lanes past the
-// column's end (whose shadows need not be empty) add there, and the passes need no
-// per-voxel bound test
-constexpr int kLaccPad = 64;
-static_assert(kRowsF % 4 == 0 && kStageF % 4 == 0, "per-wave stage: 16-byte multiples");
-
-// bp_cell_sum over a view whose columns are already combined per row in LDS
-// (lR[v] = sum_u wu y[u][v], rows past DNV zero, two zero rows past the stage), with the
-// same sum: the row weights min(vhi, e) - vlo, clamp(d, 0, 1), clamp(d - 1, 0, 1) of a
-// shadow over at most three rows are exactly the first / interior / last weights of
-// edge_weights (d = vhi - e and d - 1 are exact differences), and taps past the shadow
-// add exact zeros (the third row's is added in every pass: most passes have a lane that
-// needs it), so the choice between the two forms may be made for the whole wave.
-__device__ __forceinline__ float bp_lds_sum(const float* lR, float vlo, float vhi, int DNV) {
-#pragma clang fp contract(off)
-  const float fv = floorf(vlo + 0.5f);
-  const float e = fv + 0.5f;
-  const int v0 = (int)fv;
-  const float d = vhi - e;
-  float s;
-  if (!__any(d > 2.f)) {
-    const float wv0 = __builtin_elementwise_minimum(vhi, e) - vlo;
-    const float wv1 = __builtin_amdgcn_fmed3f(d, 0.f, 1.f);
-    s = wv0 * lR[v0];
-    s = fmaf(wv1, lR[v0 + 1], s);
-    s = fmaf(__builtin_amdgcn_fmed3f(d - 1.f, 0.f, 1.f), lR[v0 + 2], s);
-  } else {
-    const int nv = min((int)floorf(vhi + 0.5f), DNV - 1) - v0 + 1;
-    float wv0, wvl;
-    edge_weights(vlo, vhi, v0, nv, wv0, wvl);
-    s = 0.f;
-    for (int iv = 0; iv < nv; ++iv)
-      s = fmaf((iv == 0) ? wv0 : (iv == nv - 1 ? wvl : 1.f), lR[v0 + iv], s);
-  }
-  return s;
-}
-
 // Final value of voxel z of a column: vol = acc, or the OS-SART update
 // vol += acc * invCol (and its BF16 shadow).
 template <bool UPDATE, typename T>
@@ -915,29 +829,246 @@ __device__ __forceinline__ void bp_ref_body(const BpArgs<T>& A, int col, int zbl
   }
 }
 
+// Voxels of a column that view q's row shadow can reach: those with
+// fmaf(dZ, rlS, cB) > -0.5 and fmaf(dZ, rlS, cA) < DNV - 0.5 lie in an open interval of
+// voxel indices whose FP32 ends are within ~1e-4 of it, so the integers inside it widened
+// by 1e-2 include every one of them.
+__device__ __forceinline__ void bp_window(const Dims& d, const BpView& q, int& z0, int& z1) {
+  const float DNVh = (float)d.DNV - 0.5f, ZNf = (float)d.ZN, idz = 1.f / d.dz;
+  const float ea = (-0.5f - q.cB) / q.rlS, eb = (DNVh - q.cA) / q.rlS;
+  const float za = fminf(fmaxf((fminf(ea, eb) + q.sz) * idz + d.ocz, -4.f), ZNf + 4.f);
+  const float zb = fminf(fmaxf((fmaxf(ea, eb) + q.sz) * idz + d.ocz, -4.f), ZNf + 4.f);
+  z0 = max((int)floorf(za - 1e-2f) + 1, 0);
+  z1 = min((int)ceilf(zb + 1e-2f) - 1, d.ZN - 1);
+}
+
+// Runs f(slot, j) ... over the set bits j of m with the fetches of the next bit in flight:
+// fetch(j, set) loads into one of two register sets, use(j, set) consumes it.
+template <typename Set, typename Fetch, typename Use>
+__device__ __forceinline__ void pipelined(uint64_t m, Fetch fetch, Use use) {
+  Set x0, x1;
+  int j0 = __builtin_ctzll(m), j1;
+  m &= m - 1;
+  fetch(j0, x0);
+  while (true) {
+    if (!m) {
+      use(j0, x0);
+      break;
+    }
+    j1 = __builtin_ctzll(m);
+    m &= m - 1;
+    fetch(j1, x1);
+    use(j0, x0);
+    if (!m) {
+      use(j1, x1);
+      break;
+    }
+    j0 = __builtin_ctzll(m);
+    m &= m - 1;
+    fetch(j0, x0);
+    use(j1, x1);
+  }
+}
+
 // Windowed form of bp_ref_body: one wave per voxel column over all of its z.  On a
 // helical scan a view's cone covers a window of a few dozen voxels of a column, which
-// the fixed lane -> z groups above cover with one 64-lane pass per group it touches
-// (about half the lanes idle).  Here the lanes take the view's own window, z0 + lane,
-// z0 + 64 + lane, ... (z0, z1: the voxels of the row shadow's open interval, with a
-// 1e-2-voxel margin; the per-voxel test decides), and the column's sums live in LDS
-// (lacc: ZN floats of this wave), each
-// updated by one lane per view, views in order.  Per-voxel arithmetic as bp_ref_body.
-// ONES: the back projection of a sinogram of ones (the column sums of OS-SART), read
-// from no sinogram: the row weights of a shadow sum to its clipped height vhi - vlo and
-// the column weights to Wu = wu0 + (nu - 2) + fh (wu0 alone for one column), so a voxel
-// adds cosVal * Wu * (vhi - vlo) (the same sum in another rounding order).
+// fixed lane -> z groups cover with one 64-lane pass per group it touches (about half the
+// lanes idle).  Here the lanes take the view's own window, z0 + lane, z0 + 64 + lane, ...,
+// and the column's sums live in LDS.
 //
-// stg (kStageF floats of this wave, 16-byte aligned, or NULL): with DNV <= kStageRows the
-// views are staged (lacc then holds ZN + kLaccPad floats).  Lane l writes view k0 + l's record (row-shadow and cosVal constants,
-// column weights) to the wave's table; then, visible view by visible view, every lane
-// loads its row of the view's first four columns (issued while the previous view's voxels
-// are summed), combines them (R[v] = sum_u wu y[u][v], the column order and rounding of
-// bp_cells) into LDS, and the voxels of the window read two or three values of R there;
-// the sums are those of the direct gathers, bit for bit.
+// Staged rows (DNV <= 64 RC, RC = 1, 2, 4): 64 views at a time, lane l evaluates view
+// k0 + l (fan-angle shadow in FP64, column weights times cosVal's width factor, the row
+// shadow T(z) = T0 + (z - z0) s of its window in units of rows, row edges at integers) into
+// the wave's LDS records and sorts the view into a class by its number of columns and of
+// 64-voxel passes.  Each class runs its views in a loop of straight-line code: every lane
+// loads its row of the view's columns (the next view's rows load meanwhile) and combines
+// them (R[v] = sum_u w_u y[u][v]) into LDS, four rows of zeros on either side, and a voxel
+// takes the three rows that its shadow [T, T + s] can overlap, without clamps.
+constexpr int kPadRows = 4;
+template <int RC>
+constexpr int kRowsLds = 64 * RC + 3 * kPadRows;  // zeros, rows, zeros, a slot for idle lanes
+template <int RC>
+constexpr int kStagedF = kRowsLds<RC> + 64 * 8;   // floats of a staged wave before its sums
+
+// Rows of a staged wave: the zero rows written once, and each lane's slot for row
+// lane + 64 c (idle lanes write to a slot that is never read).
+template <int RC>
+__device__ __forceinline__ void stage_rows(float* rows, int DNV, int lane, int (&row)[RC],
+                                           int (&slot)[RC]) {
+  if (lane < kPadRows) {
+    rows[lane] = 0.f;
+    rows[kPadRows + DNV + lane] = 0.f;
+  }
+#pragma unroll
+  for (int c = 0; c < RC; ++c) {
+    const int v = lane + 64 * c;
+    row[c] = min(v, DNV - 1);
+    slot[c] = v < DNV ? v + kPadRows : 64 * RC + 2 * kPadRows;
+  }
+}
+
+//
+// ONES: the back projection of a sinogram of ones (the column sums of OS-SART), read from no
+// sinogram, with the weights of the back projection itself: a voxel that a shadow grazes by a
+// rounding error then has a column sum that matches its update.
+template <bool UPDATE, typename T, int RC, bool ONES = false>
+__device__ __forceinline__ void bp_staged_body(const BpArgs<T>& A, int col, float* lds) {
+#pragma clang fp contract(off)
+  const Dims& d = A.d;
+  const BpConsts64& c64 = A.c64;
+  const int lane = threadIdx.x & 63;
+  if (col >= d.XN * d.YN) return;
+  const int y = col / d.XN, x = col - y * d.XN;
+  CTR_GLOBAL float* vcol = gp(A.vol) + (size_t)col * d.ZN;
+  if (gp(A.mask)[col] != 1) {
+    if constexpr (!UPDATE) {
+      for (int z = lane; z < d.ZN; z += 64) vcol[z] = 0.f;
+    }
+    return;
+  }
+  float* rows = lds;
+  float4* rec = reinterpret_cast<float4*>(lds + kRowsLds<RC>);  // [64][2]
+  float* lacc = lds + kStagedF<RC>;
+  for (int z = lane; z < d.ZN; z += 64) lacc[z] = 0.f;
+  const int DNV = d.DNV;
+  int row[RC], slot[RC];
+  stage_rows<RC>(rows, DNV, lane, row, slot);
+  const double Px = ((double)x - c64.ocx) * c64.dx;
+  const double Py = ((double)y - c64.ocy) * c64.dx;
+  const float Pxf = (float)Px, Pyf = (float)Py;
+  const int frame = d.DNU * DNV;
+  const float lanef = (float)lane;
+  for (int k0 = 0; k0 < A.vc; k0 += 64) {
+    const int kl = k0 + lane;
+    int z0 = 0, z1 = -1, q_o = 0, key = 0;
+    if (kl < A.vc) {
+      const BpView q = bp_view(A, A.vb + kl * A.vs, Px, Py, Pxf, Pyf);
+      bp_window(d, q, z0, z1);
+      if (q.uvis && z0 <= z1) {
+        // row shadow of the window's first voxel and its step, dZ of that voxel
+        const double rlS = q.rl * c64.S, dz = (double)d.dz;
+        const double dZ = ((double)z0 - c64.ocz) * dz - (double)q.sz;
+        const float s = (float)(dz * rlS);
+        const float T0 = (float)((dZ - 0.5 * dz) * rlS + (c64.cV + 0.5));
+        const int nu = q.nu;
+        rec[2 * lane] = make_float4(T0, s, (float)dZ, q.l2);
+        rec[2 * lane + 1] = make_float4(
+            q.cws * q.wu0, nu > 1 ? q.cws * (nu == 2 ? q.fh : 1.f) : 0.f,
+            nu > 2 ? q.cws * (nu == 3 ? q.fh : 1.f) : 0.f, nu > 3 ? q.cws * q.fh : 0.f);
+        q_o = lane * frame + q.u0 * DNV;
+        // the class: columns * 2 + (more than one pass); 1 the general form
+        key = nu > 4 || s > 2.f ? 1 : 2 * nu + (z1 - z0 >= 64 ? 1 : 0);
+      }
+    }
+    if (!__any(key)) continue;
+    const Buf<T> P(A.prj + (size_t)k0 * frame, (uint32_t)min(64, A.vc - k0) * (uint32_t)frame);
+    auto run = [&](auto NU_, auto MULTI_) {
+      constexpr int NU = decltype(NU_)::value;
+      constexpr bool MULTI = decltype(MULTI_)::value;
+      const uint64_t m = __ballot(key == 2 * NU + (MULTI ? 1 : 0));
+      if (!m) return;
+      struct Set {
+        uint32_t y[NU][RC];
+      };
+      pipelined<Set>(
+          m,
+          [&](int j, Set& f) {
+            if constexpr (ONES) return;
+            const int o = __builtin_amdgcn_readlane(q_o, j);
+#pragma unroll
+            for (int iu = 0; iu < NU; ++iu)
+#pragma unroll
+              for (int c = 0; c < RC; ++c) f.y[iu][c] = P.at_bits(row[c], o + iu * DNV);
+          },
+          [&](int j, const Set& f) {
+            const float4 r = rec[2 * j], w = rec[2 * j + 1];
+            const float wu[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+            for (int c = 0; c < RC; ++c) {
+              float R = wu[0] * (ONES ? 1.f : Buf<T>::widen(f.y[0][c]));
+#pragma unroll
+              for (int iu = 1; iu < NU; ++iu)
+                R = fmaf(wu[iu], ONES ? 1.f : Buf<T>::widen(f.y[iu][c]), R);
+              rows[slot[c]] = R;
+            }
+            const int zf = __builtin_amdgcn_readlane(z0, j);
+            const int n = __builtin_amdgcn_readlane(z1, j) - zf;
+            auto pass = [&](float zi, int zz) {
+              const Overlap3 o = overlap3<3>(fmaf(zi, r.y, r.x), r.y);
+              const float* R = rows + kPadRows + o.k;
+              float sum = o.w0 * R[0];
+              sum = fmaf(o.w1, R[1], sum);
+              sum = fmaf(o.w2, R[2], sum);
+              const float dZ = fmaf(zi, d.dz, r.z);
+              const float cosv = __builtin_amdgcn_sqrtf(fmaf(dZ, dZ, r.w));
+              float* a = lacc + zf + zz + lane;
+              *a = fmaf(cosv, sum, *a);
+            };
+            if constexpr (MULTI) {
+              float zi = lanef;
+              for (int zz = 0; zz <= n; zz += 64, zi += 64.f)
+                if (lane <= n - zz) pass(zi, zz);
+            } else {
+              if (lane <= n) pass(lanef, 0);
+            }
+          });
+    };
+    using std::integral_constant;
+    using F = std::false_type;
+    using M = std::true_type;
+    run(integral_constant<int, 1>{}, F{});
+    run(integral_constant<int, 1>{}, M{});
+    run(integral_constant<int, 2>{}, F{});
+    run(integral_constant<int, 2>{}, M{});
+    run(integral_constant<int, 3>{}, F{});
+    run(integral_constant<int, 3>{}, M{});
+    run(integral_constant<int, 4>{}, F{});
+    run(integral_constant<int, 4>{}, M{});
+    // the general form: any number of columns and rows
+    uint64_t m = __ballot(key == 1);
+    BpView q{};
+    if (m && kl < A.vc) q = bp_view(A, A.vb + kl * A.vs, Px, Py, Pxf, Pyf);
+    while (m) {
+      const int j = __builtin_ctzll(m);
+      m &= m - 1;
+      const int o = __builtin_amdgcn_readlane(q_o, j), nu = __builtin_amdgcn_readlane(q.nu, j);
+      const float wu0 = rdl(q.wu0, j), fh = rdl(q.fh, j), cws = rdl(q.cws, j);
+#pragma unroll
+      for (int c = 0; c < RC; ++c) {
+        float R = cws * wu0 * (ONES ? 1.f : P.at(row[c], o));
+        for (int iu = 1; iu < nu; ++iu)
+          R = fmaf(cws * (iu == nu - 1 ? fh : 1.f), ONES ? 1.f : P.at(row[c], o + iu * DNV), R);
+        rows[slot[c]] = R;
+      }
+      const float4 r = rec[2 * j];
+      const int zf = __builtin_amdgcn_readlane(z0, j), zl = __builtin_amdgcn_readlane(z1, j);
+      for (int z = zf + lane; z <= zl; z += 64) {
+        const float zi = (float)(z - zf);
+        const float t = fmaf(zi, r.y, r.x);
+        const float tl = fmaxf(t, 0.f), th = fminf(t + r.y, (float)DNV);
+        if (!(tl < th)) continue;
+        const int v0 = (int)floorf(tl);
+        const int v1 = min((int)ceilf(th), DNV) - 1;
+        float sum = 0.f;
+        for (int v = v0; v <= v1; ++v)
+          sum = fmaf(fminf(th, (float)(v + 1)) - fmaxf(tl, (float)v), rows[kPadRows + v], sum);
+        const float dZ = fmaf(zi, d.dz, r.z);
+        lacc[z] = fmaf(__builtin_amdgcn_sqrtf(fmaf(dZ, dZ, r.w)), sum, lacc[z]);
+      }
+    }
+  }
+  for (int z = lane; z < d.ZN; z += 64) bp_store<UPDATE>(A, vcol, col, z, lacc[z]);
+}
+
+// The windowed form without staged rows (more than 256 detector rows, or frames too large
+// for the staged loads' 32-bit offsets), gathering each voxel's rows from memory; lacc: ZN
+// floats of this wave, each updated by one lane per view, views in order.  Per-voxel
+// arithmetic as bp_ref_body.
+// ONES: the back projection of a sinogram of ones, read from no sinogram: the row weights of
+// a shadow sum to its clipped height vhi - vlo and the column weights to Wu = wu0 + (nu - 2)
+// + fh (wu0 alone for one column), so a voxel adds cosVal * Wu * (vhi - vlo).
 template <bool UPDATE, typename T, bool ONES = false>
-__device__ __forceinline__ void bp_win_body(const BpArgs<T>& A, int col, float* lacc,
-                                            float* stg) {
+__device__ __forceinline__ void bp_win_body(const BpArgs<T>& A, int col, float* lacc) {
   const Dims& d = A.d;
   const BpConsts64& c64 = A.c64;
   const int lane = threadIdx.x & 63;
@@ -955,126 +1086,17 @@ __device__ __forceinline__ void bp_win_body(const BpArgs<T>& A, int col, float* 
   const double Py = ((double)y - c64.ocy) * c64.dx;
   const float Pxf = (float)Px, Pyf = (float)Py;
   const float DNVh = (float)d.DNV - 0.5f;
-  const float ZNf = (float)d.ZN;
-  const float idz = 1.f / d.dz;
   const int DNV = d.DNV;
   const uint32_t frame = (uint32_t)(d.DNU * d.DNV);
-  const bool stage = !ONES && stg != nullptr && DNV <= kStageRows;
-  float* lR = stg;                                         // rows of the current view
-  float4* rec = reinterpret_cast<float4*>(stg + kRowsF);  // [64][3] float4 records
-  if (stage && lane < kStagePad - kStageRows) lR[kStageRows + lane] = 0.f;
-  const int row = min(lane, DNV - 1);  // the row a lane stages
-  const float zlane = (float)lane - d.ocz;
   for (int k0 = 0; k0 < A.vc; k0 += 64) {
     const int kl = k0 + lane;
     BpView q{};
     int q_z0 = 0, q_z1 = -1;
     if (kl < A.vc) {
       q = bp_view(A, A.vb + kl * A.vs, Px, Py, Pxf, Pyf);
-      // voxels with fmaf(dZ, rlS, cB) > -0.5 and fmaf(dZ, rlS, cA) < DNV - 0.5 lie in the
-      // open interval (za, zb) of voxel indices; za, zb are within ~1e-4 of it (FP32), so
-      // the integers inside (za - m, zb + m), m = 1e-2, include every one of them
-      const float ea = (-0.5f - q.cB) / q.rlS, eb = (DNVh - q.cA) / q.rlS;
-      const float za = fminf(fmaxf((fminf(ea, eb) + q.sz) * idz + d.ocz, -4.f), ZNf + 4.f);
-      const float zb = fminf(fmaxf((fmaxf(ea, eb) + q.sz) * idz + d.ocz, -4.f), ZNf + 4.f);
-      q_z0 = max((int)floorf(za - 1e-2f) + 1, 0);
-      q_z1 = min((int)ceilf(zb + 1e-2f) - 1, d.ZN - 1);
+      bp_window(d, q, q_z0, q_z1);
     }
     uint64_t live = __ballot(q.uvis && q_z0 <= q_z1);
-    if (stage && live) {
-#pragma clang fp contract(off)
-      {
-        // column weights of view k0 + lane: first wu0, interior 1, last fh, past nu 0
-        const int nu = q.nu;
-        const float w1 = nu > 1 ? (nu == 2 ? q.fh : 1.f) : 0.f;
-        const float w2 = nu > 2 ? (nu == 3 ? q.fh : 1.f) : 0.f;
-        const float w3 = nu > 3 ? (nu == 4 ? q.fh : 1.f) : 0.f;
-        rec[3 * lane + 0] = make_float4(q.rlS, q.cA, q.cB, q.sz);
-        rec[3 * lane + 1] = make_float4(q.l2, q.cws, q.wu0, w1);
-        rec[3 * lane + 2] = make_float4(w2, w3, 0.f, 0.f);
-      }
-      // rows of view k0 + j: columns u0 + min(iu, nu - 1) (a repeated column has weight 0)
-      // (stored bits, widened at their use: the next view's loads stay in flight while
-      // this view's voxels are summed)
-      auto load_rows = [&](int j, uint32_t (&yb)[4]) {
-        const int un = __builtin_amdgcn_readlane(q.u0, j);
-        const int nn = __builtin_amdgcn_readlane(q.nu, j);
-        const Buf<T> pn(A.prj + (size_t)(k0 + j) * frame, frame);
-#pragma unroll
-        for (int iu = 0; iu < 4; ++iu) yb[iu] = pn.at_bits(row, (un + min(iu, nn - 1)) * DNV);
-      };
-      int j = __builtin_ctzll(live);
-      uint32_t yb[4];
-      load_rows(j, yb);
-      while (true) {
-        const int nu = __builtin_amdgcn_readlane(q.nu, j);
-        const int z0 = __builtin_amdgcn_readlane(q_z0, j), z1 = __builtin_amdgcn_readlane(q_z1, j);
-        const float4 r0 = rec[3 * j], r1 = rec[3 * j + 1], r2 = rec[3 * j + 2];
-        float R = r1.z * Buf<T>::widen(yb[0]);
-        R = fmaf(r1.w, Buf<T>::widen(yb[1]), R);
-        R = fmaf(r2.x, Buf<T>::widen(yb[2]), R);
-        R = fmaf(r2.y, Buf<T>::widen(yb[3]), R);
-        if (nu > 4) {
-          const int un = __builtin_amdgcn_readlane(q.u0, j);
-          const float fh = rdl(q.fh, j);
-          const Buf<T> pn(A.prj + (size_t)(k0 + j) * frame, frame);
-          for (int iu = 4; iu < nu; ++iu)
-            R = fmaf((iu == nu - 1) ? fh : 1.f, pn.at(row, (un + iu) * DNV), R);
-        }
-        lR[lane] = lane < DNV ? R : 0.f;
-        // the next visible view's rows load while this view's voxels are summed
-        live &= live - 1;
-        const int jn = live ? __builtin_ctzll(live) : -1;
-        if (jn >= 0) load_rows(jn, yb);
-        const float rlS = r0.x, cA = r0.y, cB = r0.z, vsz = r0.w, l2f = r1.x, cws = r1.y;
-        for (int zz = z0; zz <= z1; zz += 64) {
-          // (float)(zz + lane) - ocz, exactly (half-integers far below 2^23); voxels past
-          // z1 lie outside the shadow's open interval with the window's 1e-2-voxel margin
-          // (empty shadows), those past the column add to lacc's padding
-          const float dZ = fmaf((float)zz + zlane, d.dz, -vsz);
-          const float vlo = fmaxf(fmaf(dZ, rlS, cA), -0.5f);
-          const float vhi = __builtin_elementwise_minimum(fmaf(dZ, rlS, cB), DNVh);
-          if (vlo < vhi) {
-            const float cosVal = cws * __builtin_amdgcn_sqrtf(fmaf(dZ, dZ, l2f));
-            float* lz = lacc + zz;
-            lz[lane] = fmaf(cosVal, bp_lds_sum(lR, vlo, vhi, DNV), lz[lane]);
-          }
-        }
-        if (jn < 0) break;
-        j = jn;
-      }
-      continue;
-    }
-    if constexpr (ONES) {
-      // views' constants (with the column-weight sum Wu) from a table in LDS (stg: 64
-      // records of 8 floats), read at a uniform address instead of by readlanes
-      if (live) {
-        float4* rec1 = reinterpret_cast<float4*>(stg);
-        const int nu = q.nu;
-        const float Wu = nu == 1 ? q.wu0 : q.wu0 + (float)(nu - 2) + q.fh;
-        rec1[2 * lane] = make_float4(q.rlS, q.cA, q.cB, q.sz);
-        rec1[2 * lane + 1] = make_float4(q.l2, q.cws, Wu, 0.f);
-        while (live) {
-          const int j = __builtin_ctzll(live);
-          live &= live - 1;
-          const int z0 = __builtin_amdgcn_readlane(q_z0, j), z1 = __builtin_amdgcn_readlane(q_z1, j);
-          const float4 r0 = rec1[2 * j], r1 = rec1[2 * j + 1];
-          const float rlS = r0.x, cA = r0.y, cB = r0.z, vsz = r0.w;
-          const float l2f = r1.x, cws = r1.y, Wv = r1.z;
-          for (int zz = z0; zz <= z1; zz += 64) {
-            const int z = zz + lane;
-            const float dZ = fmaf((float)z - d.ocz, d.dz, -vsz);
-            const float vlo = fmaxf(fmaf(dZ, rlS, cA), -0.5f);
-            const float vhi = fminf(fmaf(dZ, rlS, cB), DNVh);
-            if (z <= z1 && vlo < vhi) {
-              const float cosVal = cws * __builtin_amdgcn_sqrtf(fmaf(dZ, dZ, l2f));
-              lacc[z] = fmaf(cosVal, Wv * (vhi - vlo), lacc[z]);
-            }
-          }
-        }
-      }
-      continue;
-    }
     while (live) {
       const int j = __builtin_ctzll(live);
       live &= live - 1;
@@ -1085,7 +1107,6 @@ __device__ __forceinline__ void bp_win_body(const BpArgs<T>& A, int col, float* 
       const int u0 = __builtin_amdgcn_readlane(q.u0, j), nu = __builtin_amdgcn_readlane(q.nu, j);
       const int z0 = __builtin_amdgcn_readlane(q_z0, j), z1 = __builtin_amdgcn_readlane(q_z1, j);
       const Buf<T> pp(A.prj + (size_t)k * frame, frame);
-      const float Wu = nu == 1 ? wu0 : wu0 + (float)(nu - 2) + fh;
       for (int zz = z0; zz <= z1; zz += 64) {
         const int z = zz + lane;
         const float dZ = fmaf((float)z - d.ocz, d.dz, -vsz);
@@ -1094,14 +1115,28 @@ __device__ __forceinline__ void bp_win_body(const BpArgs<T>& A, int col, float* 
         const bool vok = z <= z1 && vlo < vhi;
         if (!vok) continue;
         const float cosVal = cws * __builtin_amdgcn_sqrtf(fmaf(dZ, dZ, l2f));
-        if constexpr (ONES)
+        if constexpr (ONES) {
+          const float Wu = nu == 1 ? wu0 : wu0 + (float)(nu - 2) + fh;
           lacc[z] = fmaf(cosVal, Wu * (vhi - vlo), lacc[z]);
-        else
+        } else {
           lacc[z] = fmaf(cosVal, bp_cell_sum(pp, u0, nu, wu0, fh, vlo, vhi, DNV), lacc[z]);
+        }
       }
     }
   }
   for (int z = lane; z < d.ZN; z += 64) bp_store<UPDATE>(A, vcol, col, z, lacc[z]);
+}
+
+// The windowed body with staged rows (RC = 1, 2, 4) or without (RC = 0); lds: bp_win_floats
+// of this wave.
+__host__ __device__ constexpr int bp_win_floats(int RC, int ZN) {
+  return (RC == 1 ? kStagedF<1> : RC == 2 ? kStagedF<2> : RC == 4 ? kStagedF<4> : 0) +
+         ((ZN + 3) & ~3);
+}
+template <bool UPDATE, typename T, int RC, bool ONES = false>
+__device__ __forceinline__ void bp_any_win_body(const BpArgs<T>& A, int col, float* lds) {
+  if constexpr (RC > 0) bp_staged_body<UPDATE, T, RC, ONES>(A, col, lds);
+  else bp_win_body<UPDATE, T, ONES>(A, col, lds);
 }
 
 template <bool UPDATE, int ZG, typename T>
@@ -1110,76 +1145,61 @@ __global__ __launch_bounds__(kBlock) void bp_ref_kernel(BpArgs<T> A) {
   bp_ref_body<UPDATE, ZG, T>(A, col, blockIdx.y);
 }
 
-// Windowed reference back projection; dynamic LDS: kWaves * kStageF floats of staged
-// views (DNV <= kStageRows; none otherwise), then kWaves * (ZN + kLaccPad) floats of
-// column sums (kWaves * ZN unstaged).
-// At most 72 VGPRs (7 waves per SIMD; no scratch).
-template <bool UPDATE, typename T>
-__global__ __launch_bounds__(kBlock, 7) void bp_win_kernel(BpArgs<T> A) {
+// Windowed reference back projection; dynamic LDS: kWaves * bp_win_floats(RC, ZN) floats.
+template <bool UPDATE, typename T, int RC>
+__global__ __launch_bounds__(kBlock, RC == 4 ? 5 : RC == 2 ? 6 : RC == 1 ? 8 : 7) void bp_win_kernel(BpArgs<T> A) {
   extern __shared__ float4 lds_win[];
   float* lds = reinterpret_cast<float*>(lds_win);
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const bool stage = A.d.DNV <= kStageRows;
-  float* lacc = lds + (stage ? kWaves * kStageF : 0) + wid * (A.d.ZN + (stage ? kLaccPad : 0));
-  bp_win_body<UPDATE, T>(A, blockIdx.x * kWaves + wid, lacc,
-                         stage ? lds + wid * kStageF : nullptr);
+  bp_any_win_body<UPDATE, T, RC>(A, blockIdx.x * kWaves + wid,
+                                 lds + wid * bp_win_floats(RC, A.d.ZN));
 }
 
-// Back projection of a sinogram of ones (A.prj unused); dynamic LDS: kWaves * 512
-// floats of view records, then kWaves * ZN floats of column sums.
-constexpr int kOnesRecF = 512;
-__global__ __launch_bounds__(kBlock, 8) void bp_win_ones_kernel(BpArgs<float> A) {
-  extern __shared__ float4 lds_ones[];
-  float* lds = reinterpret_cast<float*>(lds_ones);
+// Back projection of a sinogram of ones (A.prj unused); dynamic LDS as bp_win_kernel.
+template <int RC>
+__global__ __launch_bounds__(kBlock, RC == 4 ? 5 : 7) void bp_win_ones_kernel(BpArgs<float> A) {
+  extern __shared__ float4 lds_win[];
+  float* lds = reinterpret_cast<float*>(lds_win);
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  bp_win_body<false, float, true>(A, blockIdx.x * kWaves + wid,
-                                  lds + kWaves * kOnesRecF + wid * A.d.ZN,
-                                  lds + wid * kOnesRecF);
+  bp_any_win_body<false, float, RC, true>(A, blockIdx.x * kWaves + wid,
+                                          lds + wid * bp_win_floats(RC, A.d.ZN));
 }
 
 // Batched windowed reference back projection: flat work list of (scan, block of 4
-// columns); dynamic LDS: kWaves * kStageF floats of staged views (every scan of the batch
-// has DNV <= kStageRows: staged; otherwise none), then kWaves * (zmax + kLaccPad) floats
-// (zmax: the tallest column of the batch; kWaves * zmax unstaged).
-template <typename T>
-__global__ __launch_bounds__(kBlock, 7) void bp_batch_win_kernel(const BpBatchItem<T>* __restrict__ D,
+// columns); RC as the scan of most rows needs it, dynamic LDS: kWaves *
+// bp_win_floats(RC, zmax) floats (zmax: the tallest column of the batch).
+template <typename T, int RC>
+__global__ __launch_bounds__(kBlock, RC == 4 ? 5 : RC == 2 ? 6 : 7) void bp_batch_win_kernel(const BpBatchItem<T>* __restrict__ D,
                                                               int nscan, int total, int sched,
-                                                              int zmax, int staged) {
+                                                              int zmax) {
   extern __shared__ float4 lds_win[];
-  float* lds = reinterpret_cast<float*>(lds_win);
   int i0, step, i1;
   batch_range(D, nscan, total, sched, i0, step, i1);
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  float* lds = reinterpret_cast<float*>(lds_win) + wid * bp_win_floats(RC, zmax);
   int s = 0;
   for (int item = i0; item < i1; item += step) {
     if (sched == 1) s = 0;
     while (s + 1 < nscan && D[s + 1].begin <= item) ++s;
     const BpBatchItem<T>& B = D[s];
-    bp_win_body<true, T>(B.a, (item - B.begin) * kWaves + wid,
-                         lds + (staged ? kWaves * kStageF : 0) +
-                             wid * (zmax + (staged ? kLaccPad : 0)),
-                         staged ? lds + wid * kStageF : nullptr);
+    bp_any_win_body<true, T, RC>(B.a, (item - B.begin) * kWaves + wid, lds);
   }
 }
 
 // bp_batch_win_kernel for the one-workgroup-per-item schedule (grid = total): no item
-// loop, so nothing stays live around the column body.  Both batched windowed kernels are
-// held to 72 VGPRs (7 waves per SIMD), as bp_win_kernel.
-template <typename T>
-__global__ __launch_bounds__(kBlock, 7) void bp_batch_win1_kernel(
-    const BpBatchItem<T>* __restrict__ D, int nscan, int total, int zmax, int staged) {
+// loop, so nothing stays live around the column body.
+template <typename T, int RC>
+__global__ __launch_bounds__(kBlock, RC == 4 ? 5 : RC == 2 ? 6 : 7) void bp_batch_win1_kernel(
+    const BpBatchItem<T>* __restrict__ D, int nscan, int total, int zmax) {
   extern __shared__ float4 lds_win[];
-  float* lds = reinterpret_cast<float*>(lds_win);
   int i0, step, i1;
   batch_range(D, nscan, total, 2, i0, step, i1);
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  float* lds = reinterpret_cast<float*>(lds_win) + wid * bp_win_floats(RC, zmax);
   int s = 0;
   while (s + 1 < nscan && D[s + 1].begin <= i0) ++s;
   const BpBatchItem<T>& B = D[s];
-  bp_win_body<true, T>(B.a, (i0 - B.begin) * kWaves + wid,
-                       lds + (staged ? kWaves * kStageF : 0) +
-                           wid * (zmax + (staged ? kLaccPad : 0)),
-                       staged ? lds + wid * kStageF : nullptr);
+  bp_any_win_body<true, T, RC>(B.a, (i0 - B.begin) * kWaves + wid, lds);
 }
 
 // Batched persistent reference back projection: flat work list of (scan, z block,
@@ -1651,6 +1671,251 @@ __global__ __launch_bounds__(kBlock) void bp_matched_win_kernel(
   }
 }
 
+// A view's detector columns meeting one voxel's cell on its slice: the boundary lines of
+// fp_kernel in FP64, walked from the column that the voxel centre's fan angle suggests.
+// next() steps to the next column while one meets the cell.
+struct MatchedCols {
+  const double2* bt;
+  double fi, dir, cl, ch, su, su1;
+  int u, DNU;
+  __device__ __forceinline__ MatchedCols(const ViewP& vp, const double2* bnd, int p, int x, int y,
+                                         float Px, float Py, const Dims& d, float inv_sid) {
+    const int ii = vp.xmarch ? x : y, j = vp.xmarch ? y : x;
+    DNU = d.DNU;
+    fi = (double)ii;
+    bt = bnd + (size_t)p * (DNU + 1);
+    dir = (double)vp.bdir;
+    cl = (vp.bdir > 0) ? (double)j - 0.5 : -((double)j + 0.5);
+    ch = cl + 1.0;
+    const float dX = Px - vp.sx, dY = Py - vp.sy;
+    const float beta = asinf((vp.sy * dX - vp.sx * dY) * inv_sid * rsqrtf(dX * dX + dY * dY));
+    u = (int)fminf(fmaxf(floorf((beta - d.beta0) / d.dbeta_g), 0.f), (float)(DNU - 1));
+    su = at(u);
+    while (u > 0 && su > cl) su = at(--u);
+    su1 = at(u + 1);
+    while (u < DNU - 1 && su1 <= cl) {
+      ++u;
+      su = su1;
+      su1 = at(u + 1);
+    }
+  }
+  __device__ __forceinline__ double at(int b) const {
+    const double2 t = gload(bt, b);
+    return dir * fma(fi, t.y, t.x);
+  }
+  __device__ __forceinline__ bool meets() const { return u < DNU && su < ch; }
+  // overlap of the column with the cell (<= 0: none)
+  __device__ __forceinline__ double overlap() const { return fmin(su1, ch) - fmax(su, cl); }
+  __device__ __forceinline__ void next() {
+    ++u;
+    if (u < DNU) {
+      su = su1;
+      su1 = at(u + 1);
+    }
+  }
+};
+
+// Windowed matched adjoint with staged rows, for detectors of evenly spaced rows
+// (d.even_rows; DNV <= 64 RC): bp_staged_body's scheme with one row set per detector column,
+// since each column's rows have their own magnification r.  In units of the rows the cell
+// of voxel z meets column t's rows over [T, T + s], T = T0 + (z - z0) s, s = 1 / (r dB), and
+// its overlap with a row, times the column's in-plane overlap over its footprint's area, is
+// the forward projector's weight: w_t = overlap dB / (tr - tl), r cancelling.  Lane l
+// evaluates view k0 + l (columns, T0 and s in FP64); the row sets hold w_t y[u + t][v].
+// Views of more than four columns, of more than three rows per voxel, or whose columns'
+// rows differ by over a row across the window take the row walk.
+// bound by VALU issue as bp_staged_body, with about 11 instructions per column and pass.
+template <int RC>
+constexpr int kMatchedF = 4 * kRowsLds<RC> + 64 * 16;
+__host__ __device__ constexpr int bp_matched_floats(int RC, int ZN) {
+  return (RC == 1 ? kMatchedF<1> : RC == 2 ? kMatchedF<2> : kMatchedF<4>) + ((ZN + 3) & ~3);
+}
+template <bool UPDATE, int RC>
+__global__ __launch_bounds__(kBlock, RC == 4 ? 4 : 6) void bp_matched_staged_kernel(
+    const float* __restrict__ yp, float* __restrict__ vol, const ViewP* __restrict__ views,
+    const double2* __restrict__ bnd, const float4* __restrict__ cols,
+    const float* __restrict__ Bz, const uint8_t* __restrict__ mask, Dims d, BpConsts c,
+    int vb, int vs, int vc, const float* __restrict__ invCol, uint16_t* __restrict__ shadow) {
+  extern __shared__ float4 lds_win[];
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  float* rows = reinterpret_cast<float*>(lds_win) + wid * bp_matched_floats(RC, d.ZN);
+  float4* rec = reinterpret_cast<float4*>(rows + 4 * kRowsLds<RC>);  // [64][4]
+  float* lacc = rows + kMatchedF<RC>;
+  const int col = blockIdx.x * kWaves + wid;
+  if (col >= d.XN * d.YN) return;
+  const int y = col / d.XN, x = col - y * d.XN;
+  float* vcol = vol + (size_t)col * d.ZN;
+  const float mk = (float)mask[col];
+  if (mk == 0.f) {
+    if constexpr (!UPDATE) {
+      for (int z = lane; z < d.ZN; z += 64) vcol[z] = 0.f;
+    }
+    return;
+  }
+  for (int z = lane; z < d.ZN; z += 64) lacc[z] = 0.f;
+  const int DNU = d.DNU, DNV = d.DNV, frame = DNU * DNV;
+  int row[RC], slot[RC];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) stage_rows<RC>(rows + t * kRowsLds<RC>, DNV, lane, row, slot);
+  const float Px = ((float)x - d.ocx) * d.dx, Py = ((float)y - d.ocy) * d.dx;
+  const float lanef = (float)lane, ZNf = (float)d.ZN;
+  const double B0 = d.B0_64, idB = 1.0 / d.dB_64;
+  for (int k0 = 0; k0 < vc; k0 += 64) {
+    const int kl = k0 + lane;
+    int z0 = 0, z1 = -1, q_o = 0, key = 0;
+    if (kl < vc) {
+      const int p = vb + kl * vs;
+      const ViewP vp = views[p];
+      const float4* ctab = cols + (size_t)p * DNU;
+      const float fii = (float)(vp.xmarch ? x : y);
+      MatchedCols mc(vp, bnd, p, x, y, Px, Py, d, c.inv_sid);
+      q_o = lane * frame + mc.u * DNV;
+      float rt[4] = {1.f, 1.f, 1.f, 1.f}, wt[4] = {0.f, 0.f, 0.f, 0.f};
+      float rmin = 3.4e38f, rmax = -3.4e38f;
+      int n = 0;
+      for (; mc.meets(); mc.next()) {
+        const float4 ct = ctab[mc.u];
+        const float r = fmaf(fii, ct.y, ct.x);
+        const double wy = mc.overlap();
+        const float w = wy > 0.0 ? (float)(wy / (mc.su1 - mc.su) * d.dB_64) : 0.f;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          if (n == t) {
+            rt[t] = r;
+            wt[t] = w;
+          }
+        rmin = fminf(rmin, r);
+        rmax = fmaxf(rmax, r);
+        ++n;
+      }
+      if (n > 0 && rmin > 0.f) {
+        // z cells [k - .5, k + .5] meeting [az + r Bz[0], az + r Bz[DNV]] for some column,
+        // with a margin of 1e-2 (relative to azi, as fp_kernel)
+        const float lo = fminf(fmaf(rmin, Bz[0], vp.azf), fmaf(rmax, Bz[0], vp.azf));
+        const float hi = fmaxf(fmaf(rmin, Bz[DNV], vp.azf), fmaf(rmax, Bz[DNV], vp.azf));
+        const float fazi = (float)vp.azi;
+        const float za = fminf(fmaxf(lo - 0.51f, -4.f - fazi), (ZNf + 4.f) - fazi);
+        const float zb = fminf(fmaxf(hi + 0.51f, -4.f - fazi), (ZNf + 4.f) - fazi);
+        z0 = max((int)floorf(za) + 1 + vp.azi, 0);
+        z1 = min((int)ceilf(zb) - 1 + vp.azi, d.ZN - 1);
+        if (z0 <= z1) {
+          bool plain = n <= 4;
+          const double e0 = (double)(z0 - vp.azi) - 0.5 - (double)vp.azf;
+#pragma unroll
+          for (int t = 0; t < 4; ++t)
+            if (t < n) {
+              const double s = idB / (double)rt[t];
+              const float sf = (float)s, T0 = (float)(e0 * s - B0 * idB);
+              // taps stay on the row set and its zeros over the whole window
+              plain = plain && sf <= 2.f && T0 >= (float)-kPadRows &&
+                      fmaf((float)(z1 - z0), sf, T0) < (float)(DNV + kPadRows - 2);
+              rec[4 * lane + t] = make_float4(T0, sf, wt[t], 0.f);
+            }
+          // the class: columns * 2 + (more than one pass); 1 the row walk
+          key = plain ? 2 * n + (z1 - z0 >= 64 ? 1 : 0) : 1;
+        }
+      }
+    }
+    if (!__any(key)) continue;
+    const Buf<float> P(yp + (size_t)k0 * frame, (uint32_t)min(64, vc - k0) * (uint32_t)frame);
+    auto run = [&](auto NU_, auto MULTI_) {
+      constexpr int NU = decltype(NU_)::value;
+      constexpr bool MULTI = decltype(MULTI_)::value;
+      const uint64_t m = __ballot(key == 2 * NU + (MULTI ? 1 : 0));
+      if (!m) return;
+      struct Set {
+        float y[NU][RC];
+      };
+      pipelined<Set>(
+          m,
+          [&](int j, Set& f) {
+            const int o = __builtin_amdgcn_readlane(q_o, j);
+#pragma unroll
+            for (int t = 0; t < NU; ++t)
+#pragma unroll
+              for (int h = 0; h < RC; ++h) f.y[t][h] = P.at(row[h], o + t * DNV);
+          },
+          [&](int j, const Set& f) {
+            float4 r[NU];
+#pragma unroll
+            for (int t = 0; t < NU; ++t) {
+              r[t] = rec[4 * j + t];
+#pragma unroll
+              for (int h = 0; h < RC; ++h) rows[t * kRowsLds<RC> + slot[h]] = r[t].z * f.y[t][h];
+            }
+            const int zf = __builtin_amdgcn_readlane(z0, j);
+            const int n = __builtin_amdgcn_readlane(z1, j) - zf;
+            auto pass = [&](float zi, int zz) {
+              float g = 0.f;
+#pragma unroll
+              for (int t = 0; t < NU; ++t) {
+                const Overlap3 o = overlap3<3>(fmaf(zi, r[t].y, r[t].x), r[t].y);
+                const float* R = rows + t * kRowsLds<RC> + kPadRows + o.k;
+                g = t == 0 ? o.w0 * R[0] : fmaf(o.w0, R[0], g);
+                g = fmaf(o.w1, R[1], g);
+                g = fmaf(o.w2, R[2], g);
+              }
+              lacc[zf + zz + lane] += g;
+            };
+            if constexpr (MULTI) {
+              float zi = lanef;
+              for (int zz = 0; zz <= n; zz += 64, zi += 64.f)
+                if (lane <= n - zz) pass(zi, zz);
+            } else {
+              if (lane <= n) pass(lanef, 0);
+            }
+          });
+    };
+    using std::integral_constant;
+    using F = std::false_type;
+    using M = std::true_type;
+    run(integral_constant<int, 1>{}, F{});
+    run(integral_constant<int, 1>{}, M{});
+    run(integral_constant<int, 2>{}, F{});
+    run(integral_constant<int, 2>{}, M{});
+    run(integral_constant<int, 3>{}, F{});
+    run(integral_constant<int, 3>{}, M{});
+    run(integral_constant<int, 4>{}, F{});
+    run(integral_constant<int, 4>{}, M{});
+    uint64_t m = __ballot(key == 1);
+    while (m) {
+      const int j = __builtin_ctzll(m);
+      m &= m - 1;
+      const int k = k0 + j, p = vb + k * vs;
+      const ViewP vp = views[p];
+      const float4* ctab = cols + (size_t)p * DNU;
+      const float fii = (float)(vp.xmarch ? x : y);
+      const int zf = __builtin_amdgcn_readlane(z0, j), zl = __builtin_amdgcn_readlane(z1, j);
+      for (int z = zf + lane; z <= zl; z += 64) {
+        const float zlo = (float)(z - vp.azi) - 0.5f;
+        float a = lacc[z];
+        for (MatchedCols mc(vp, bnd, p, x, y, Px, Py, d, c.inv_sid); mc.meets(); mc.next()) {
+          const double wy = mc.overlap();
+          if (!(wy > 0.0)) continue;
+          const float4 ct = ctab[mc.u];
+          const float r = fmaf(fii, ct.y, ct.x);
+          const float w = (float)wy * __builtin_amdgcn_rcpf((float)(mc.su1 - mc.su) * r);
+          a = fmaf(w, matched_rows(yp + (size_t)k * frame + (size_t)mc.u * DNV, Bz, DNV, r,
+                                   vp.azf, zlo, d.B0, d.dB), a);
+        }
+        lacc[z] = a;
+      }
+    }
+  }
+  for (int z = lane; z < d.ZN; z += 64) {
+    const float a = lacc[z] * mk;
+    if constexpr (UPDATE) {
+      const size_t i = (size_t)col * d.ZN + z;
+      const float nx = fmaf(a, invCol[i], vcol[z]);
+      vcol[z] = nx;
+      if (shadow) shadow[i] = to_bf16_dither(nx, i);
+    } else {
+      vcol[z] = a;
+    }
+  }
+}
+
 // yp[k][u][v] = y[k][u][v] * K(p,u,v) * invdB[v]: the per-ray factors of fp_kernel
 // (y stored as float or BF16, yp FP32).
 template <typename T>
@@ -1857,20 +2122,36 @@ int launch_fp(const Plan& P, const TV* vol, TO* out, int vb, int vs, int vc, hip
 
 int launch_fp_ones(const Plan& P, float* out, int vb, int vs, int vc, hipStream_t st) {
   if (vc <= 0) return CTR_OK;
-  dim3 grid((P.d.DNU * P.d.DNV + kBlock - 1) / kBlock, vc);
   const FpArgs<float, float> A =
       fp_args<float, float>(P, nullptr, out, vb, vs, nullptr, nullptr, nullptr);
-  if (P.d.DNV == 64) hipLaunchKernelGGL((fp_ones_kernel<true>), grid, dim3(kBlock), 0, st, A);
-  else hipLaunchKernelGGL((fp_ones_kernel<false>), grid, dim3(kBlock), 0, st, A);
+  const int bpv = fp_blocks_of(P, A.lg);
+  const dim3 grid(xcd_chunked_grid((long long)bpv * vc));
+  if (A.lg == 6)
+    hipLaunchKernelGGL((fp_ones_kernel<true>), grid, dim3(kBlock), 0, st, A, bpv, vc);
+  else
+    hipLaunchKernelGGL((fp_ones_kernel<false>), grid, dim3(kBlock), 0, st, A, bpv, vc);
   return check_launch("fp_ones_kernel");
+}
+
+// Row chunks (of 64) a staged wave holds for a detector, 0 for the unstaged form: over 256
+// rows, or 64 frames past the staged loads' 32-bit byte offsets.
+int bp_row_chunks(int DNU, int DNV) {
+  if (DNV > 256 || (long long)DNU * DNV > (1ll << 23)) return 0;
+  return DNV <= 64 ? 1 : DNV <= 128 ? 2 : 4;
 }
 
 int launch_bp_ones(const Plan& P, float* vol, int vb, int vs, int vc, hipStream_t st) {
   if (P.d.ZN > kWinMaxZ) return fail(CTR_ERR_ARG, "bp of ones: columns over the LDS limit");
   const BpArgs<float> A = bp_args<float>(P, nullptr, vol, vb, vs, vc, nullptr, nullptr);
   const dim3 wgrid((P.d.XN * P.d.YN + kWaves - 1) / kWaves);
-  hipLaunchKernelGGL(bp_win_ones_kernel, wgrid, dim3(kBlock),
-                     (size_t)kWaves * (kOnesRecF + P.d.ZN) * sizeof(float), st, A);
+  const int rc = bp_row_chunks(P.d.DNU, P.d.DNV);
+  const size_t lds = (size_t)kWaves * bp_win_floats(rc, P.d.ZN) * sizeof(float);
+  switch (rc) {
+    case 1: hipLaunchKernelGGL(bp_win_ones_kernel<1>, wgrid, dim3(kBlock), lds, st, A); break;
+    case 2: hipLaunchKernelGGL(bp_win_ones_kernel<2>, wgrid, dim3(kBlock), lds, st, A); break;
+    case 4: hipLaunchKernelGGL(bp_win_ones_kernel<4>, wgrid, dim3(kBlock), lds, st, A); break;
+    default: hipLaunchKernelGGL(bp_win_ones_kernel<0>, wgrid, dim3(kBlock), lds, st, A); break;
+  }
   return check_launch("bp_win_ones_kernel");
 }
 
@@ -1883,6 +2164,29 @@ int launch_bp(const Plan& P, const T* prj, float* vol, int vb, int vs, int vc, i
     if constexpr (!std::is_same<T, float>::value) {
       return fail(CTR_ERR_ARG, "the matched back projector reads the FP32 scaled sinogram");
     } else {
+      const int rc = bp_row_chunks(P.d.DNU, P.d.DNV);
+      const size_t slds = (size_t)kWaves * bp_matched_floats(rc, P.d.ZN) * sizeof(float);
+      if (P.d.even_rows && rc > 0 && P.d.ZN <= kWinMaxZ && slds <= 65536) {
+        const dim3 wgrid((P.d.XN * P.d.YN + kWaves - 1) / kWaves);
+#define CTR_BPMS(UPD, RC, IC, SH)                                                              \
+  hipLaunchKernelGGL((bp_matched_staged_kernel<UPD, RC>), wgrid, dim3(kBlock), slds, st, prj,  \
+                     vol, P.views, P.bnd64, P.cols, P.Bz, P.mask, P.d, P.bc, vb, vs, vc, IC, SH)
+        if (accumulate) {
+          switch (rc) {
+            case 1: CTR_BPMS(true, 1, invCol, shadow); break;
+            case 2: CTR_BPMS(true, 2, invCol, shadow); break;
+            default: CTR_BPMS(true, 4, invCol, shadow); break;
+          }
+        } else {
+          switch (rc) {
+            case 1: CTR_BPMS(false, 1, nullptr, nullptr); break;
+            case 2: CTR_BPMS(false, 2, nullptr, nullptr); break;
+            default: CTR_BPMS(false, 4, nullptr, nullptr); break;
+          }
+        }
+#undef CTR_BPMS
+        return check_launch("bp_matched_staged_kernel");
+      }
       // windowed kernel while its row table and column sums fit 64 KiB of LDS
       const size_t lds =
           ((size_t)((P.d.DNV + 1 + 3) & ~3) + (size_t)kWaves * P.d.ZN) * sizeof(float);
@@ -1924,12 +2228,22 @@ int launch_bp(const Plan& P, const T* prj, float* vol, int vb, int vs, int vc, i
                                  accumulate ? shadow : nullptr);
   if (P.d.ZN <= kWinMaxZ) {
     const dim3 wgrid((P.d.XN * P.d.YN + kWaves - 1) / kWaves);
-    const size_t stg = P.d.DNV <= kStageRows ? kStageF + kLaccPad : 0;  // staged views
-    const size_t lds = (size_t)kWaves * (P.d.ZN + stg) * sizeof(float);
-    if (accumulate)
-      hipLaunchKernelGGL((bp_win_kernel<true, T>), wgrid, dim3(kBlock), lds, st, A);
-    else
-      hipLaunchKernelGGL((bp_win_kernel<false, T>), wgrid, dim3(kBlock), lds, st, A);
+    const int rc = bp_row_chunks(P.d.DNU, P.d.DNV);
+    const size_t lds = (size_t)kWaves * bp_win_floats(rc, P.d.ZN) * sizeof(float);
+#define CTR_BPW(RC)                                                                           \
+  do {                                                                                        \
+    if (accumulate)                                                                           \
+      hipLaunchKernelGGL((bp_win_kernel<true, T, RC>), wgrid, dim3(kBlock), lds, st, A);      \
+    else                                                                                      \
+      hipLaunchKernelGGL((bp_win_kernel<false, T, RC>), wgrid, dim3(kBlock), lds, st, A);     \
+  } while (0)
+    switch (rc) {
+      case 1: CTR_BPW(1); break;
+      case 2: CTR_BPW(2); break;
+      case 4: CTR_BPW(4); break;
+      default: CTR_BPW(0); break;
+    }
+#undef CTR_BPW
     return check_launch("bp_win_kernel");
   }
 #define CTR_BPREF(UPD, ZGV) \
@@ -1996,21 +2310,29 @@ int launch_bp_batch(const BpBatchItem<T>* items, int nscan, int total, int zg, i
 }
 
 template <typename T>
-int launch_bp_batch_win(const BpBatchItem<T>* items, int nscan, int total, int zmax,
-                        int maxDNV, int grid, int strided, hipStream_t st) {
+int launch_bp_batch_win(const BpBatchItem<T>* items, int nscan, int total, int zmax, int rc,
+                        int grid, int strided, hipStream_t st) {
   if (total <= 0) return CTR_OK;
   if (zmax < 1 || zmax > kWinMaxZ) return fail(CTR_ERR_ARG, "bp_batch_win: column height");
   const int sched = grid <= 0 ? 2 : (strided ? 1 : 0);
   grid = grid <= 0 ? total : std::max(1, std::min(grid, total));
-  const int staged = maxDNV <= kStageRows ? 1 : 0;
-  const size_t lds =
-      (size_t)kWaves * (zmax + (staged ? kStageF + kLaccPad : 0)) * sizeof(float);
-  if (sched == 2)
-    hipLaunchKernelGGL((bp_batch_win1_kernel<T>), dim3(grid), dim3(kBlock), lds, st, items,
-                       nscan, total, zmax, staged);
-  else
-    hipLaunchKernelGGL((bp_batch_win_kernel<T>), dim3(grid), dim3(kBlock), lds, st, items,
-                       nscan, total, sched, zmax, staged);
+  const size_t lds = (size_t)kWaves * bp_win_floats(rc, zmax) * sizeof(float);
+#define CTR_BPBW(RC)                                                                          \
+  do {                                                                                        \
+    if (sched == 2)                                                                           \
+      hipLaunchKernelGGL((bp_batch_win1_kernel<T, RC>), dim3(grid), dim3(kBlock), lds, st,    \
+                         items, nscan, total, zmax);                                          \
+    else                                                                                      \
+      hipLaunchKernelGGL((bp_batch_win_kernel<T, RC>), dim3(grid), dim3(kBlock), lds, st,     \
+                         items, nscan, total, sched, zmax);                                   \
+  } while (0)
+  switch (rc) {
+    case 1: CTR_BPBW(1); break;
+    case 2: CTR_BPBW(2); break;
+    case 4: CTR_BPBW(4); break;
+    default: CTR_BPBW(0); break;
+  }
+#undef CTR_BPBW
   return check_launch("bp_batch_win_kernel");
 }
 

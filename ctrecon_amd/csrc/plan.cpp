@@ -155,6 +155,16 @@ static int build_tables(const ctr_geometry* g, Plan& P, double half = 0.0) {
   for (int v = 1; v < DNV; ++v) d.dBmin = std::min(d.dBmin, Bz[v + 1] - Bz[v]);
 
   d.dBmax = *std::max_element(dBz.begin(), dBz.end());
+  d.B0_64 = (bz[0] - z0) / dz;
+  d.dB_64 = (bz[DNV] - bz[0]) / dz / DNV;
+  {
+    double far = 0.0, off = 0.0;
+    for (int v = 0; v <= DNV; ++v) {
+      far = std::max(far, std::fabs(bz[v]));
+      off = std::max(off, std::fabs(bz[v] - (bz[0] + (bz[DNV] - bz[0]) * v / DNV)));
+    }
+    d.even_rows = off <= 4.0 * 0x1p-24 * far ? 1 : 0;
+  }
 
   // fan angles of the column boundaries seen from the source (rotation invariant)
   const double sid = std::sqrt(x0 * x0 + y0 * y0);

@@ -260,8 +260,9 @@ typedef struct ctr_batch_info {
   int fp_colw;        /* forward mapping: 1 = one wave per detector column, 0 = per ray */
   int fp_grid;        /* persistent workgroups of the forward launch (0: one per item) */
   int fp_strided;     /* 1: interleaved item ranges, 0: contiguous */
-  int bp_zg;          /* back projector: z groups per lane 1..4, 0: each scan's ceil(ZN/64),
-                         5: windowed (one wave per column over all z, sums in LDS) */
+  int bp_zg;          /* back projector of columns over 2048 voxels: z groups per lane 1..4,
+                         0 or 5: each scan's ceil(ZN/64); shorter columns always run windowed
+                         (one wave per column over all z, sums in LDS) */
   int bp_grid;        /* persistent workgroups of the back-projection launch (0: one per item) */
   int bp_strided;     /* 1: interleaved item ranges, 0: contiguous */
   double setup_ms;    /* row / column sums of all scans */
