@@ -884,6 +884,10 @@ __device__ __forceinline__ void pipelined(uint64_t m, Fetch fetch, Use use) {
 // loads its row of the view's columns (the next view's rows load meanwhile) and combines
 // them (R[v] = sum_u w_u y[u][v]) into LDS, four rows of zeros on either side, and a voxel
 // takes the three rows that its shadow [T, T + s] can overlap, without clamps.
+// Bound by VALU issue (0.96 of the chip's rate).  512^2 x 256, 197 views of 888 x 64:
+// 3.76 ms with the views in order, four column loads and two-row clamps for each, 2.51 ms
+// (BF16 sinogram 3.85 ms, 2.51 ms); 277^2 x 165, 164 views of 611 x 80 in BF16, without
+// staged rows 1.78 ms, with two chunks of rows 0.69 ms.
 constexpr int kPadRows = 4;
 template <int RC>
 constexpr int kRowsLds = 64 * RC + 3 * kPadRows;  // zeros, rows, zeros, a slot for idle lanes
@@ -1724,7 +1728,9 @@ struct MatchedCols {
 // evaluates view k0 + l (columns, T0 and s in FP64); the row sets hold w_t y[u + t][v].
 // Views of more than four columns, of more than three rows per voxel, or whose columns'
 // rows differ by over a row across the window take the row walk.
-// bound by VALU issue as bp_staged_body, with about 11 instructions per column and pass.
+// Bound by VALU issue (0.73 of the chip's rate) and the texture unit's row loads.  256^2 x
+// 128, 197 views of 888 x 64: 3.94 ms with a search and a gather of the rows per voxel
+// (bp_matched_win_kernel), 0.88 ms; 512^2 x 256: 18.0 ms, 4.0 ms.
 template <int RC>
 constexpr int kMatchedF = 4 * kRowsLds<RC> + 64 * 16;
 __host__ __device__ constexpr int bp_matched_floats(int RC, int ZN) {
@@ -2187,7 +2193,8 @@ int launch_bp(const Plan& P, const T* prj, float* vol, int vb, int vs, int vc, i
 #undef CTR_BPMS
         return check_launch("bp_matched_staged_kernel");
       }
-      // windowed kernel while its row table and column sums fit 64 KiB of LDS
+      // (unevenly spaced or over 256 rows) the searching windowed kernel while its row table
+      // and column sums fit 64 KiB of LDS
       const size_t lds =
           ((size_t)((P.d.DNV + 1 + 3) & ~3) + (size_t)kWaves * P.d.ZN) * sizeof(float);
       if (P.d.ZN <= kWinMaxZ && lds <= 65536) {

@@ -78,10 +78,10 @@ struct ctr_unet {
   Buf params, grads, m, v;
   Buf wf[kNL], wb[kNL];
   // activations (level 1 / 2 / 3 grids)
-  Buf in0, a0, cat1, p1, a2, cat2, p2, a4, b3, a6, d2, a8, d1, h;
+  Buf in0, a0, s1, p1, a2, s2, p2, a4, b3, a6, d2, a8, d1, h;
   // gradients
   Buf gA1, gB1, gC1, gA2, gB2, gC2, gB3, gC3, gP3, gP2, dh;
-  Buf wpart, bpart, dpart, loss;
+  Buf wpart, bpart, dpart, lpart;
 };
 
 namespace {
@@ -110,22 +110,21 @@ int ensure_buffers(ctr_unet& N, long long V, bool train) {
   struct Req {
     Buf* buf;
     size_t bytes;
-  } fwd[] = {{&N.in0, V1 * 8 * b},  {&N.a0, V1 * 16 * b}, {&N.cat1, V1 * 48 * b},
-             {&N.p1, V2 * 16 * b},  {&N.a2, V2 * 32 * b}, {&N.cat2, V2 * 96 * b},
-             {&N.p2, V3 * 32 * b},  {&N.a4, V3 * 64 * b}, {&N.b3, V3 * 64 * b},
-             {&N.a6, V2 * 32 * b},  {&N.d2, V2 * 32 * b}, {&N.a8, V1 * 16 * b},
-             {&N.d1, V1 * 16 * b},  {&N.h, V1 * 4}};
+  } fwd[] = {{&N.a0, V1 * 16 * b}, {&N.s1, V1 * 16 * b}, {&N.p1, V2 * 16 * b},
+             {&N.a2, V2 * 32 * b}, {&N.s2, V2 * 32 * b}, {&N.p2, V3 * 32 * b},
+             {&N.a4, V3 * 64 * b}, {&N.b3, V3 * 64 * b}, {&N.a6, V2 * 32 * b},
+             {&N.d2, V2 * 32 * b}, {&N.a8, V1 * 16 * b}};
   for (auto& r : fwd)
     if ((rc = r.buf->ensure(r.bytes))) return rc;
   if (!train) return CTR_OK;
-  const int nsplit = 64;
-  size_t wmax = 0;
-  for (int l = 0; l < kNL; ++l) wmax = std::max(wmax, (size_t)27 * kL[l].cin * kL[l].cout);
-  Req bwd[] = {{&N.gA1, V1 * 48 * b}, {&N.gB1, V1 * 16 * b},  {&N.gC1, V1 * 16 * b},
+  Req bwd[] = {{&N.in0, V1 * 8 * b},  {&N.d1, V1 * 16 * b},   {&N.h, V1 * 4},
+               {&N.gA1, V1 * 48 * b}, {&N.gB1, V1 * 16 * b},  {&N.gC1, V1 * 16 * b},
                {&N.gA2, V2 * 96 * b}, {&N.gB2, V2 * 32 * b},  {&N.gC2, V2 * 32 * b},
                {&N.gB3, V3 * 64 * b}, {&N.gC3, V3 * 64 * b},  {&N.gP3, V3 * 32 * b},
-               {&N.gP2, V2 * 16 * b}, {&N.dh, V1 * 4},         {&N.wpart, (size_t)nsplit * wmax * 4},
-               {&N.bpart, (size_t)nsplit * 64 * 4}, {&N.dpart, (size_t)1024 * 17 * 8}, {&N.loss, 8}};
+               {&N.gP2, V2 * 16 * b}, {&N.dh, V1 * 4},
+               {&N.wpart, (size_t)kWgradBlocks * 27 * 16 * 32 * 4},
+               {&N.bpart, (size_t)kWgradBlocks * 64 * 4},
+               {&N.dpart, (size_t)1024 * 17 * 8}, {&N.lpart, (size_t)1024 * 8}};
   for (auto& r : bwd)
     if ((rc = r.buf->ensure(r.bytes))) return rc;
   return CTR_OK;
@@ -137,99 +136,122 @@ int ensure_buffers(ctr_unet& N, long long V, bool train) {
     if (rc_) return rc_;  \
   } while (0)
 
-int forward(ctr_unet& N, const float* x, const float* d, Grid3 g1, float head_scale,
+// Inputs of the decoder's first layers: the skip, then the upsampled coarser level.
+ConvIn cat1(ctr_unet& N) { return ConvIn{N.s1.h(), 16, 16, N.d2.h(), 32}; }
+ConvIn cat2(ctr_unet& N) { return ConvIn{N.s2.h(), 32, 32, N.b3.h(), 64}; }
+
+// The network on x, d.  train: every activation that backward() reads is kept (the packed
+// input, the head's input and output N.h, head scale 1); otherwise the head's output times
+// s_out goes straight to `update`.
+int forward(ctr_unet& N, const float* x, const float* d, Grid3 g1, bool train, float* update,
             hipStream_t st) {
   const long long V1 = (long long)g1.Y * g1.X * g1.Z;
   const Grid3 g2{g1.Y / 2, g1.X / 2, g1.Z / 2}, g3{g1.Y / 4, g1.X / 4, g1.Z / 4};
   const float* P = N.params.f();
-  auto B = [&](int l) { return P + kLay.boff[l]; };
   TRY(refresh_weights(N, st));
-  TRY(pack_input(x, d, N.s_x, N.s_d, V1, N.in0.h(), st));
-  TRY(conv3(N.in0.h(), 8, 8, N.wf[0].h(), B(0), N.a0.h(), 16, 16, true, g1, st));
-  TRY(conv3(N.a0.h(), 16, 16, N.wf[1].h(), B(1), N.cat1.h(), 48, 16, true, g1, st));  // s1
-  TRY(pool(N.cat1.h(), 48, 16, g1, N.p1.h(), 16, st));
-  TRY(conv3(N.p1.h(), 16, 16, N.wf[2].h(), B(2), N.a2.h(), 32, 32, true, g2, st));
-  TRY(conv3(N.a2.h(), 32, 32, N.wf[3].h(), B(3), N.cat2.h(), 96, 32, true, g2, st));  // s2
-  TRY(pool(N.cat2.h(), 96, 32, g2, N.p2.h(), 32, st));
-  TRY(conv3(N.p2.h(), 32, 32, N.wf[4].h(), B(4), N.a4.h(), 64, 64, true, g3, st));
-  TRY(conv3(N.a4.h(), 64, 64, N.wf[5].h(), B(5), N.b3.h(), 64, 64, true, g3, st));
-  TRY(upsample(N.b3.h(), 64, 64, g2, N.cat2.h() + 32, 96, st));
-  TRY(conv3(N.cat2.h(), 96, 96, N.wf[6].h(), B(6), N.a6.h(), 32, 32, true, g2, st));
-  TRY(conv3(N.a6.h(), 32, 32, N.wf[7].h(), B(7), N.d2.h(), 32, 32, true, g2, st));
-  TRY(upsample(N.d2.h(), 32, 32, g1, N.cat1.h() + 16, 48, st));
-  TRY(conv3(N.cat1.h(), 48, 48, N.wf[8].h(), B(8), N.a8.h(), 16, 16, true, g1, st));
-  TRY(conv3(N.a8.h(), 16, 16, N.wf[9].h(), B(9), N.d1.h(), 16, 16, true, g1, st));
-  return head(N.d1.h(), P + kLay.head, V1, head_scale, N.h.f(), st);
+  // layer l with ReLU into out (channel stride = its channel count), pooled into p if set
+  auto layer = [&](int l, const ConvIn& in, uint16_t* out, Grid3 g, uint16_t* p) {
+    ConvOut o;
+    o.out = out;
+    o.cs_out = kL[l].cout;
+    o.relu = 1;
+    o.pool = p;
+    o.cs_pool = kL[l].cout;
+    return conv3(in, kL[l].cin, N.wf[l].h(), P + kLay.boff[l], kL[l].cout, o, g, st);
+  };
+  ConvIn in0;
+  if (train) {
+    TRY(pack_input(x, d, N.s_x, N.s_d, V1, N.in0.h(), st));
+    in0 = conv_in(N.in0.h(), 8);
+  } else {
+    in0.fx = x;
+    in0.fd = d;
+    in0.s0 = N.s_x;
+    in0.s1 = N.s_d;
+  }
+  TRY(layer(0, in0, N.a0.h(), g1, nullptr));
+  TRY(layer(1, conv_in(N.a0.h(), 16), N.s1.h(), g1, N.p1.h()));
+  TRY(layer(2, conv_in(N.p1.h(), 16), N.a2.h(), g2, nullptr));
+  TRY(layer(3, conv_in(N.a2.h(), 32), N.s2.h(), g2, N.p2.h()));
+  TRY(layer(4, conv_in(N.p2.h(), 32), N.a4.h(), g3, nullptr));
+  TRY(layer(5, conv_in(N.a4.h(), 64), N.b3.h(), g3, nullptr));
+  TRY(layer(6, cat2(N), N.a6.h(), g2, nullptr));
+  TRY(layer(7, conv_in(N.a6.h(), 32), N.d2.h(), g2, nullptr));
+  TRY(layer(8, cat1(N), N.a8.h(), g1, nullptr));
+  if (train) {
+    TRY(layer(9, conv_in(N.a8.h(), 16), N.d1.h(), g1, nullptr));
+    return head(N.d1.h(), P + kLay.head, V1, 1.f, N.h.f(), st);
+  }
+  ConvOut o;
+  o.relu = 1;
+  o.head = P + kLay.head;
+  o.hscale = N.s_out;
+  o.h = update;
+  return conv3(conv_in(N.a8.h(), 16), 16, N.wf[9].h(), P + kLay.boff[9], 16, o, g1, st);
 }
 
 // Loss and gradients of the last forward pass (head scale 1) against target t.
 int backward(ctr_unet& N, const float* t, Grid3 g1, hipStream_t st, double* loss) {
-  const long long V1 = (long long)g1.Y * g1.X * g1.Z, V2 = V1 / 8, V3 = V1 / 64;
+  const long long V1 = (long long)g1.Y * g1.X * g1.Z;
   const Grid3 g2{g1.Y / 2, g1.X / 2, g1.Z / 2}, g3{g1.Y / 4, g1.X / 4, g1.Z / 4};
   const float* P = N.params.f();
   float* G = N.grads.f();
-  auto GW = [&](int l) { return G + kLay.woff[l]; };
-  auto GB = [&](int l) { return G + kLay.boff[l]; };
-  float* wp = N.wpart.f();
-  float* bp = N.bpart.f();
   long long nb = (V1 + 255) / 256;
   if (nb > 1024) nb = 1024;
-  TRY(mse(N.h.f(), t, 1.f / N.s_out, V1, N.dh.f(), N.dpart.d(), (int)nb, st));
+  // weight gradient of layer l from its input and output gradient
+  auto wg = [&](int l, const ConvIn& X, const uint16_t* dY, int cs, Grid3 g) {
+    return wgrad(X, kL[l].cin, dY, cs, kL[l].cout, g, N.wpart.f(), N.bpart.f(),
+                 G + kLay.woff[l], G + kLay.boff[l], st);
+  };
+  // gradient of layer l's input (stride: its channel count), masked by the ReLU of y if set
+  auto dx = [&](int l, const uint16_t* dY, int cs, uint16_t* out, const uint16_t* y, Grid3 g) {
+    ConvOut o;
+    o.out = out;
+    o.cs_out = kL[l].cin;
+    o.gate = y;
+    o.cs_gate = kL[l].cin;
+    return conv3(conv_in(dY, cs), kL[l].cout, N.wb[l].h(), nullptr, kL[l].cin, o, g, st);
+  };
+  TRY(mse(N.h.f(), t, 1.f / N.s_out, V1, N.dh.f(), (double*)N.lpart.p, (int)nb, st));
+  // head (with the ReLU of d1b)
+  TRY(head_bwd(N.d1.h(), P + kLay.head, N.dh.f(), V1, N.gB1.h(), N.dpart.d(), (int)nb,
+               G + kLay.head, st));
+  TRY(wg(9, conv_in(N.a8.h(), 16), N.gB1.h(), 16, g1));
+  TRY(dx(9, N.gB1.h(), 16, N.gC1.h(), N.a8.h(), g1));
+  TRY(wg(8, cat1(N), N.gC1.h(), 16, g1));
+  TRY(dx(8, N.gC1.h(), 16, N.gA1.h(), nullptr, g1));
+  TRY(upsample_bwd(N.gA1.h() + 16, 48, 32, g1, N.gB2.h(), 32, N.d2.h(), 32, st));
+  TRY(wg(7, conv_in(N.a6.h(), 32), N.gB2.h(), 32, g2));
+  TRY(dx(7, N.gB2.h(), 32, N.gC2.h(), N.a6.h(), g2));
+  TRY(wg(6, cat2(N), N.gC2.h(), 32, g2));
+  TRY(dx(6, N.gC2.h(), 32, N.gA2.h(), nullptr, g2));
+  TRY(upsample_bwd(N.gA2.h() + 32, 96, 64, g2, N.gB3.h(), 64, N.b3.h(), 64, st));
+  TRY(wg(5, conv_in(N.a4.h(), 64), N.gB3.h(), 64, g3));
+  TRY(dx(5, N.gB3.h(), 64, N.gC3.h(), N.a4.h(), g3));
+  TRY(wg(4, conv_in(N.p2.h(), 32), N.gC3.h(), 64, g3));
+  TRY(dx(4, N.gC3.h(), 64, N.gP3.h(), nullptr, g3));
+  // d s2 = skip part of d cat2 + pooling adjoint
+  TRY(pool_bwd(N.gP3.h(), 32, 32, g2, N.gA2.h(), 96, N.s2.h(), 32, st));
+  TRY(wg(3, conv_in(N.a2.h(), 32), N.gA2.h(), 96, g2));
+  TRY(dx(3, N.gA2.h(), 96, N.gB2.h(), N.a2.h(), g2));
+  TRY(wg(2, conv_in(N.p1.h(), 16), N.gB2.h(), 32, g2));
+  TRY(dx(2, N.gB2.h(), 32, N.gP2.h(), nullptr, g2));
+  // d s1 = skip part of d cat1 + pooling adjoint
+  TRY(pool_bwd(N.gP2.h(), 16, 16, g1, N.gA1.h(), 48, N.s1.h(), 16, st));
+  TRY(wg(1, conv_in(N.a0.h(), 16), N.gA1.h(), 48, g1));
+  TRY(dx(1, N.gA1.h(), 48, N.gB1.h(), N.a0.h(), g1));
+  TRY(wg(0, conv_in(N.in0.h(), 8), N.gB1.h(), 16, g1));
   if (loss) {
     std::vector<double> h(nb);
-    if (hipMemcpyAsync(h.data(), N.dpart.p, nb * sizeof(double), hipMemcpyDeviceToHost, st) !=
+    if (hipMemcpyAsync(h.data(), N.lpart.p, nb * sizeof(double), hipMemcpyDeviceToHost, st) !=
             hipSuccess ||
         hipStreamSynchronize(st) != hipSuccess)
       return fail(CTR_ERR_HIP, "loss readback");
     double s = 0;
-    for (double x : h) s += x;
+    for (double v : h) s += v;
     *loss = s / (2.0 * (double)V1);
   }
-  // head (with the ReLU of d1b)
-  TRY(head_bwd(N.d1.h(), P + kLay.head, N.dh.f(), V1, N.gB1.h(), N.dpart.d(), (int)nb,
-               G + kLay.head, st));
-  // d1b: input a8
-  TRY(wgrad(N.a8.h(), 16, 16, N.gB1.h(), 16, 16, g1, wp, bp, GW(9), GB(9), st));
-  TRY(conv3(N.gB1.h(), 16, 16, N.wb[9].h(), nullptr, N.gC1.h(), 16, 16, false, g1, st));
-  TRY(relu_bwd(N.a8.h(), 16, N.gC1.h(), 16, 16, V1, N.gC1.h(), 16, st));
-  // d1a: input cat1
-  TRY(wgrad(N.cat1.h(), 48, 48, N.gC1.h(), 16, 16, g1, wp, bp, GW(8), GB(8), st));
-  TRY(conv3(N.gC1.h(), 16, 16, N.wb[8].h(), nullptr, N.gA1.h(), 48, 48, false, g1, st));
-  TRY(upsample_bwd(N.gA1.h() + 16, 48, 32, g1, N.gB2.h(), 32, st));
-  TRY(relu_bwd(N.d2.h(), 32, N.gB2.h(), 32, 32, V2, N.gB2.h(), 32, st));
-  // d2b: input a6
-  TRY(wgrad(N.a6.h(), 32, 32, N.gB2.h(), 32, 32, g2, wp, bp, GW(7), GB(7), st));
-  TRY(conv3(N.gB2.h(), 32, 32, N.wb[7].h(), nullptr, N.gC2.h(), 32, 32, false, g2, st));
-  TRY(relu_bwd(N.a6.h(), 32, N.gC2.h(), 32, 32, V2, N.gC2.h(), 32, st));
-  // d2a: input cat2
-  TRY(wgrad(N.cat2.h(), 96, 96, N.gC2.h(), 32, 32, g2, wp, bp, GW(6), GB(6), st));
-  TRY(conv3(N.gC2.h(), 32, 32, N.wb[6].h(), nullptr, N.gA2.h(), 96, 96, false, g2, st));
-  TRY(upsample_bwd(N.gA2.h() + 32, 96, 64, g2, N.gB3.h(), 64, st));
-  TRY(relu_bwd(N.b3.h(), 64, N.gB3.h(), 64, 64, V3, N.gB3.h(), 64, st));
-  // e3b: input a4
-  TRY(wgrad(N.a4.h(), 64, 64, N.gB3.h(), 64, 64, g3, wp, bp, GW(5), GB(5), st));
-  TRY(conv3(N.gB3.h(), 64, 64, N.wb[5].h(), nullptr, N.gC3.h(), 64, 64, false, g3, st));
-  TRY(relu_bwd(N.a4.h(), 64, N.gC3.h(), 64, 64, V3, N.gC3.h(), 64, st));
-  // e3a: input p2
-  TRY(wgrad(N.p2.h(), 32, 32, N.gC3.h(), 64, 64, g3, wp, bp, GW(4), GB(4), st));
-  TRY(conv3(N.gC3.h(), 64, 64, N.wb[4].h(), nullptr, N.gP3.h(), 32, 32, false, g3, st));
-  TRY(pool_bwd(N.gP3.h(), 32, 32, g2, N.gA2.h(), 96, st));  // d s2 += pool adjoint
-  TRY(relu_bwd(N.cat2.h(), 96, N.gA2.h(), 96, 32, V2, N.gA2.h(), 96, st));
-  // e2b: input a2, gradient = gA2[:, :32]
-  TRY(wgrad(N.a2.h(), 32, 32, N.gA2.h(), 96, 32, g2, wp, bp, GW(3), GB(3), st));
-  TRY(conv3(N.gA2.h(), 96, 32, N.wb[3].h(), nullptr, N.gB2.h(), 32, 32, false, g2, st));
-  TRY(relu_bwd(N.a2.h(), 32, N.gB2.h(), 32, 32, V2, N.gB2.h(), 32, st));
-  // e2a: input p1
-  TRY(wgrad(N.p1.h(), 16, 16, N.gB2.h(), 32, 32, g2, wp, bp, GW(2), GB(2), st));
-  TRY(conv3(N.gB2.h(), 32, 32, N.wb[2].h(), nullptr, N.gP2.h(), 16, 16, false, g2, st));
-  TRY(pool_bwd(N.gP2.h(), 16, 16, g1, N.gA1.h(), 48, st));  // d s1 += pool adjoint
-  TRY(relu_bwd(N.cat1.h(), 48, N.gA1.h(), 48, 16, V1, N.gA1.h(), 48, st));
-  // e1b: input a0, gradient = gA1[:, :16]
-  TRY(wgrad(N.a0.h(), 16, 16, N.gA1.h(), 48, 16, g1, wp, bp, GW(1), GB(1), st));
-  TRY(conv3(N.gA1.h(), 48, 16, N.wb[1].h(), nullptr, N.gB1.h(), 16, 16, false, g1, st));
-  TRY(relu_bwd(N.a0.h(), 16, N.gB1.h(), 16, 16, V1, N.gB1.h(), 16, st));
-  // e1a: input in0
-  return wgrad(N.in0.h(), 8, 8, N.gB1.h(), 16, 16, g1, wp, bp, GW(0), GB(0), st);
+  return CTR_OK;
 }
 
 }  // namespace
@@ -316,11 +338,8 @@ int ctr_unet_forward(ctr_unet* net, const float* d_x, const float* d_delta, floa
   if (rc) return rc;
   CTR_HIP(hipSetDevice(net->device));
   hipStream_t st = (hipStream_t)stream;
-  const long long V = (long long)Y * X * Z;
-  if ((rc = ensure_buffers(*net, V, false))) return rc;
-  if ((rc = forward(*net, d_x, d_delta, Grid3{Y, X, Z}, net->s_out, st))) return rc;
-  CTR_HIP(hipMemcpyAsync(d_update, net->h.p, V * sizeof(float), hipMemcpyDeviceToDevice, st));
-  return CTR_OK;
+  if ((rc = ensure_buffers(*net, (long long)Y * X * Z, false))) return rc;
+  return forward(*net, d_x, d_delta, Grid3{Y, X, Z}, false, d_update, st);
 }
 
 int ctr_unet_loss_grad(ctr_unet* net, const float* d_x, const float* d_delta,
@@ -333,7 +352,7 @@ int ctr_unet_loss_grad(ctr_unet* net, const float* d_x, const float* d_delta,
   const long long V = (long long)Y * X * Z;
   if ((rc = ensure_buffers(*net, V, true))) return rc;
   const Grid3 g{Y, X, Z};
-  if ((rc = forward(*net, d_x, d_delta, g, 1.f, nullptr))) return rc;
+  if ((rc = forward(*net, d_x, d_delta, g, true, nullptr, nullptr))) return rc;
   if ((rc = backward(*net, d_target, g, nullptr, loss))) return rc;
   if (host_grads)
     CTR_HIP(hipMemcpy(host_grads, net->grads.p, kLay.n * sizeof(float), hipMemcpyDeviceToHost));
@@ -351,7 +370,7 @@ int ctr_unet_train_step(ctr_unet* net, const float* d_x, const float* d_delta,
   const long long V = (long long)Y * X * Z;
   if ((rc = ensure_buffers(*net, V, true))) return rc;
   const Grid3 g{Y, X, Z};
-  if ((rc = forward(*net, d_x, d_delta, g, 1.f, nullptr))) return rc;
+  if ((rc = forward(*net, d_x, d_delta, g, true, nullptr, nullptr))) return rc;
   if ((rc = backward(*net, d_target, g, nullptr, loss))) return rc;
   net->step += 1;
   if ((rc = adam(net->params.f(), net->grads.f(), net->m.f(), net->v.f(), kLay.n, lr, 0.9f,
