@@ -135,12 +135,47 @@ struct ReduceItem {
   double* out;
 };
 
+// Line of detector column boundary `e` (x, y) in a view rotated by (c, s) with its source at
+// (sx, sy): (a, f) of t(ii) = a + ii f, the in-plane cell coordinate on slice ii.
+__host__ __device__ inline double2 boundary_line(double2 e, double c, double s, double sx,
+                                                 double sy, bool xmarch, double ocx, double ocy,
+                                                 double dx, double half) {
+#pragma clang fp contract(off)
+  const double Bx = e.x * c - e.y * s, By = e.x * s + e.y * c;
+  if (xmarch) {
+    const double f = (By - sy) / (Bx - sx);
+    return make_double2(((-ocx * dx - Bx) * f + By) / dx + ocy + half, f);
+  }
+  const double f = (Bx - sx) / (By - sy);
+  return make_double2(((-ocy * dx - By) * f + Bx) / dx + ocx + half, f);
+}
+
+// What launch_plan_tables reads (uploaded) and fills; see Plan for the tables.
+struct PlanTables {
+  int PN, DNU, DNV, XN, YN;
+  double ocx, ocy, dx, dz, z0, half;
+  const ViewP* views;
+  const double2 *src64, *rot64, *det64;
+  const double2* edge64;  // [DNU+1] column boundaries (x, y)
+  const double* bz64;     // [DNV+1] row boundaries
+  const double* zds64;    // [DNV]
+  const uint8_t* mask;
+  float2* bnd;
+  double2* bnd64;
+  float4* cols;
+  float *Bz, *dBz, *h2, *invdB, *zc, *maskf;
+  float2* mext;
+};
+int launch_plan_tables(const PlanTables& T, hipStream_t st);
+
 struct Plan {
   int device = 0;
   Dims d{};
   BpConsts bc{};
   BpConsts64 bc64{};
-  // device tables
+  // device tables: views, src64, rot64, sz64, det64 and mask lie in `uploaded`, the rest are
+  // computed on the device (launch_plan_tables)
+  void* uploaded = nullptr;
   ViewP* views = nullptr;      // [PN]
   double2* src64 = nullptr;    // [PN]         rotated source (x, y) in FP64
   float2* bnd = nullptr;       // [PN][DNU+1]  (a_b, f_b): t_b(ii) = a_b + ii*f_b

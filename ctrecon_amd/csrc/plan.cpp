@@ -89,15 +89,36 @@ bool finite_array(const float* a, int n) {
   return true;
 }
 
-template <typename T>
-int upload(T** dst, const std::vector<T>& src) {
-  if (dev_malloc((void**)dst, sizeof(T) * std::max<size_t>(src.size(), 1)) != hipSuccess) {
-    *dst = nullptr;
-    return fail(CTR_ERR_NOMEM, "cannot allocate the plan's geometry tables");
-  }
-  CTR_HIP(hipMemcpy(*dst, src.data(), sizeof(T) * src.size(), hipMemcpyHostToDevice));
-  return CTR_OK;
+int table_alloc(void** p, size_t bytes) {
+  if (dev_malloc(p, bytes) == hipSuccess) return CTR_OK;
+  *p = nullptr;
+  return fail(CTR_ERR_NOMEM, "cannot allocate the plan's geometry tables");
 }
+
+// Tables packed into one host buffer, 256-byte aligned, for one copy to the device.
+struct Packed {
+  std::vector<char> h;
+  std::vector<std::pair<const void**, size_t>> at;  // device pointer to set, offset
+  template <typename T>
+  T* add(T** dst, size_t n) {  // valid until the next add
+    const size_t o = (h.size() + 255) & ~(size_t)255;
+    h.resize(o + n * sizeof(T));
+    at.emplace_back((const void**)dst, o);
+    return (T*)(h.data() + o);
+  }
+  template <typename T, typename S>
+  void add(T** dst, const std::vector<S>& v) {
+    using V = std::remove_const_t<T>;
+    std::copy(v.begin(), v.end(), const_cast<V*>(add(dst, v.size())));
+  }
+  int upload(void** dev) {
+    int rc = table_alloc(dev, h.size());
+    if (rc) return rc;
+    CTR_HIP(hipMemcpy(*dev, h.data(), h.size(), hipMemcpyHostToDevice));
+    for (auto& a : at) *a.first = (const char*)*dev + a.second;
+    return CTR_OK;
+  }
+};
 
 int validate_geometry(const ctr_geometry* g) {
   if (!g) return fail(CTR_ERR_ARG, "geometry is NULL");
@@ -122,7 +143,8 @@ int validate_geometry(const ctr_geometry* g) {
 
 }  // namespace
 
-// Builds every table of the plan in FP64 on the host.
+// Builds every table of the plan in FP64: per-view and per-row values on the host, the rest on
+// the device (null stream; not waited for).
 // half: 0, or 0.5 to move the footprints of the forward projector half a cell along the
 // in-plane axis across the rays and along z (the sampling of the reference's FP64
 // branchless projector, DD3_GPU.cu:350-360 / 414-422).
@@ -141,20 +163,13 @@ static int build_tables(const ctr_geometry* g, Plan& P, double half = 0.0) {
                             bz = boundaries(g->zds, DNV);
 
   // rows
-  std::vector<float> Bz(DNV + 1), dBz(DNV), h2(DNV), invdB(DNV);
-  for (int v = 0; v <= DNV; ++v) Bz[v] = (float)((bz[v] - z0) / dz);
-  for (int v = 0; v < DNV; ++v) {
-    const double h = g->zds[v] - z0;
-    h2[v] = (float)(h * h);
-    invdB[v] = (float)(dz / (bz[v + 1] - bz[v]));
-    dBz[v] = (float)((bz[v + 1] - bz[v]) / dz);
-  }
-  d.B0 = Bz[0];
+  auto Bz = [&](int v) { return (float)((bz[v] - z0) / dz); };
+  d.B0 = Bz(0);
   d.dB = (float)((bz[DNV] - bz[0]) / dz / DNV);
-  d.dBmin = Bz[1] - Bz[0];
-  for (int v = 1; v < DNV; ++v) d.dBmin = std::min(d.dBmin, Bz[v + 1] - Bz[v]);
-
-  d.dBmax = *std::max_element(dBz.begin(), dBz.end());
+  d.dBmin = Bz(1) - Bz(0);
+  for (int v = 1; v < DNV; ++v) d.dBmin = std::min(d.dBmin, Bz(v + 1) - Bz(v));
+  d.dBmax = (float)((bz[1] - bz[0]) / dz);
+  for (int v = 1; v < DNV; ++v) d.dBmax = std::max(d.dBmax, (float)((bz[v + 1] - bz[v]) / dz));
   d.B0_64 = (bz[0] - z0) / dz;
   d.dB_64 = (bz[DNV] - bz[0]) / dz / DNV;
   {
@@ -215,14 +230,10 @@ static int build_tables(const ctr_geometry* g, Plan& P, double half = 0.0) {
 
   // per-view tables
   std::vector<ViewP> views(PN);
-  std::vector<double2> src64(PN), rot64(PN), det64(DNU);
-  std::vector<double> sz64(PN);
-  std::vector<float> zc(DNV);
+  std::vector<double2> src64(PN), rot64(PN), det64(DNU), edge64(DNU + 1);
+  std::vector<double> sz64(PN), zds64(g->zds, g->zds + DNV);
   for (int u = 0; u < DNU; ++u) det64[u] = make_double2(g->xds[u], g->yds[u]);
-  for (int v = 0; v < DNV; ++v) zc[v] = (float)((g->zds[v] - z0) / dz);
-  std::vector<float2> bnd((size_t)PN * (DNU + 1));
-  std::vector<double2> bnd64((size_t)PN * (DNU + 1));
-  std::vector<float4> cols((size_t)PN * DNU);
+  for (int b = 0; b <= DNU; ++b) edge64[b] = make_double2(bx[b], by[b]);
   for (int p = 0; p < PN; ++p) {
     const double th = regularize((double)g->angles[p]);
     const double c = std::cos(th), s = std::sin(th);
@@ -241,40 +252,11 @@ static int build_tables(const ctr_geometry* g, Plan& P, double half = 0.0) {
     vp.wx = std::fabs(sx) > std::fabs(sy) ? 1 : 0;  // DD3_GPU.cu:1453
     const int NS = vp.xmarch ? g->XN : g->YN;
     const double mid = 0.5 * (NS - 1);
-    for (int b = 0; b <= DNU; ++b) {
-      const double Bx = bx[b] * c - by[b] * s, By = bx[b] * s + by[b] * c;
-      double f, a;
-      if (vp.xmarch) {
-        f = (By - sy) / (Bx - sx);
-        a = ((-ocx * dx - Bx) * f + By) / dx + ocy + half;
-      } else {
-        f = (Bx - sx) / (By - sy);
-        a = ((-ocy * dx - By) * f + Bx) / dx + ocx + half;
-      }
-      bnd[(size_t)p * (DNU + 1) + b] = make_float2((float)a, (float)f);
-      bnd64[(size_t)p * (DNU + 1) + b] = make_double2(a, f);
-    }
-    {
-      const float2 b0 = bnd[(size_t)p * (DNU + 1)], bN = bnd[(size_t)p * (DNU + 1) + DNU];
-      vp.bdir = ((bN.x + mid * bN.y) >= (b0.x + mid * b0.y)) ? 1 : -1;
-    }
-    for (int u = 0; u < DNU; ++u) {
-      const double Dx = (double)g->xds[u] * c - (double)g->yds[u] * s;
-      const double Dy = (double)g->xds[u] * s + (double)g->yds[u] * c;
-      const double ex = Dx - sx, ey = Dy - sy;
-      double r0, r1, Q;
-      if (vp.xmarch) {
-        r0 = (-ocx * dx - sx) / ex;
-        r1 = dx / ex;
-        Q = dx / std::fabs(ex);
-      } else {
-        r0 = (-ocy * dx - sy) / ey;
-        r1 = dx / ey;
-        Q = dx / std::fabs(ey);
-      }
-      cols[(size_t)p * DNU + u] = make_float4((float)r0, (float)r1, (float)(ex * ex + ey * ey),
-                                              (float)Q);
-    }
+    auto mid_of = [&](int b) {
+      const double2 l = boundary_line(edge64[b], c, s, sx, sy, vp.xmarch, ocx, ocy, dx, half);
+      return (float)l.x + mid * (float)l.y;
+    };
+    vp.bdir = mid_of(DNU) >= mid_of(0) ? 1 : -1;
   }
   P.h_views = views;
   {
@@ -290,54 +272,45 @@ static int build_tables(const ctr_geometry* g, Plan& P, double half = 0.0) {
     h.bzN = bz[DNV] - z0;
   }
 
-  std::vector<uint8_t> mask((size_t)g->XN * g->YN, 1);
-  if (g->mask) std::memcpy(mask.data(), g->mask, mask.size());
-
-  // per-slice extent of the non-zero mask: x-slices (cells along y), then y-slices
-  std::vector<float2> mext(g->XN + g->YN);
-  for (int x = 0; x < g->XN; ++x) {
-    int lo = g->YN, hi = -1;
-    for (int y = 0; y < g->YN; ++y)
-      if (mask[(size_t)y * g->XN + x]) { lo = std::min(lo, y); hi = std::max(hi, y); }
-    mext[x] = (hi >= lo) ? make_float2(lo - 0.5f, hi + 0.5f) : make_float2(0.f, -1.f);
-  }
-  for (int y = 0; y < g->YN; ++y) {
-    int lo = g->XN, hi = -1;
-    for (int x = 0; x < g->XN; ++x)
-      if (mask[(size_t)y * g->XN + x]) { lo = std::min(lo, x); hi = std::max(hi, x); }
-    mext[g->XN + y] = (hi >= lo) ? make_float2(lo - 0.5f, hi + 0.5f) : make_float2(0.f, -1.f);
-  }
-
-  std::vector<float> maskf(mask.begin(), mask.end());
-
+  PlanTables T{PN, DNU, DNV, g->XN, g->YN, ocx, ocy, dx, dz, z0, half};
+  Packed up;
+  up.add(&P.views, views);
+  up.add(&P.src64, src64);
+  up.add(&P.rot64, rot64);
+  up.add(&P.sz64, sz64);
+  up.add(&P.det64, det64);
+  up.add(&T.edge64, edge64);
+  up.add(&T.bz64, bz);
+  up.add(&T.zds64, zds64);
+  const size_t cells = (size_t)g->XN * g->YN;
+  uint8_t* mask = up.add(&P.mask, cells);
+  if (g->mask) std::memcpy(mask, g->mask, cells);
+  else std::memset(mask, 1, cells);
   int rc;
-  if ((rc = upload(&P.mext, mext))) return rc;
-  if ((rc = upload(&P.maskf, maskf))) return rc;
-  if ((rc = upload(&P.views, views))) return rc;
-  if ((rc = upload(&P.src64, src64))) return rc;
-  if ((rc = upload(&P.rot64, rot64))) return rc;
-  if ((rc = upload(&P.sz64, sz64))) return rc;
-  if ((rc = upload(&P.det64, det64))) return rc;
-  if ((rc = upload(&P.zc, zc))) return rc;
-  if ((rc = upload(&P.bnd, bnd))) return rc;
-  if ((rc = upload(&P.bnd64, bnd64))) return rc;
-  if ((rc = upload(&P.cols, cols))) return rc;
-  if ((rc = upload(&P.Bz, Bz))) return rc;
-  if ((rc = upload(&P.dBz, dBz))) return rc;
-  if ((rc = upload(&P.h2, h2))) return rc;
-  if ((rc = upload(&P.invdB, invdB))) return rc;
-  if ((rc = upload(&P.mask, mask))) return rc;
-  return CTR_OK;
+  if ((rc = up.upload(&P.uploaded))) return rc;
+  const size_t lines = (size_t)PN * (DNU + 1);
+  if ((rc = table_alloc((void**)&P.bnd, lines * sizeof(float2))) ||
+      (rc = table_alloc((void**)&P.bnd64, lines * sizeof(double2))) ||
+      (rc = table_alloc((void**)&P.cols, (size_t)PN * DNU * sizeof(float4))) ||
+      (rc = table_alloc((void**)&P.Bz, (DNV + 1) * sizeof(float))) ||
+      (rc = table_alloc((void**)&P.dBz, DNV * sizeof(float))) ||
+      (rc = table_alloc((void**)&P.h2, DNV * sizeof(float))) ||
+      (rc = table_alloc((void**)&P.invdB, DNV * sizeof(float))) ||
+      (rc = table_alloc((void**)&P.zc, DNV * sizeof(float))) ||
+      (rc = table_alloc((void**)&P.maskf, cells * sizeof(float))) ||
+      (rc = table_alloc((void**)&P.mext, (size_t)(g->XN + g->YN) * sizeof(float2))))
+    return rc;
+  T.views = P.views; T.src64 = P.src64; T.rot64 = P.rot64; T.det64 = P.det64; T.mask = P.mask;
+  T.bnd = P.bnd; T.bnd64 = P.bnd64; T.cols = P.cols;
+  T.Bz = P.Bz; T.dBz = P.dBz; T.h2 = P.h2; T.invdB = P.invdB; T.zc = P.zc;
+  T.maskf = P.maskf; T.mext = P.mext;
+  return launch_plan_tables(T, nullptr);
 }
 
 static void free_plan(Plan* P) {
   if (!P) return;
-  (void)hipFree(P->views);
-  (void)hipFree(P->src64);
-  (void)hipFree(P->rot64);
-  (void)hipFree(P->sz64);
+  (void)hipFree(P->uploaded);
   (void)hipFree(P->zl_cpre);
-  (void)hipFree(P->det64);
   (void)hipFree(P->zc);
   (void)hipFree(P->bnd);
   (void)hipFree(P->bnd64);
@@ -346,7 +319,6 @@ static void free_plan(Plan* P) {
   (void)hipFree(P->dBz);
   (void)hipFree(P->h2);
   (void)hipFree(P->invdB);
-  (void)hipFree(P->mask);
   (void)hipFree(P->mext);
   (void)hipFree(P->maskf);
   (void)hipFree(P->scratch_prj);
@@ -628,7 +600,10 @@ const char* ctr_last_error(void) { return last_error_cstr(); }
 const char* ctr_version(void) { return "ctrecon_amd 0.1 (gfx950)"; }
 
 // A plan on `device` with tables built at offset `half` (build_tables) and its stream.
-static int make_plan(const ctr_geometry* geom, int device, double half, ctr_plan** out) {
+// one_call: the plan serves null-stream work of one entry point only, which the tables' kernel
+// precedes by itself, and has no stream (creating and destroying one: 0.07 ms).
+static int make_plan(const ctr_geometry* geom, int device, double half, bool one_call,
+                     ctr_plan** out) {
   if (!out) return fail(CTR_ERR_ARG, "out is NULL");
   *out = nullptr;
   int rc = validate_geometry(geom);
@@ -640,10 +615,17 @@ static int make_plan(const ctr_geometry* geom, int device, double half, ctr_plan
     free_plan(P);
     return rc;
   }
-  if (hipStreamCreate(&P->stream) != hipSuccess) {
-    P->stream = nullptr;
-    free_plan(P);
-    return fail(CTR_ERR_HIP, "cannot create the plan's stream");
+  if (!one_call) {
+    if (hipStreamCreate(&P->stream) != hipSuccess) {
+      P->stream = nullptr;
+      free_plan(P);
+      return fail(CTR_ERR_HIP, "cannot create the plan's stream");
+    }
+    // the caller may use any stream from here on
+    if (hipStreamSynchronize(nullptr) != hipSuccess) {
+      free_plan(P);
+      return fail(CTR_ERR_HIP, "cannot build the plan's tables");
+    }
   }
   *out = new ctr_plan{P};
   set_error("");
@@ -651,7 +633,7 @@ static int make_plan(const ctr_geometry* geom, int device, double half, ctr_plan
 }
 
 int ctr_plan_create(const ctr_geometry* geom, int device, ctr_plan** out) {
-  return make_plan(geom, device, 0.0, out);
+  return make_plan(geom, device, 0.0, false, out);
 }
 
 int ctr_plan_destroy(ctr_plan* plan) {
@@ -1163,7 +1145,7 @@ int ctr_dd3_proj(float x0, float y0, float z0, int DNU, int DNV, const float* xd
   PlanGuard pg;
   int rc;
   // prjMode 2: the branchless footprint model, sampled half a cell off (build_tables)
-  if ((rc = make_plan(&g, gpunum, m == Model::Fp64Sat ? 0.5 : 0.0, &pg.p))) return rc;
+  if ((rc = make_plan(&g, gpunum, m == Model::Fp64Sat ? 0.5 : 0.0, true, &pg.p))) return rc;
   if (m == Model::PseudoDD && (rc = ctr_plan_set_method(pg.p, CTR_METHOD_PSEUDO_DD))) return rc;
   const size_t NV = (size_t)XN * YN * ZN, NS = (size_t)DNU * DNV * PN;
   DBuf dv, dp;
@@ -1190,7 +1172,7 @@ int ctr_dd3_back(float x0, float y0, float z0, int DNU, int DNV, const float* xd
                                  imgZCenter, hangs, hzPos, PN, XN, YN, ZN, dx, dz, mask);
   PlanGuard pg;
   int rc;
-  if ((rc = ctr_plan_create(&g, gpunum, &pg.p))) return rc;
+  if ((rc = make_plan(&g, gpunum, 0.0, true, &pg.p))) return rc;
   if (m == Model::PseudoDD && (rc = ctr_plan_set_method(pg.p, CTR_METHOD_PSEUDO_DD))) return rc;
   if (m == Model::ZLine && (rc = ctr_plan_set_method(pg.p, CTR_METHOD_ZLINE))) return rc;
   const size_t NV = (size_t)XN * YN * ZN, NS = (size_t)DNU * DNV * PN;
