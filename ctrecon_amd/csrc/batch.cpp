@@ -71,13 +71,14 @@ struct ctr_batch {
   Mem fpItems, redItems;
   std::vector<int> fpTotal;
   // back-projection work lists by class: c = 1..4 z groups per lane, c = 0 the windowed
-  // form (one wave per column over all z); the scans of the class, and per subset step
-  // their items (and timing copies with a zero column sum)
-  std::vector<int> clsScans[5];
-  Mem bpItems[5], tuneBpItems[5];
-  std::vector<int> bpTotal[5];
-  int winZ = 0;    // tallest column of the windowed class
-  int winRC = 0;   // row chunks of the windowed class (bp_row_chunks)
+  // form (one wave per column over all z), c = 5 the windowed form of packed views; the scans
+  // of the class, and per subset step their items (and timing copies with a zero column sum)
+  static constexpr int kClasses = 6, kPackedClass = 5;
+  std::vector<int> clsScans[kClasses];
+  Mem bpItems[kClasses], tuneBpItems[kClasses];
+  std::vector<int> bpTotal[kClasses];
+  int winZ = 0, packSums = 0;  // most column sums of a wave of classes 0 and 5 (BpShape)
+  int winRC = 0;               // row chunks of the windowed class (bp_row_chunks)
   bool colw = false;
   // zg: z groups per lane (1..4; 0 and kZgWindow: each scan's own ceil(ZN / 64)) of the scans
   // with columns taller than kWinMaxZ; every other scan runs the windowed form
@@ -100,9 +101,10 @@ namespace {
 
 constexpr int kZgWindow = 5;
 
-// back-projection class of a scan (0: windowed)
+// back-projection class of a scan
 int scan_zg(const ctr_batch& B, const Plan& P) {
-  if (P.d.ZN <= kWinMaxZ) return 0;  // the windowed form, whatever zg
+  if (P.d.ZN <= kWinMaxZ)  // a windowed form, whatever zg
+    return bp_shape(P, false).rc == kPacked ? ctr_batch::kPackedClass : 0;
   return (B.zg > 0 && B.zg < kZgWindow) ? B.zg : std::min(4, (P.d.ZN + 63) / 64);
 }
 
@@ -113,21 +115,23 @@ int build_tables(ctr_batch& B) {
   std::vector<FpBatchItem<T>> fp((size_t)S * n);
   std::vector<ReduceItem> red((size_t)S * n);
   B.fpTotal.assign(S, 0);
-  for (int c = 0; c <= 4; ++c) {
+  for (int c = 0; c < B.kClasses; ++c) {
     B.clsScans[c].clear();
     B.bpTotal[c].assign(S, 0);
   }
-  B.winZ = 0;
+  B.winZ = B.packSums = 0;
   bool staged = true;
   B.winRC = 0;
   for (int i = 0; i < n; ++i) {
     const int c = scan_zg(B, *B.scans[i]->P);
     B.clsScans[c].push_back(i);
+    const BpShape sh = bp_shape(*B.scans[i]->P, false);
     if (c == 0) {
-      B.winZ = std::max(B.winZ, B.scans[i]->P->d.ZN);
-      const int rc = bp_row_chunks(B.scans[i]->P->d.DNU, B.scans[i]->P->d.DNV);
-      staged = staged && rc > 0;
-      B.winRC = std::max(B.winRC, rc);
+      B.winZ = std::max(B.winZ, sh.sums);
+      staged = staged && sh.rc > 0;
+      B.winRC = std::max(B.winRC, sh.rc);
+    } else if (c == B.kPackedClass) {
+      B.packSums = std::max(B.packSums, sh.sums);
     }
   }
   if (!staged) B.winRC = 0;
@@ -160,7 +164,7 @@ int build_tables(ctr_batch& B) {
     B.fpTotal[s] = fb;
   }
   int rc;
-  for (int cz = 0; cz <= 4; ++cz) {
+  for (int cz = 0; cz < B.kClasses; ++cz) {
     const std::vector<int>& L = B.clsScans[cz];
     if (L.empty()) continue;
     const size_t m = L.size();
@@ -176,7 +180,8 @@ int build_tables(ctr_batch& B) {
                          B.bf ? c.xs.h() : nullptr);
         b.begin = bb;
         b.colBlocks = (P.d.XN * P.d.YN + 3) / 4;
-        const int zblocks = cz == 0 ? 1 : (P.d.ZN + 64 * cz - 1) / (64 * cz);
+        const int zblocks =
+            cz == 0 || cz == B.kPackedClass ? 1 : (P.d.ZN + 64 * cz - 1) / (64 * cz);
         bb += vc > 0 ? b.colBlocks * zblocks : 0;
         BpBatchItem<T>& t = tbp[(size_t)s * m + j];
         t = b;
@@ -201,15 +206,18 @@ int step_fp(ctr_batch& B, int s) {
 
 template <typename T>
 int step_bp(ctr_batch& B, int s, bool tuning) {
-  for (int cz = 0; cz <= 4; ++cz) {
+  for (int cz = 0; cz < B.kClasses; ++cz) {
     const size_t m = B.clsScans[cz].size();
     if (!m) continue;
     const Mem& mem = tuning ? B.tuneBpItems[cz] : B.bpItems[cz];
     const BpBatchItem<T>* items = (const BpBatchItem<T>*)mem.p + (size_t)s * m;
-    int rc = cz == 0 ? launch_bp_batch_win<T>(items, (int)m, B.bpTotal[0][s], B.winZ,
-                                              B.winRC, B.bpGrid, B.bpStrided, B.st)
-                     : launch_bp_batch<T>(items, (int)m, B.bpTotal[cz][s], cz, B.bpGrid,
-                                          B.bpStrided, B.st);
+    const bool packed = cz == B.kPackedClass;
+    int rc = cz == 0 || packed
+                 ? launch_bp_batch_win<T>(items, (int)m, B.bpTotal[cz][s],
+                                          packed ? B.packSums : B.winZ, packed ? kPacked : B.winRC,
+                                          B.bpGrid, B.bpStrided, B.st)
+                 : launch_bp_batch<T>(items, (int)m, B.bpTotal[cz][s], cz, B.bpGrid, B.bpStrided,
+                                      B.st);
     if (rc) return rc;
   }
   return CTR_OK;
@@ -539,7 +547,7 @@ int ctr_batch_get_info(const ctr_batch* B, ctr_batch_info* info) {
   long long f = 0, b = 0;
   for (int s = 0; s < B->osNum; ++s) {
     f += B->fpTotal[s];
-    for (int cz = 0; cz <= 4; ++cz)
+    for (int cz = 0; cz < B->kClasses; ++cz)
       if (!B->bpTotal[cz].empty()) b += B->bpTotal[cz][s];
   }
   info->fp_items = f;

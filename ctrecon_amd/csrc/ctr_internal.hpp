@@ -113,6 +113,7 @@ struct BpArgs {
   int vb, vs, vc;
   const float* invCol;
   uint16_t* shadow;
+  int lanes;  // of a packed wave's groups (bp_pack_lanes)
 };
 
 // Batched launches: one work list over several scans.  Work items [begin, begin + n)
@@ -283,12 +284,20 @@ int launch_fp_batch(const FpBatchItem<T>* items, int nscan, int total, bool colw
 template <typename T>
 int launch_bp_batch(const BpBatchItem<T>* items, int nscan, int total, int zg, int grid,
                     int strided, hipStream_t st);
-// windowed form: one work item per block of 4 columns over all z; zmax = tallest column,
-// rc = the row chunks of its staged waves (bp_row_chunks; 0 when a scan needs the unstaged
-// form)
+// windowed form: one work item per block of 4 columns over all z; sums = floats of a wave's
+// column sums, the most of any scan, rc = the row chunks of its staged waves (bp_row_chunks; 0
+// when a scan needs the unstaged form; kPacked for a list of packed scans)
 int bp_row_chunks(int DNU, int DNV);
+int bp_pack_lanes(const Plan& P, bool matched);
+constexpr int kPacked = -1, kPackSums = 1536;
+static_assert(kPackSums <= kWinMaxZ, "a packed wave's sums");
+// A windowed back projector of a plan: rc and sums as above (ZN <= kWinMaxZ).
+struct BpShape {
+  int rc, sums;
+};
+BpShape bp_shape(const Plan& P, bool matched);
 template <typename T>
-int launch_bp_batch_win(const BpBatchItem<T>* items, int nscan, int total, int zmax, int rc,
+int launch_bp_batch_win(const BpBatchItem<T>* items, int nscan, int total, int sums, int rc,
                         int grid, int strided, hipStream_t st);
 int launch_reduce_batch(const ReduceItem* items, int nscan, hipStream_t st);
 int launch_to_bf16(uint16_t* dst, const float* src, size_t n, hipStream_t st);

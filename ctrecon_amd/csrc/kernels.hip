@@ -99,6 +99,11 @@ __device__ __forceinline__ int floor_i(float x) {
 
 __device__ __forceinline__ float sat(float x) { return __builtin_amdgcn_fmed3f(x, 0.f, 1.f); }
 
+// Infinities and NaNs.  Taps of zero weight may read a cell outside a footprint, and 0 * x is
+// not 0 for these.  A wave whose sums are not all finite computes them again in the general form,
+// which reads the footprint's cells only ("exact").
+__device__ __forceinline__ bool not_finite(float x) { return __builtin_amdgcn_classf(x, 0x207); }
+
 // Overlaps of [t, t + h] (cell edges at integers, h <= 2) with the cells k = floor(t),
 // k + 1, k + 2.
 struct Overlap3 {
@@ -115,6 +120,22 @@ __device__ __forceinline__ Overlap3 overlap3(float t, float h) {
   o.w0 = __builtin_elementwise_minimum(h, a);
   o.w1 = sat(h - a);
   o.w2 = NT == 3 ? sat((h - 2.f) + fr) : 0.f;
+  return o;
+}
+
+// The overlaps with five cells (h <= 4).
+struct Overlap5 {
+  float w[5];
+  int k;
+};
+__device__ __forceinline__ Overlap5 overlap5(float t, float h) {
+#pragma clang fp contract(off)
+  Overlap5 o;
+  const float a = 1.f - __builtin_amdgcn_fractf(t);
+  o.k = floor_i(t);
+  o.w[0] = __builtin_elementwise_minimum(h, a);
+#pragma unroll
+  for (int i = 1; i < 5; ++i) o.w[i] = sat((h - (float)(i - 1)) - a);
   return o;
 }
 
@@ -220,7 +241,8 @@ __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk
     const Buf<TV> V(A.vol, (uint32_t)NV);
     const CTR_GLOBAL float* maskf = gp(A.maskf);
     float acc = 0.f;
-    // one slice in the general form (any number of cells and taps), all quantities per lane
+    // one slice in the general form (any number of cells and taps; reads the footprint's cells
+    // only), all quantities per lane
     auto general = [&](int ii) {
       SliceIP o;
       if (!vok || !fp_inplane(bl, br, ct, gload(me, ii), ii, NI, o)) return;
@@ -465,6 +487,12 @@ __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk
         const int j = __builtin_ctzll(m);
         m &= m - 1;
         general(ii0 + j);
+      }
+    }
+    if constexpr (!ONES) {
+      if (__builtin_expect(__any(vok && not_finite(acc)), 0)) {
+        acc = 0.f;
+        for (int ii = 0; ii < NS; ++ii) general(ii);
       }
     }
     if (vok) {
@@ -870,6 +898,21 @@ __device__ __forceinline__ void pipelined(uint64_t m, Fetch fetch, Use use) {
   }
 }
 
+// The same over i = 0 ... n - 1 (n > 0).
+template <typename Set, typename Fetch, typename Use>
+__device__ __forceinline__ void pipelined_n(int n, Fetch fetch, Use use) {
+  Set x0, x1;
+  fetch(0, x0);
+  for (int i = 0;; i += 2) {
+    if (i + 1 < n) fetch(i + 1, x1);
+    use(i, x0);
+    if (i + 1 >= n) break;
+    if (i + 2 < n) fetch(i + 2, x0);
+    use(i + 1, x1);
+    if (i + 2 >= n) break;
+  }
+}
+
 // Windowed form of bp_ref_body: one wave per voxel column over all of its z.  On a
 // helical scan a view's cone covers a window of a few dozen voxels of a column, which
 // fixed lane -> z groups cover with one 64-lane pass per group it touches (about half the
@@ -884,13 +927,16 @@ __device__ __forceinline__ void pipelined(uint64_t m, Fetch fetch, Use use) {
 // loads its row of the view's columns (the next view's rows load meanwhile) and combines
 // them (R[v] = sum_u w_u y[u][v]) into LDS, four rows of zeros on either side, and a voxel
 // takes the three rows that its shadow [T, T + s] can overlap, without clamps.
+// Views of more than four columns, or whose shadows are taller than two rows (key 1), follow in
+// a second loop: any number of columns, five rows, or the shadow's own rows.
 // Bound by VALU issue (0.96 of the chip's rate).  512^2 x 256, 197 views of 888 x 64:
-// 3.76 ms with the views in order, four column loads and two-row clamps for each, 2.51 ms
-// (BF16 sinogram 3.85 ms, 2.51 ms); 277^2 x 165, 164 views of 611 x 80 in BF16, without
-// staged rows 1.78 ms, with two chunks of rows 0.69 ms.
-constexpr int kPadRows = 4;
+// 3.76 ms with the views in order, four column loads and two-row clamps for each, 2.46 ms
+// (BF16 sinogram 3.85 ms, 2.46 ms); 256^2 x 128 of 1.4 mm, where most views are of the second
+// kind, 1.17 ms, 1.06 ms, of 1 mm 1.09 ms, 0.89 ms; 277^2 x 165, 164 views of 611 x 80 in BF16,
+// without staged rows 1.78 ms, with two chunks of rows 0.69 ms.
+constexpr int kPadRows = 4, kPadEnd = 5;
 template <int RC>
-constexpr int kRowsLds = 64 * RC + 3 * kPadRows;  // zeros, rows, zeros, a slot for idle lanes
+constexpr int kRowsLds = 64 * RC + 12;  // zeros, rows, zeros, a slot for idle lanes
 template <int RC>
 constexpr int kStagedF = kRowsLds<RC> + 64 * 8;   // floats of a staged wave before its sums
 
@@ -899,19 +945,138 @@ constexpr int kStagedF = kRowsLds<RC> + 64 * 8;   // floats of a staged wave bef
 template <int RC>
 __device__ __forceinline__ void stage_rows(float* rows, int DNV, int lane, int (&row)[RC],
                                            int (&slot)[RC]) {
-  if (lane < kPadRows) {
-    rows[lane] = 0.f;
-    rows[kPadRows + DNV + lane] = 0.f;
-  }
+  if (lane < kPadRows) rows[lane] = 0.f;
+  if (lane < kPadEnd) rows[kPadRows + DNV + lane] = 0.f;
 #pragma unroll
   for (int c = 0; c < RC; ++c) {
     const int v = lane + 64 * c;
     row[c] = min(v, DNV - 1);
-    slot[c] = v < DNV ? v + kPadRows : 64 * RC + 2 * kPadRows;
+    slot[c] = v < DNV ? v + kPadRows : 64 * RC + kPadRows + kPadEnd;
   }
 }
 
-//
+// View kl's record: the window z0 ... z1; r = (T0, s, dZ of voxel z0, l^2); the weights w of up
+// to four columns; the offset o of the first; its class key = columns * 2 + (more than `lanes`
+// voxels), 0 when nothing is visible.  key = 1: more than four columns, or shadows of more than
+// two rows, or `exact`; then w = (width factor, first, last partial weight, number of columns).
+struct BpRecord {
+  float4 r, w;
+  int z0, z1, o, key;
+};
+template <typename T>
+__device__ __forceinline__ BpRecord bp_record(const BpArgs<T>& A, int kl, double Px, double Py,
+                                              float Pxf, float Pyf, int lanes, bool exact) {
+#pragma clang fp contract(off)
+  const Dims& d = A.d;
+  const BpConsts64& c64 = A.c64;
+  BpRecord v{};
+  v.z1 = -1;
+  const BpView q = bp_view(A, A.vb + kl * A.vs, Px, Py, Pxf, Pyf);
+  bp_window(d, q, v.z0, v.z1);
+  if (q.uvis && v.z0 <= v.z1) {
+    // row shadow of the window's first voxel and its step, dZ of that voxel
+    const double rlS = q.rl * c64.S, dz = (double)d.dz;
+    const double dZ = ((double)v.z0 - c64.ocz) * dz - (double)q.sz;
+    const float s = (float)(dz * rlS);
+    const float T0 = (float)((dZ - 0.5 * dz) * rlS + (c64.cV + 0.5));
+    const int nu = q.nu;
+    v.r = make_float4(T0, s, (float)dZ, q.l2);
+    v.w = make_float4(q.cws * q.wu0, nu > 1 ? q.cws * (nu == 2 ? q.fh : 1.f) : 0.f,
+                      nu > 2 ? q.cws * (nu == 3 ? q.fh : 1.f) : 0.f, nu > 3 ? q.cws * q.fh : 0.f);
+    v.o = q.u0 * d.DNV;
+    v.key = 2 * nu + (v.z1 - v.z0 >= lanes ? 1 : 0);
+    if (exact || nu > 4 || s > 2.f) {
+      v.key = 1;
+      v.w = make_float4(q.cws, q.wu0, q.fh, __int_as_float(nu));
+    }
+  }
+  return v;
+}
+
+// Column c's weight of a record of key 1.
+__device__ __forceinline__ float rest_weight(const float4& w, int c, int n) {
+#pragma clang fp contract(off)
+  return w.x * (c == 0 ? w.y : c == n - 1 ? w.z : 1.f);
+}
+
+// Shadows of five taps: under four rows by more than the window's margin, so that the first tap
+// lies on the row set's zeros (the last does for any).
+constexpr float kTaps5 = 3.9f;
+
+// Sum of the rows R[0 ... DNV) that [t, t + s] overlaps, for shadows of any height.
+__device__ __forceinline__ float tall_rows(const float* R, float t, float s, float DNVf) {
+#pragma clang fp contract(off)
+  const float lo = fmaxf(t, 0.f), hi = fminf(t + s, DNVf);
+  if (!(lo < hi)) return 0.f;
+  const int v0 = (int)lo, v1 = (int)ceilf(hi) - 1;
+  const float first = R[v0], last = R[v1];
+  float mid = 0.f;
+  // the rows between, four reads at a time (past the end: the last row, not added)
+  for (int v = v0 + 1; v < v1; v += 4) {
+    float a[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a[i] = R[min(v + i, v1)];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) mid += v + i < v1 ? a[i] : 0.f;
+  }
+  const float sum = fmaf(fminf(hi, (float)(v0 + 1)) - lo, first, mid);
+  return v1 > v0 ? fmaf(hi - (float)v1, last, sum) : sum;
+}
+
+// A voxel's share of a view: its shadow's overlaps with the rows (R0: the row set's first row)
+// times cosVal, in TAPS rows (3: shadows of up to two rows, 5: of up to kTaps5) or, 0, only the
+// rows that it overlaps.
+template <int TAPS>
+__device__ __forceinline__ float bp_voxel(const Dims& d, const float4& r, float zi,
+                                          const float* R0, float acc) {
+#pragma clang fp contract(off)
+  const float t = fmaf(zi, r.y, r.x);
+  float sum;
+  if constexpr (TAPS == 0) {
+    sum = tall_rows(R0, t, r.y, (float)d.DNV);
+  } else if constexpr (TAPS == 5) {
+    const Overlap5 o = overlap5(t, r.y);
+    const float* R = R0 + o.k;
+    sum = o.w[0] * R[0];
+#pragma unroll
+    for (int i = 1; i < 5; ++i) sum = fmaf(o.w[i], R[i], sum);
+  } else {
+    const Overlap3 o = overlap3<3>(t, r.y);
+    const float* R = R0 + o.k;
+    sum = o.w0 * R[0];
+    sum = fmaf(o.w1, R[1], sum);
+    sum = fmaf(o.w2, R[2], sum);
+  }
+  const float dZ = fmaf(zi, d.dz, r.z);
+  return fmaf(__builtin_amdgcn_sqrtf(fmaf(dZ, dZ, r.w)), sum, acc);
+}
+
+// f(columns, more than one pass) for every class of up to four columns.
+template <typename F>
+__device__ __forceinline__ void for_classes(F f) {
+  using std::integral_constant;
+  using N = std::false_type;
+  using Y = std::true_type;
+  f(integral_constant<int, 1>{}, N{});
+  f(integral_constant<int, 1>{}, Y{});
+  f(integral_constant<int, 2>{}, N{});
+  f(integral_constant<int, 2>{}, Y{});
+  f(integral_constant<int, 3>{}, N{});
+  f(integral_constant<int, 3>{}, Y{});
+  f(integral_constant<int, 4>{}, N{});
+  f(integral_constant<int, 4>{}, Y{});
+}
+
+// Whether any of a wave's n sums is not finite; they are zeroed then.
+__device__ __forceinline__ bool reset_not_finite(float* lacc, int n) {
+  const int lane = threadIdx.x & 63;
+  bool bad = false;
+  for (int i = lane; i < n; i += 64) bad = bad || not_finite(lacc[i]);
+  if (!__any(bad)) return false;
+  for (int i = lane; i < n; i += 64) lacc[i] = 0.f;
+  return true;
+}
+
 // ONES: the back projection of a sinogram of ones (the column sums of OS-SART), read from no
 // sinogram, with the weights of the back projection itself: a voxel that a shadow grazes by a
 // rounding error then has a column sum that matches its update.
@@ -942,31 +1107,20 @@ __device__ __forceinline__ void bp_staged_body(const BpArgs<T>& A, int col, floa
   const float Pxf = (float)Px, Pyf = (float)Py;
   const int frame = d.DNU * DNV;
   const float lanef = (float)lane;
+  bool rest = false;
   for (int k0 = 0; k0 < A.vc; k0 += 64) {
     const int kl = k0 + lane;
-    int z0 = 0, z1 = -1, q_o = 0, key = 0;
-    if (kl < A.vc) {
-      const BpView q = bp_view(A, A.vb + kl * A.vs, Px, Py, Pxf, Pyf);
-      bp_window(d, q, z0, z1);
-      if (q.uvis && z0 <= z1) {
-        // row shadow of the window's first voxel and its step, dZ of that voxel
-        const double rlS = q.rl * c64.S, dz = (double)d.dz;
-        const double dZ = ((double)z0 - c64.ocz) * dz - (double)q.sz;
-        const float s = (float)(dz * rlS);
-        const float T0 = (float)((dZ - 0.5 * dz) * rlS + (c64.cV + 0.5));
-        const int nu = q.nu;
-        rec[2 * lane] = make_float4(T0, s, (float)dZ, q.l2);
-        rec[2 * lane + 1] = make_float4(
-            q.cws * q.wu0, nu > 1 ? q.cws * (nu == 2 ? q.fh : 1.f) : 0.f,
-            nu > 2 ? q.cws * (nu == 3 ? q.fh : 1.f) : 0.f, nu > 3 ? q.cws * q.fh : 0.f);
-        q_o = lane * frame + q.u0 * DNV;
-        // the class: columns * 2 + (more than one pass); 1 the general form
-        key = nu > 4 || s > 2.f ? 1 : 2 * nu + (z1 - z0 >= 64 ? 1 : 0);
-      }
-    }
+    BpRecord v{};
+    if (kl < A.vc) v = bp_record(A, kl, Px, Py, Pxf, Pyf, 64, false);
+    const int z0 = v.z0, z1 = v.z1, q_o = lane * frame + v.o, key = v.key;
     if (!__any(key)) continue;
+    rest = rest || __any(key == 1);
+    if (key) {
+      rec[2 * lane] = v.r;
+      rec[2 * lane + 1] = v.w;
+    }
     const Buf<T> P(A.prj + (size_t)k0 * frame, (uint32_t)min(64, A.vc - k0) * (uint32_t)frame);
-    auto run = [&](auto NU_, auto MULTI_) {
+    for_classes([&](auto NU_, auto MULTI_) {
       constexpr int NU = decltype(NU_)::value;
       constexpr bool MULTI = decltype(MULTI_)::value;
       const uint64_t m = __ballot(key == 2 * NU + (MULTI ? 1 : 0));
@@ -998,15 +1152,8 @@ __device__ __forceinline__ void bp_staged_body(const BpArgs<T>& A, int col, floa
             const int zf = __builtin_amdgcn_readlane(z0, j);
             const int n = __builtin_amdgcn_readlane(z1, j) - zf;
             auto pass = [&](float zi, int zz) {
-              const Overlap3 o = overlap3<3>(fmaf(zi, r.y, r.x), r.y);
-              const float* R = rows + kPadRows + o.k;
-              float sum = o.w0 * R[0];
-              sum = fmaf(o.w1, R[1], sum);
-              sum = fmaf(o.w2, R[2], sum);
-              const float dZ = fmaf(zi, d.dz, r.z);
-              const float cosv = __builtin_amdgcn_sqrtf(fmaf(dZ, dZ, r.w));
               float* a = lacc + zf + zz + lane;
-              *a = fmaf(cosv, sum, *a);
+              *a = bp_voxel<3>(d, r, zi, rows + kPadRows, *a);
             };
             if constexpr (MULTI) {
               float zi = lanef;
@@ -1016,52 +1163,278 @@ __device__ __forceinline__ void bp_staged_body(const BpArgs<T>& A, int col, floa
               if (lane <= n) pass(lanef, 0);
             }
           });
-    };
-    using std::integral_constant;
-    using F = std::false_type;
-    using M = std::true_type;
-    run(integral_constant<int, 1>{}, F{});
-    run(integral_constant<int, 1>{}, M{});
-    run(integral_constant<int, 2>{}, F{});
-    run(integral_constant<int, 2>{}, M{});
-    run(integral_constant<int, 3>{}, F{});
-    run(integral_constant<int, 3>{}, M{});
-    run(integral_constant<int, 4>{}, F{});
-    run(integral_constant<int, 4>{}, M{});
-    // the general form: any number of columns and rows
-    uint64_t m = __ballot(key == 1);
-    BpView q{};
-    if (m && kl < A.vc) q = bp_view(A, A.vb + kl * A.vs, Px, Py, Pxf, Pyf);
-    while (m) {
-      const int j = __builtin_ctzll(m);
-      m &= m - 1;
-      const int o = __builtin_amdgcn_readlane(q_o, j), nu = __builtin_amdgcn_readlane(q.nu, j);
-      const float wu0 = rdl(q.wu0, j), fh = rdl(q.fh, j), cws = rdl(q.cws, j);
-#pragma unroll
-      for (int c = 0; c < RC; ++c) {
-        float R = cws * wu0 * (ONES ? 1.f : P.at(row[c], o));
-        for (int iu = 1; iu < nu; ++iu)
-          R = fmaf(cws * (iu == nu - 1 ? fh : 1.f), ONES ? 1.f : P.at(row[c], o + iu * DNV), R);
-        rows[slot[c]] = R;
-      }
-      const float4 r = rec[2 * j];
-      const int zf = __builtin_amdgcn_readlane(z0, j), zl = __builtin_amdgcn_readlane(z1, j);
-      for (int z = zf + lane; z <= zl; z += 64) {
-        const float zi = (float)(z - zf);
-        const float t = fmaf(zi, r.y, r.x);
-        const float tl = fmaxf(t, 0.f), th = fminf(t + r.y, (float)DNV);
-        if (!(tl < th)) continue;
-        const int v0 = (int)floorf(tl);
-        const int v1 = min((int)ceilf(th), DNV) - 1;
-        float sum = 0.f;
-        for (int v = v0; v <= v1; ++v)
-          sum = fmaf(fminf(th, (float)(v + 1)) - fmaxf(tl, (float)v), rows[kPadRows + v], sum);
-        const float dZ = fmaf(zi, d.dz, r.z);
-        lacc[z] = fmaf(__builtin_amdgcn_sqrtf(fmaf(dZ, dZ, r.w)), sum, lacc[z]);
-      }
-    }
+    });
   }
+  // the views of key 1; all of them where a sum is not finite
+  bool exact = false;
+  if constexpr (!ONES) exact = reset_not_finite(lacc, d.ZN);
+  if (rest || exact)
+    for (int k0 = 0; k0 < A.vc; k0 += 64) {
+      const int kl = k0 + lane;
+      BpRecord v{};
+      if (kl < A.vc) v = bp_record(A, kl, Px, Py, Pxf, Pyf, 64, exact);
+      const uint64_t m = __ballot(v.key == 1);
+      if (!m) continue;
+      rec[2 * lane] = v.r;
+      rec[2 * lane + 1] = v.w;
+      const int q_o = lane * frame + v.o;
+      const Buf<T> P(A.prj + (size_t)k0 * frame, (uint32_t)min(64, A.vc - k0) * (uint32_t)frame);
+      struct Set {
+        uint32_t y[4][RC];
+      };
+      auto load = [&](int o, int c0, int n, Set& f) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int c = 0; c < RC; ++c)
+            f.y[i][c] = ONES ? 0u : P.at_bits(row[c], o + min(c0 + i, n - 1) * DNV);
+      };
+      pipelined<Set>(
+          m,
+          [&](int j, Set& f) {
+            load(__builtin_amdgcn_readlane(q_o, j), 0, __float_as_int(rdl(v.w.w, j)), f);
+          },
+          [&](int j, const Set& f0) {
+            const float4 r = rec[2 * j], w = rec[2 * j + 1];
+            const int o = __builtin_amdgcn_readlane(q_o, j);
+            const int n = __float_as_int(rdl(v.w.w, j));
+            float R[RC] = {};
+            Set f = f0;
+            for (int c0 = 0;;) {
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                if (c0 + i < n) {
+                  const float wc = rest_weight(w, c0 + i, n);
+#pragma unroll
+                  for (int c = 0; c < RC; ++c)
+                    R[c] = fmaf(wc, ONES ? 1.f : Buf<T>::widen(f.y[i][c]), R[c]);
+                }
+              if ((c0 += 4) >= n) break;
+              load(o, c0, n, f);
+            }
+#pragma unroll
+            for (int c = 0; c < RC; ++c) rows[slot[c]] = R[c];
+            bool own = exact || rdl(v.r.y, j) > kTaps5;  // read the shadow's own rows only
+#pragma unroll
+            for (int c = 0; c < RC; ++c) own = own || not_finite(R[c]);
+            const int zf = __builtin_amdgcn_readlane(v.z0, j);
+            const int zn = __builtin_amdgcn_readlane(v.z1, j) - zf;
+            const float* R0 = rows + kPadRows;
+            float* a = lacc + zf;
+            if (__any(own)) {
+              for (int zz = lane; zz <= zn; zz += 64)
+                a[zz] = bp_voxel<0>(d, r, (float)zz, R0, a[zz]);
+            } else {
+              for (int zz = lane; zz <= zn; zz += 64)
+                a[zz] = bp_voxel<5>(d, r, (float)zz, R0, a[zz]);
+            }
+          });
+    }
   for (int z = lane; z < d.ZN; z += 64) bp_store<UPDATE>(A, vcol, col, z, lacc[z]);
+}
+
+// Staged rows with several views at a time, for detectors of few rows (bp_pack_lanes): the wave
+// is split into G = 64 / L groups of L lanes, as many as a view's rows and its window of a
+// column take, and each group takes its own view of a class, with its own rows and column sums
+// in LDS (added up at the end, groups in order).  The records are sorted by class, so that a
+// group reads its view's next to its neighbour's.  Otherwise as bp_staged_body.
+// 197 views of 888 columns, one view at a time and packed: 64^3, 16 rows 71 us, 30 us (3 groups);
+// 256^2 x 128, 16 rows 573 us, 327 us, 8 rows 567 us, 236 us (6 groups).
+constexpr int kPackRowsLds = 64 + 8 * (kPadRows + kPadEnd + 1);  // up to 8 groups of rows
+constexpr int kPackF = kPackRowsLds + 64 * 12;  // floats of a wave before its sums
+struct Groups {
+  int L, G, inv, grp, gl, row, slot, rows, sums;
+  // rows, sums: offsets of the group's rows and column sums (ZN4 floats each)
+  __device__ __forceinline__ Groups(int L_, int DNV, int ZN4)
+      : L(L_), G(64 / L_), inv((65536 + G - 1) / G) {
+    const int lane = threadIdx.x & 63;
+    grp = min(lane / L, G - 1);
+    gl = lane - grp * L;  // (lanes past the last group: >= L, never active)
+    row = min(gl, DNV - 1);
+    rows = grp * (L + kPadRows + kPadEnd + 1);
+    slot = gl < DNV ? gl + kPadRows : L + kPadRows + kPadEnd;
+    sums = grp * ZN4;
+  }
+  // ceil(n / G), n <= 64
+  __device__ __forceinline__ int rounds(int n) const { return ((n + G - 1) * inv) >> 16; }
+  __device__ __forceinline__ void zero_pads(float* set, int DNV) const {
+    if (gl < kPadRows) set[rows + gl] = 0.f;
+    if (gl < kPadEnd) set[rows + kPadRows + DNV + gl] = 0.f;
+  }
+};
+// Sorts the lanes by class: returns this lane's position, first[k] that of class k's first lane
+// (k = 1 ... 9, first[10] the total).  Lanes of key 0 have none.
+__device__ __forceinline__ int sort_classes(int key, int (&first)[11]) {
+  int pos = 0, base = 0;
+#pragma unroll
+  for (int k = 1; k <= 9; ++k) {
+    const uint64_t m = __ballot(key == k);
+    first[k] = base;
+    if (key == k)
+      pos = base + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                  __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+    base += __builtin_popcountll(m);
+  }
+  first[10] = base;
+  return pos;
+}
+
+template <bool UPDATE, typename T, bool ONES = false>
+__device__ __forceinline__ void bp_packed_body(const BpArgs<T>& A, int col, float* lds) {
+#pragma clang fp contract(off)
+  const Dims& d = A.d;
+  const BpConsts64& c64 = A.c64;
+  const int lane = threadIdx.x & 63;
+  if (col >= d.XN * d.YN) return;
+  const int y = col / d.XN, x = col - y * d.XN;
+  CTR_GLOBAL float* vcol = gp(A.vol) + (size_t)col * d.ZN;
+  if (gp(A.mask)[col] != 1) {
+    if constexpr (!UPDATE) {
+      for (int z = lane; z < d.ZN; z += 64) vcol[z] = 0.f;
+    }
+    return;
+  }
+  const int DNV = d.DNV, ZN4 = (d.ZN + 3) & ~3;
+  const Groups g(A.lanes, DNV, ZN4);
+  float4* rec = reinterpret_cast<float4*>(lds + kPackRowsLds);  // [64][3]
+  float* lacc = lds + kPackF;
+  for (int i = lane; i < g.G * ZN4; i += 64) lacc[i] = 0.f;
+  g.zero_pads(lds, DNV);
+  float* rows = lds + g.rows;
+  float* gacc = lacc + g.sums;
+  const double Px = ((double)x - c64.ocx) * c64.dx;
+  const double Py = ((double)y - c64.ocy) * c64.dx;
+  const float Pxf = (float)Px, Pyf = (float)Py;
+  const int frame = d.DNU * DNV;
+  const float glf = (float)g.gl;
+  bool rest = false;
+  // a view's (offset of its first column, z0, z1 - z0)
+  auto ints = [&](const BpRecord& v) {
+    return make_float4(__int_as_float(lane * frame + v.o), __int_as_float(v.z0),
+                       __int_as_float(v.z1 - v.z0), 0.f);
+  };
+  for (int k0 = 0; k0 < A.vc; k0 += 64) {
+    const int kl = k0 + lane;
+    BpRecord v{};
+    if (kl < A.vc) v = bp_record(A, kl, Px, Py, Pxf, Pyf, g.L, false);
+    if (!__any(v.key)) continue;
+    rest = rest || __any(v.key == 1);
+    int first[11];
+    const int pos = sort_classes(v.key, first);
+    if (v.key) {
+      rec[3 * pos] = v.r;
+      rec[3 * pos + 1] = v.w;
+      rec[3 * pos + 2] = ints(v);
+    }
+    const Buf<T> P(A.prj + (size_t)k0 * frame, (uint32_t)min(64, A.vc - k0) * (uint32_t)frame);
+    for_classes([&](auto NU_, auto MULTI_) {
+      constexpr int NU = decltype(NU_)::value;
+      constexpr bool MULTI = decltype(MULTI_)::value;
+      constexpr int K = 2 * NU + (MULTI ? 1 : 0);
+      const int n = first[K + 1] - first[K];
+      if (!n) return;
+      const float4* rc = rec + 3 * first[K];
+      struct Set {
+        uint32_t y[NU];
+      };
+      pipelined_n<Set>(
+          g.rounds(n),
+          [&](int i, Set& f) {
+            if constexpr (ONES) return;
+            const int e = min(i * g.G + g.grp, n - 1);
+            const int o = __float_as_int(rc[3 * e + 2].x) + g.row;
+#pragma unroll
+            for (int iu = 0; iu < NU; ++iu) f.y[iu] = P.at_bits(o, iu * DNV);
+          },
+          [&](int i, const Set& f) {
+            const int e = i * g.G + g.grp;
+            const float4* re = rc + 3 * min(e, n - 1);
+            const float4 r = re[0], w = re[1], oz = re[2];
+            const float wu[4] = {w.x, w.y, w.z, w.w};
+            float R = wu[0] * (ONES ? 1.f : Buf<T>::widen(f.y[0]));
+#pragma unroll
+            for (int iu = 1; iu < NU; ++iu)
+              R = fmaf(wu[iu], ONES ? 1.f : Buf<T>::widen(f.y[iu]), R);
+            rows[g.slot] = R;
+            const int last = e < n && g.gl < g.L ? __float_as_int(oz.z) : -1;
+            float* a = gacc + __float_as_int(oz.y) + g.gl;
+            if constexpr (MULTI) {
+              float zi = glf;
+              for (int zz = 0; __any(zz <= last); zz += g.L, zi += (float)g.L)
+                if (g.gl <= last - zz) a[zz] = bp_voxel<3>(d, r, zi, rows + kPadRows, a[zz]);
+            } else {
+              if (g.gl <= last) *a = bp_voxel<3>(d, r, glf, rows + kPadRows, *a);
+            }
+          });
+    });
+  }
+  // the views of key 1; all of them where a sum is not finite
+  bool exact = false;
+  if constexpr (!ONES) exact = reset_not_finite(lacc, g.G * ZN4);
+  if (rest || exact)
+    for (int k0 = 0; k0 < A.vc; k0 += 64) {
+      const int kl = k0 + lane;
+      BpRecord v{};
+      if (kl < A.vc) v = bp_record(A, kl, Px, Py, Pxf, Pyf, g.L, exact);
+      int first[11];
+      const int pos = sort_classes(v.key, first), n = first[2];
+      if (!n) continue;
+      if (v.key == 1) {
+        rec[3 * pos] = v.r;
+        rec[3 * pos + 1] = v.w;
+        rec[3 * pos + 2] = ints(v);
+      }
+      const Buf<T> P(A.prj + (size_t)k0 * frame, (uint32_t)min(64, A.vc - k0) * (uint32_t)frame);
+      struct Set {
+        uint32_t y[4];
+      };
+      auto load = [&](int o, int c0, int nc, Set& f) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          f.y[i] = ONES ? 0u : P.at_bits(o + min(c0 + i, nc - 1) * DNV, 0);
+      };
+      pipelined_n<Set>(
+          g.rounds(n),
+          [&](int i, Set& f) {
+            const float4* re = rec + 3 * min(i * g.G + g.grp, n - 1);
+            load(__float_as_int(re[2].x) + g.row, 0, __float_as_int(re[1].w), f);
+          },
+          [&](int i, const Set& f0) {
+            const int e = i * g.G + g.grp;
+            const float4* re = rec + 3 * min(e, n - 1);
+            const float4 r = re[0], w = re[1], oz = re[2];
+            const int nc = __float_as_int(w.w);
+            float R = 0.f;
+            Set f = f0;
+            for (int c0 = 0;;) {
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                const float t = fmaf(rest_weight(w, c0 + i, nc),
+                                     ONES ? 1.f : Buf<T>::widen(f.y[i]), R);
+                R = c0 + i < nc ? t : R;
+              }
+              c0 += 4;
+              if (!__any(c0 < nc)) break;
+              load(__float_as_int(oz.x) + g.row, c0, nc, f);
+            }
+            rows[g.slot] = R;
+            const int last = e < n && g.gl < g.L ? __float_as_int(oz.z) : -1;
+            float* a = gacc + __float_as_int(oz.y);
+            const float* R0 = rows + kPadRows;
+            if (exact || __any(r.y > kTaps5 || not_finite(R))) {
+              for (int zz = g.gl; zz <= last; zz += g.L)
+                a[zz] = bp_voxel<0>(d, r, (float)zz, R0, a[zz]);
+            } else {
+              for (int zz = g.gl; zz <= last; zz += g.L)
+                a[zz] = bp_voxel<5>(d, r, (float)zz, R0, a[zz]);
+            }
+          });
+    }
+  for (int z = lane; z < d.ZN; z += 64) {
+    float a = lacc[z];
+    for (int k = 1; k < g.G; ++k) a += lacc[k * ZN4 + z];
+    bp_store<UPDATE>(A, vcol, col, z, a);
+  }
 }
 
 // The windowed form without staged rows (more than 256 detector rows, or frames too large
@@ -1131,15 +1504,22 @@ __device__ __forceinline__ void bp_win_body(const BpArgs<T>& A, int col, float* 
   for (int z = lane; z < d.ZN; z += 64) bp_store<UPDATE>(A, vcol, col, z, lacc[z]);
 }
 
-// The windowed body with staged rows (RC = 1, 2, 4) or without (RC = 0); lds: bp_win_floats
-// of this wave.
-__host__ __device__ constexpr int bp_win_floats(int RC, int ZN) {
-  return (RC == 1 ? kStagedF<1> : RC == 2 ? kStagedF<2> : RC == 4 ? kStagedF<4> : 0) +
-         ((ZN + 3) & ~3);
+// The windowed body with staged rows (RC = 1, 2, 4), of packed views (kPacked) or without
+// either (0); lds: bp_win_floats of this wave, sums = the floats of its column sums.
+__host__ __device__ constexpr int bp_win_floats(int RC, int sums) {
+  return (RC == kPacked ? kPackF
+          : RC == 1     ? kStagedF<1>
+          : RC == 2     ? kStagedF<2>
+          : RC == 4     ? kStagedF<4>
+                        : 0) +
+         ((sums + 3) & ~3);
 }
+// Waves per SIMD that the registers of a body leave room for.
+constexpr int bp_waves(int RC) { return RC == 4 ? 5 : RC == 2 || RC == kPacked ? 6 : 7; }
 template <bool UPDATE, typename T, int RC, bool ONES = false>
 __device__ __forceinline__ void bp_any_win_body(const BpArgs<T>& A, int col, float* lds) {
-  if constexpr (RC > 0) bp_staged_body<UPDATE, T, RC, ONES>(A, col, lds);
+  if constexpr (RC == kPacked) bp_packed_body<UPDATE, T, ONES>(A, col, lds);
+  else if constexpr (RC > 0) bp_staged_body<UPDATE, T, RC, ONES>(A, col, lds);
   else bp_win_body<UPDATE, T, ONES>(A, col, lds);
 }
 
@@ -1149,38 +1529,39 @@ __global__ __launch_bounds__(kBlock) void bp_ref_kernel(BpArgs<T> A) {
   bp_ref_body<UPDATE, ZG, T>(A, col, blockIdx.y);
 }
 
-// Windowed reference back projection; dynamic LDS: kWaves * bp_win_floats(RC, ZN) floats.
+// Windowed reference back projection; dynamic LDS: kWaves * bp_win_floats(RC, sums) floats.
 template <bool UPDATE, typename T, int RC>
-__global__ __launch_bounds__(kBlock, RC == 4 ? 5 : RC == 2 ? 6 : RC == 1 ? 8 : 7) void bp_win_kernel(BpArgs<T> A) {
+__global__ __launch_bounds__(kBlock, RC == 1 ? 8 : bp_waves(RC)) void bp_win_kernel(
+    BpArgs<T> A, int sums) {
   extern __shared__ float4 lds_win[];
   float* lds = reinterpret_cast<float*>(lds_win);
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   bp_any_win_body<UPDATE, T, RC>(A, blockIdx.x * kWaves + wid,
-                                 lds + wid * bp_win_floats(RC, A.d.ZN));
+                                 lds + wid * bp_win_floats(RC, sums));
 }
 
 // Back projection of a sinogram of ones (A.prj unused); dynamic LDS as bp_win_kernel.
 template <int RC>
-__global__ __launch_bounds__(kBlock, RC == 4 ? 5 : 7) void bp_win_ones_kernel(BpArgs<float> A) {
+__global__ __launch_bounds__(kBlock, bp_waves(RC)) void bp_win_ones_kernel(BpArgs<float> A,
+                                                                          int sums) {
   extern __shared__ float4 lds_win[];
   float* lds = reinterpret_cast<float*>(lds_win);
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   bp_any_win_body<false, float, RC, true>(A, blockIdx.x * kWaves + wid,
-                                          lds + wid * bp_win_floats(RC, A.d.ZN));
+                                          lds + wid * bp_win_floats(RC, sums));
 }
 
 // Batched windowed reference back projection: flat work list of (scan, block of 4
-// columns); RC as the scan of most rows needs it, dynamic LDS: kWaves *
-// bp_win_floats(RC, zmax) floats (zmax: the tallest column of the batch).
+// columns); RC as the scan of most rows needs it (packed scans have a list of their own),
+// dynamic LDS: kWaves * bp_win_floats(RC, sums) floats (sums: the most of any scan).
 template <typename T, int RC>
-__global__ __launch_bounds__(kBlock, RC == 4 ? 5 : RC == 2 ? 6 : 7) void bp_batch_win_kernel(const BpBatchItem<T>* __restrict__ D,
-                                                              int nscan, int total, int sched,
-                                                              int zmax) {
+__global__ __launch_bounds__(kBlock, bp_waves(RC)) void bp_batch_win_kernel(
+    const BpBatchItem<T>* __restrict__ D, int nscan, int total, int sched, int sums) {
   extern __shared__ float4 lds_win[];
   int i0, step, i1;
   batch_range(D, nscan, total, sched, i0, step, i1);
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  float* lds = reinterpret_cast<float*>(lds_win) + wid * bp_win_floats(RC, zmax);
+  float* lds = reinterpret_cast<float*>(lds_win) + wid * bp_win_floats(RC, sums);
   int s = 0;
   for (int item = i0; item < i1; item += step) {
     if (sched == 1) s = 0;
@@ -1193,13 +1574,13 @@ __global__ __launch_bounds__(kBlock, RC == 4 ? 5 : RC == 2 ? 6 : 7) void bp_batc
 // bp_batch_win_kernel for the one-workgroup-per-item schedule (grid = total): no item
 // loop, so nothing stays live around the column body.
 template <typename T, int RC>
-__global__ __launch_bounds__(kBlock, RC == 4 ? 5 : RC == 2 ? 6 : 7) void bp_batch_win1_kernel(
-    const BpBatchItem<T>* __restrict__ D, int nscan, int total, int zmax) {
+__global__ __launch_bounds__(kBlock, bp_waves(RC)) void bp_batch_win1_kernel(
+    const BpBatchItem<T>* __restrict__ D, int nscan, int total, int sums) {
   extern __shared__ float4 lds_win[];
   int i0, step, i1;
   batch_range(D, nscan, total, 2, i0, step, i1);
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  float* lds = reinterpret_cast<float*>(lds_win) + wid * bp_win_floats(RC, zmax);
+  float* lds = reinterpret_cast<float*>(lds_win) + wid * bp_win_floats(RC, sums);
   int s = 0;
   while (s + 1 < nscan && D[s + 1].begin <= i0) ++s;
   const BpBatchItem<T>& B = D[s];
@@ -1726,196 +2107,368 @@ struct MatchedCols {
 // its overlap with a row, times the column's in-plane overlap over its footprint's area, is
 // the forward projector's weight: w_t = overlap dB / (tr - tl), r cancelling.  Lane l
 // evaluates view k0 + l (columns, T0 and s in FP64); the row sets hold w_t y[u + t][v].
-// Views of more than four columns, of more than three rows per voxel, or whose columns'
-// rows differ by over a row across the window take the row walk.
+// Views of more than four columns take further records for the rest.
 // Bound by VALU issue (0.73 of the chip's rate) and the texture unit's row loads.  256^2 x
 // 128, 197 views of 888 x 64: 3.94 ms with a search and a gather of the rows per voxel
-// (bp_matched_win_kernel), 0.88 ms; 512^2 x 256: 18.0 ms, 4.0 ms.
+// (bp_matched_win_kernel), 0.90 ms; 512^2 x 256: 18.0 ms, 4.1 ms; 256^2 x 128 of 1.4 mm 5.7 ms,
+// 2.2 ms.
+//
+// RC = kPacked: several views at a time, as bp_packed_body.
+// 197 views of 888 columns, one view at a time and packed: 64^3, 16 rows 104 us, 60 us; 256^2 x
+// 128, 16 rows 915 us, 584 us, 8 rows 911 us, 497 us.
 template <int RC>
 constexpr int kMatchedF = 4 * kRowsLds<RC> + 64 * 16;
-__host__ __device__ constexpr int bp_matched_floats(int RC, int ZN) {
-  return (RC == 1 ? kMatchedF<1> : RC == 2 ? kMatchedF<2> : kMatchedF<4>) + ((ZN + 3) & ~3);
+template <>
+constexpr int kMatchedF<kPacked> = 4 * kPackRowsLds + 64 * 16;
+__host__ __device__ constexpr int bp_matched_floats(int RC, int sums) {
+  return (RC == kPacked ? kMatchedF<kPacked>
+          : RC == 1     ? kMatchedF<1>
+          : RC == 2     ? kMatchedF<2>
+                        : kMatchedF<4>) +
+         ((sums + 3) & ~3);
 }
+
+// What the matched kernels read: the scaled sinogram and the plan's tables.
+struct MatchedArgs {
+  const float* yp;
+  float* vol;
+  const ViewP* views;
+  const double2* bnd;
+  const float4* cols;
+  const float* Bz;
+  const uint8_t* mask;
+  Dims d;
+  BpConsts c;
+  int vb, vs, vc, lanes;
+  const float* invCol;
+  uint16_t* shadow;
+};
+
+// View kl's record of its columns c0 ... c0 + 3: (T0, s, w) of the n columns, their window, the
+// offset of the first and the class as in BpRecord (1: shadows of more than two rows, or that
+// leave the row set's zeros at an end of the window, or `exact`).
+struct MatchedRecord {
+  float4 t[4];
+  int z0, z1, o, n, key;
+  bool more;
+};
+__device__ __forceinline__ MatchedRecord matched_record(const MatchedArgs& A, int kl, int c0,
+                                                        int x, int y, float Px, float Py,
+                                                        int lanes, bool exact) {
+  const Dims& d = A.d;
+  const int DNU = d.DNU, DNV = d.DNV, p = A.vb + kl * A.vs;
+  const float ZNf = (float)d.ZN;
+  const double idB = 1.0 / d.dB_64;
+  MatchedRecord v{};
+  v.z1 = -1;
+  const ViewP vp = A.views[p];
+  const float4* ctab = A.cols + (size_t)p * DNU;
+  const float fii = (float)(vp.xmarch ? x : y);
+  MatchedCols mc(vp, A.bnd, p, x, y, Px, Py, d, A.c.inv_sid);
+  v.o = (mc.u + c0) * DNV;
+  float rt[4] = {1.f, 1.f, 1.f, 1.f}, wt[4] = {0.f, 0.f, 0.f, 0.f};
+  float rmin = 3.4e38f, rmax = -3.4e38f;
+  int n = -c0;
+  for (; n < 4 && mc.meets(); mc.next(), ++n) {
+    if (n < 0) continue;
+    const float4 ct = ctab[mc.u];
+    const float r = fmaf(fii, ct.y, ct.x);
+    const double wy = mc.overlap();
+    const float w = wy > 0.0 ? (float)(wy / (mc.su1 - mc.su) * d.dB_64) : 0.f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      if (n == t) {
+        rt[t] = r;
+        wt[t] = w;
+      }
+    rmin = fminf(rmin, r);
+    rmax = fmaxf(rmax, r);
+  }
+  v.more = n == 4 && mc.meets();
+  if (!(n > 0 && rmin > 0.f)) return v;
+  // z cells [k - .5, k + .5] meeting [az + r Bz[0], az + r Bz[DNV]] for some column,
+  // with a margin of 1e-2 (relative to azi, as fp_kernel)
+  const float lo = fminf(fmaf(rmin, A.Bz[0], vp.azf), fmaf(rmax, A.Bz[0], vp.azf));
+  const float hi = fmaxf(fmaf(rmin, A.Bz[DNV], vp.azf), fmaf(rmax, A.Bz[DNV], vp.azf));
+  const float fazi = (float)vp.azi;
+  const float za = fminf(fmaxf(lo - 0.51f, -4.f - fazi), (ZNf + 4.f) - fazi);
+  const float zb = fminf(fmaxf(hi + 0.51f, -4.f - fazi), (ZNf + 4.f) - fazi);
+  v.z0 = max((int)floorf(za) + 1 + vp.azi, 0);
+  v.z1 = min((int)ceilf(zb) - 1 + vp.azi, d.ZN - 1);
+  if (v.z0 > v.z1) return v;
+  bool plain = !exact;
+  const double e0 = (double)(v.z0 - vp.azi) - 0.5 - (double)vp.azf;
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+    if (t < n) {
+      const double s = idB / (double)rt[t];
+      const float sf = (float)s, T0 = (float)(e0 * s - d.B0_64 * idB);
+      // taps stay on the row set and its zeros over the whole window
+      plain = plain && sf <= 2.f && T0 >= (float)-kPadRows &&
+              fmaf((float)(v.z1 - v.z0), sf, T0) < (float)(DNV + kPadRows - 2);
+      v.t[t] = make_float4(T0, sf, wt[t], 0.f);
+    }
+  v.n = n;
+  v.key = plain ? 2 * n + (v.z1 - v.z0 >= lanes ? 1 : 0) : 1;
+  return v;
+}
+
+// A voxel's share of a view of NU columns, TAPS as in bp_voxel (5 and 0: n of the NU columns):
+// r[t] its records, R0 + t * set their first rows.
+template <int NU, int TAPS>
+__device__ __forceinline__ float matched_voxel(const float4 (&r)[NU], int n, float zi,
+                                               const float* R0, int set, float DNVf) {
+  float g = 0.f;
+#pragma unroll
+  for (int t = 0; t < NU; ++t) {
+    const float T = fmaf(zi, r[t].y, r[t].x);
+    if constexpr (TAPS == 5) {
+      if (t < n) {
+        const Overlap5 o = overlap5(T, r[t].y);
+        const float* R = R0 + t * set + o.k;
+#pragma unroll
+        for (int i = 0; i < 5; ++i) g = fmaf(o.w[i], R[i], g);
+      }
+    } else if constexpr (TAPS == 0) {
+      if (t < n && r[t].z != 0.f) g += tall_rows(R0 + t * set, T, r[t].y, DNVf);
+    } else {
+      const Overlap3 o = overlap3<3>(T, r[t].y);
+      const float* R = R0 + t * set + o.k;
+      g = t == 0 ? o.w0 * R[0] : fmaf(o.w0, R[0], g);
+      g = fmaf(o.w1, R[1], g);
+      g = fmaf(o.w2, R[2], g);
+    }
+  }
+  return g;
+}
+
 template <bool UPDATE, int RC>
-__global__ __launch_bounds__(kBlock, RC == 4 ? 4 : 6) void bp_matched_staged_kernel(
-    const float* __restrict__ yp, float* __restrict__ vol, const ViewP* __restrict__ views,
-    const double2* __restrict__ bnd, const float4* __restrict__ cols,
-    const float* __restrict__ Bz, const uint8_t* __restrict__ mask, Dims d, BpConsts c,
-    int vb, int vs, int vc, const float* __restrict__ invCol, uint16_t* __restrict__ shadow) {
+__global__ __launch_bounds__(kBlock, RC == 4 ? 4 : 6) void bp_matched_staged_kernel(MatchedArgs A,
+                                                                                    int sums) {
   extern __shared__ float4 lds_win[];
+  constexpr bool PACK = RC == kPacked;
+  constexpr int SET = PACK ? kPackRowsLds : kRowsLds<PACK ? 1 : RC>;  // floats of a column's rows
+  constexpr int NC = PACK ? 1 : RC;                                    // row chunks per lane
+  const Dims& d = A.d;
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  float* rows = reinterpret_cast<float*>(lds_win) + wid * bp_matched_floats(RC, d.ZN);
-  float4* rec = reinterpret_cast<float4*>(rows + 4 * kRowsLds<RC>);  // [64][4]
+  float* rows = reinterpret_cast<float*>(lds_win) + wid * bp_matched_floats(RC, sums);
+  float4* rec = reinterpret_cast<float4*>(rows + 4 * SET);  // [64][4]
   float* lacc = rows + kMatchedF<RC>;
   const int col = blockIdx.x * kWaves + wid;
   if (col >= d.XN * d.YN) return;
   const int y = col / d.XN, x = col - y * d.XN;
-  float* vcol = vol + (size_t)col * d.ZN;
-  const float mk = (float)mask[col];
+  float* vcol = A.vol + (size_t)col * d.ZN;
+  const float mk = (float)A.mask[col];
   if (mk == 0.f) {
     if constexpr (!UPDATE) {
       for (int z = lane; z < d.ZN; z += 64) vcol[z] = 0.f;
     }
     return;
   }
-  for (int z = lane; z < d.ZN; z += 64) lacc[z] = 0.f;
-  const int DNU = d.DNU, DNV = d.DNV, frame = DNU * DNV;
-  int row[RC], slot[RC];
+  const int DNU = d.DNU, DNV = d.DNV, frame = DNU * DNV, ZN4 = (d.ZN + 3) & ~3;
+  const Groups g(PACK ? A.lanes : 64, DNV, ZN4);  // (one group when not packed)
+  for (int i = lane; i < sums; i += 64) lacc[i] = 0.f;
+  int row[NC], slot[NC];
 #pragma unroll
-  for (int t = 0; t < 4; ++t) stage_rows<RC>(rows + t * kRowsLds<RC>, DNV, lane, row, slot);
-  const float Px = ((float)x - d.ocx) * d.dx, Py = ((float)y - d.ocy) * d.dx;
-  const float lanef = (float)lane, ZNf = (float)d.ZN;
-  const double B0 = d.B0_64, idB = 1.0 / d.dB_64;
-  for (int k0 = 0; k0 < vc; k0 += 64) {
-    const int kl = k0 + lane;
-    int z0 = 0, z1 = -1, q_o = 0, key = 0;
-    if (kl < vc) {
-      const int p = vb + kl * vs;
-      const ViewP vp = views[p];
-      const float4* ctab = cols + (size_t)p * DNU;
-      const float fii = (float)(vp.xmarch ? x : y);
-      MatchedCols mc(vp, bnd, p, x, y, Px, Py, d, c.inv_sid);
-      q_o = lane * frame + mc.u * DNV;
-      float rt[4] = {1.f, 1.f, 1.f, 1.f}, wt[4] = {0.f, 0.f, 0.f, 0.f};
-      float rmin = 3.4e38f, rmax = -3.4e38f;
-      int n = 0;
-      for (; mc.meets(); mc.next()) {
-        const float4 ct = ctab[mc.u];
-        const float r = fmaf(fii, ct.y, ct.x);
-        const double wy = mc.overlap();
-        const float w = wy > 0.0 ? (float)(wy / (mc.su1 - mc.su) * d.dB_64) : 0.f;
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-          if (n == t) {
-            rt[t] = r;
-            wt[t] = w;
-          }
-        rmin = fminf(rmin, r);
-        rmax = fmaxf(rmax, r);
-        ++n;
-      }
-      if (n > 0 && rmin > 0.f) {
-        // z cells [k - .5, k + .5] meeting [az + r Bz[0], az + r Bz[DNV]] for some column,
-        // with a margin of 1e-2 (relative to azi, as fp_kernel)
-        const float lo = fminf(fmaf(rmin, Bz[0], vp.azf), fmaf(rmax, Bz[0], vp.azf));
-        const float hi = fmaxf(fmaf(rmin, Bz[DNV], vp.azf), fmaf(rmax, Bz[DNV], vp.azf));
-        const float fazi = (float)vp.azi;
-        const float za = fminf(fmaxf(lo - 0.51f, -4.f - fazi), (ZNf + 4.f) - fazi);
-        const float zb = fminf(fmaxf(hi + 0.51f, -4.f - fazi), (ZNf + 4.f) - fazi);
-        z0 = max((int)floorf(za) + 1 + vp.azi, 0);
-        z1 = min((int)ceilf(zb) - 1 + vp.azi, d.ZN - 1);
-        if (z0 <= z1) {
-          bool plain = n <= 4;
-          const double e0 = (double)(z0 - vp.azi) - 0.5 - (double)vp.azf;
-#pragma unroll
-          for (int t = 0; t < 4; ++t)
-            if (t < n) {
-              const double s = idB / (double)rt[t];
-              const float sf = (float)s, T0 = (float)(e0 * s - B0 * idB);
-              // taps stay on the row set and its zeros over the whole window
-              plain = plain && sf <= 2.f && T0 >= (float)-kPadRows &&
-                      fmaf((float)(z1 - z0), sf, T0) < (float)(DNV + kPadRows - 2);
-              rec[4 * lane + t] = make_float4(T0, sf, wt[t], 0.f);
-            }
-          // the class: columns * 2 + (more than one pass); 1 the row walk
-          key = plain ? 2 * n + (z1 - z0 >= 64 ? 1 : 0) : 1;
-        }
-      }
-    }
-    if (!__any(key)) continue;
-    const Buf<float> P(yp + (size_t)k0 * frame, (uint32_t)min(64, vc - k0) * (uint32_t)frame);
-    auto run = [&](auto NU_, auto MULTI_) {
-      constexpr int NU = decltype(NU_)::value;
-      constexpr bool MULTI = decltype(MULTI_)::value;
-      const uint64_t m = __ballot(key == 2 * NU + (MULTI ? 1 : 0));
-      if (!m) return;
-      struct Set {
-        float y[NU][RC];
-      };
-      pipelined<Set>(
-          m,
-          [&](int j, Set& f) {
-            const int o = __builtin_amdgcn_readlane(q_o, j);
-#pragma unroll
-            for (int t = 0; t < NU; ++t)
-#pragma unroll
-              for (int h = 0; h < RC; ++h) f.y[t][h] = P.at(row[h], o + t * DNV);
-          },
-          [&](int j, const Set& f) {
-            float4 r[NU];
-#pragma unroll
-            for (int t = 0; t < NU; ++t) {
-              r[t] = rec[4 * j + t];
-#pragma unroll
-              for (int h = 0; h < RC; ++h) rows[t * kRowsLds<RC> + slot[h]] = r[t].z * f.y[t][h];
-            }
-            const int zf = __builtin_amdgcn_readlane(z0, j);
-            const int n = __builtin_amdgcn_readlane(z1, j) - zf;
-            auto pass = [&](float zi, int zz) {
-              float g = 0.f;
-#pragma unroll
-              for (int t = 0; t < NU; ++t) {
-                const Overlap3 o = overlap3<3>(fmaf(zi, r[t].y, r[t].x), r[t].y);
-                const float* R = rows + t * kRowsLds<RC> + kPadRows + o.k;
-                g = t == 0 ? o.w0 * R[0] : fmaf(o.w0, R[0], g);
-                g = fmaf(o.w1, R[1], g);
-                g = fmaf(o.w2, R[2], g);
-              }
-              lacc[zf + zz + lane] += g;
-            };
-            if constexpr (MULTI) {
-              float zi = lanef;
-              for (int zz = 0; zz <= n; zz += 64, zi += 64.f)
-                if (lane <= n - zz) pass(zi, zz);
-            } else {
-              if (lane <= n) pass(lanef, 0);
-            }
-          });
-    };
-    using std::integral_constant;
-    using F = std::false_type;
-    using M = std::true_type;
-    run(integral_constant<int, 1>{}, F{});
-    run(integral_constant<int, 1>{}, M{});
-    run(integral_constant<int, 2>{}, F{});
-    run(integral_constant<int, 2>{}, M{});
-    run(integral_constant<int, 3>{}, F{});
-    run(integral_constant<int, 3>{}, M{});
-    run(integral_constant<int, 4>{}, F{});
-    run(integral_constant<int, 4>{}, M{});
-    uint64_t m = __ballot(key == 1);
-    while (m) {
-      const int j = __builtin_ctzll(m);
-      m &= m - 1;
-      const int k = k0 + j, p = vb + k * vs;
-      const ViewP vp = views[p];
-      const float4* ctab = cols + (size_t)p * DNU;
-      const float fii = (float)(vp.xmarch ? x : y);
-      const int zf = __builtin_amdgcn_readlane(z0, j), zl = __builtin_amdgcn_readlane(z1, j);
-      for (int z = zf + lane; z <= zl; z += 64) {
-        const float zlo = (float)(z - vp.azi) - 0.5f;
-        float a = lacc[z];
-        for (MatchedCols mc(vp, bnd, p, x, y, Px, Py, d, c.inv_sid); mc.meets(); mc.next()) {
-          const double wy = mc.overlap();
-          if (!(wy > 0.0)) continue;
-          const float4 ct = ctab[mc.u];
-          const float r = fmaf(fii, ct.y, ct.x);
-          const float w = (float)wy * __builtin_amdgcn_rcpf((float)(mc.su1 - mc.su) * r);
-          a = fmaf(w, matched_rows(yp + (size_t)k * frame + (size_t)mc.u * DNV, Bz, DNV, r,
-                                   vp.azf, zlo, d.B0, d.dB), a);
-        }
-        lacc[z] = a;
-      }
+  for (int t = 0; t < 4; ++t) {
+    if constexpr (PACK) {
+      g.zero_pads(rows + t * SET, DNV);
+      row[0] = g.row;
+      slot[0] = g.rows + g.slot;
+    } else {
+      stage_rows<NC>(rows + t * SET, DNV, lane, row, slot);
     }
   }
+  const float Px = ((float)x - d.ocx) * d.dx, Py = ((float)y - d.ocy) * d.dx;
+  const float lanef = (float)lane, glf = (float)g.gl;
+  const float DNVf = (float)DNV;
+  bool rest = false;
+  // views' records, [64][4]; the free fourth entries: offset of the first column, z0, z1 - z0, n
+  auto put = [&](MatchedRecord& v, int pos) {
+    v.t[0].w = __int_as_float(lane * frame + v.o);
+    v.t[1].w = __int_as_float(v.z0);
+    v.t[2].w = __int_as_float(v.z1 - v.z0);
+    v.t[3].w = __int_as_float(v.n);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) rec[4 * pos + t] = v.t[t];
+  };
+  for (int k0 = 0; k0 < A.vc; k0 += 64) {
+    const int kl = k0 + lane;
+    MatchedRecord v{};
+    if (kl < A.vc) v = matched_record(A, kl, 0, x, y, Px, Py, PACK ? g.L : 64, false);
+    rest = rest || __any(v.key == 1 || v.more);
+    if (!__any(v.key)) continue;
+    const int q_o = lane * frame + v.o;
+    int first[11], pos = lane;
+    if constexpr (PACK) pos = sort_classes(v.key, first);
+    if (v.key) put(v, pos);
+    const Buf<float> P(A.yp + (size_t)k0 * frame, (uint32_t)min(64, A.vc - k0) * (uint32_t)frame);
+    for_classes([&](auto NU_, auto MULTI_) {
+      constexpr int NU = decltype(NU_)::value;
+      constexpr bool MULTI = decltype(MULTI_)::value;
+      constexpr int K = 2 * NU + (MULTI ? 1 : 0);
+      struct Set {
+        float y[NU][NC];
+      };
+      if constexpr (PACK) {
+        const int n = first[K + 1] - first[K];
+        if (!n) return;
+        const float4* rc = rec + 4 * first[K];
+        pipelined_n<Set>(
+            g.rounds(n),
+            [&](int i, Set& f) {
+              const int o = __float_as_int(rc[4 * min(i * g.G + g.grp, n - 1)].w) + row[0];
+#pragma unroll
+              for (int t = 0; t < NU; ++t) f.y[t][0] = P.at(o, t * DNV);
+            },
+            [&](int i, const Set& f) {
+              const int e = i * g.G + g.grp;
+              const float4* re = rc + 4 * min(e, n - 1);
+              float4 r[NU];
+#pragma unroll
+              for (int t = 0; t < NU; ++t) {
+                r[t] = re[t];
+                rows[t * SET + slot[0]] = r[t].z * f.y[t][0];
+              }
+              const int zf = __float_as_int(re[1].w);
+              const int last = e < n && g.gl < g.L ? __float_as_int(re[2].w) : -1;
+              const float* R0 = rows + g.rows + kPadRows;
+              float* a = lacc + g.sums + zf + g.gl;
+              if constexpr (MULTI) {
+                float zi = glf;
+                for (int zz = 0; __any(zz <= last); zz += g.L, zi += (float)g.L)
+                  if (g.gl <= last - zz)
+                    a[zz] += matched_voxel<NU, 3>(r, NU, zi, R0, SET, DNVf);
+              } else {
+                if (g.gl <= last) *a += matched_voxel<NU, 3>(r, NU, glf, R0, SET, DNVf);
+              }
+            });
+      } else {
+        const uint64_t m = __ballot(v.key == K);
+        if (!m) return;
+        pipelined<Set>(
+            m,
+            [&](int j, Set& f) {
+              const int o = __builtin_amdgcn_readlane(q_o, j);
+#pragma unroll
+              for (int t = 0; t < NU; ++t)
+#pragma unroll
+                for (int h = 0; h < NC; ++h) f.y[t][h] = P.at(row[h], o + t * DNV);
+            },
+            [&](int j, const Set& f) {
+              float4 r[NU];
+#pragma unroll
+              for (int t = 0; t < NU; ++t) {
+                r[t] = rec[4 * j + t];
+#pragma unroll
+                for (int h = 0; h < NC; ++h) rows[t * SET + slot[h]] = r[t].z * f.y[t][h];
+              }
+              const int zf = __builtin_amdgcn_readlane(v.z0, j);
+              const int n = __builtin_amdgcn_readlane(v.z1, j) - zf;
+              auto pass = [&](float zi, int zz) {
+                lacc[zf + zz + lane] +=
+                    matched_voxel<NU, 3>(r, NU, zi, rows + kPadRows, SET, DNVf);
+              };
+              if constexpr (MULTI) {
+                float zi = lanef;
+                for (int zz = 0; zz <= n; zz += 64, zi += 64.f)
+                  if (lane <= n - zz) pass(zi, zz);
+              } else {
+                if (lane <= n) pass(lanef, 0);
+              }
+            });
+      }
+    });
+  }
+  // records of key 1 and views' further columns; all where a sum is not finite
+  const bool exact = reset_not_finite(lacc, sums);
+  if (rest || exact)
+    for (int k0 = 0, c0 = 0; k0 < A.vc;) {
+      const int kl = k0 + lane;
+      MatchedRecord v{};
+      if (kl < A.vc) v = matched_record(A, kl, c0, x, y, Px, Py, 64, exact || c0 > 0);
+      const uint64_t m = __ballot(v.key == 1);
+      if (v.key == 1)
+        put(v, PACK ? (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                     __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0))
+                    : lane);
+      const Buf<float> P(A.yp + (size_t)k0 * frame,
+                         (uint32_t)min(64, A.vc - k0) * (uint32_t)frame);
+      struct Set {
+        float y[4][NC];
+      };
+      // whether five taps stay on the row sets and their zeros over the whole window
+      auto five = [&](const float4(&r)[4], int nc, int last) {
+        bool ok = true;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          ok = ok && (t >= nc || (r[t].y <= kTaps5 && r[t].x >= (float)-kPadRows &&
+                                  fmaf((float)last, r[t].y, r[t].x) < (float)(DNV + 1)));
+        return ok;
+      };
+      // the record at re, this lane's rows from offset o, voxels gl, gl + step, ...
+      auto load = [&](const float4* re, Set& f) {
+        const int o = __float_as_int(re[0].w), last = __float_as_int(re[3].w) - 1;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int h = 0; h < NC; ++h) f.y[t][h] = P.at(o + row[h] + min(t, last) * DNV, 0);
+      };
+      auto use = [&](const float4* re, const Set& f, bool act, int gl, int step) {
+        float4 r[4];
+        bool own = exact;  // read the shadows' own rows only
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          r[t] = re[t];
+#pragma unroll
+          for (int h = 0; h < NC; ++h) {
+            rows[t * SET + slot[h]] = r[t].z * f.y[t][h];
+            own = own || not_finite(f.y[t][h]);
+          }
+        }
+        const int zf = __float_as_int(re[1].w), nc = __float_as_int(re[3].w);
+        const int last = act ? __float_as_int(re[2].w) : -1;
+        const float* R0 = rows + (PACK ? g.rows : 0) + kPadRows;
+        float* a = lacc + (PACK ? g.sums : 0) + zf;
+        if (__any(own || (act && !five(r, nc, last)))) {
+          for (int zz = gl; zz <= last; zz += step)
+            a[zz] += matched_voxel<4, 0>(r, nc, (float)zz, R0, SET, DNVf);
+        } else {
+          for (int zz = gl; zz <= last; zz += step)
+            a[zz] += matched_voxel<4, 5>(r, nc, (float)zz, R0, SET, DNVf);
+        }
+      };
+      if (m) {
+        if constexpr (PACK) {
+          const int n = __builtin_popcountll(m);
+          pipelined_n<Set>(
+              g.rounds(n),
+              [&](int i, Set& f) { load(rec + 4 * min(i * g.G + g.grp, n - 1), f); },
+              [&](int i, const Set& f) {
+                const int e = i * g.G + g.grp;
+                use(rec + 4 * min(e, n - 1), f, e < n && g.gl < g.L, g.gl, g.L);
+              });
+        } else {
+          pipelined<Set>(
+              m, [&](int j, Set& f) { load(rec + 4 * j, f); },
+              [&](int j, const Set& f) { use(rec + 4 * j, f, true, lane, 64); });
+        }
+      }
+      const bool more = __any(v.more);
+      c0 = more ? c0 + 4 : 0;
+      k0 = more ? k0 : k0 + 64;
+    }
   for (int z = lane; z < d.ZN; z += 64) {
-    const float a = lacc[z] * mk;
+    float a = lacc[z];
+    if constexpr (PACK)
+      for (int k = 1; k < g.G; ++k) a += lacc[k * ZN4 + z];
+    a *= mk;
     if constexpr (UPDATE) {
       const size_t i = (size_t)col * d.ZN + z;
-      const float nx = fmaf(a, invCol[i], vcol[z]);
+      const float nx = fmaf(a, A.invCol[i], vcol[z]);
       vcol[z] = nx;
-      if (shadow) shadow[i] = to_bf16_dither(nx, i);
+      if (A.shadow) A.shadow[i] = to_bf16_dither(nx, i);
     } else {
       vcol[z] = a;
     }
@@ -2101,7 +2654,7 @@ template <typename T>
 BpArgs<T> bp_args(const Plan& P, const T* prj, float* vol, int vb, int vs, int vc,
                   const float* invCol, uint16_t* shadow) {
   return BpArgs<T>{prj, vol, P.views, P.src64, P.mask, P.d, P.bc, P.bc64, vb, vs, vc,
-                   invCol, shadow};
+                   invCol, shadow, bp_pack_lanes(P, false)};
 }
 
 int fp_blocks_per_view(const Plan& P, bool colw) {
@@ -2116,13 +2669,16 @@ int launch_fp(const Plan& P, const TV* vol, TO* out, int vb, int vs, int vc, hip
   const int bpv = fp_blocks_of(P, A.lg);
   const dim3 grid(xcd_chunked_grid((long long)bpv * vc));
   const bool colw = A.lg == 6;
+#define CTR_FP(FUSED, COLW)                                                                   \
+  hipLaunchKernelGGL((fp_kernel<FUSED, COLW, TV, TO>), grid, dim3(kBlock), 0, st, A, bpv, vc)
   if (b) {
-    if (colw) hipLaunchKernelGGL((fp_kernel<true, true, TV, TO>), grid, dim3(kBlock), 0, st, A, bpv, vc);
-    else hipLaunchKernelGGL((fp_kernel<true, false, TV, TO>), grid, dim3(kBlock), 0, st, A, bpv, vc);
+    if (colw) CTR_FP(true, true);
+    else CTR_FP(true, false);
   } else {
-    if (colw) hipLaunchKernelGGL((fp_kernel<false, true, TV, TO>), grid, dim3(kBlock), 0, st, A, bpv, vc);
-    else hipLaunchKernelGGL((fp_kernel<false, false, TV, TO>), grid, dim3(kBlock), 0, st, A, bpv, vc);
+    if (colw) CTR_FP(false, true);
+    else CTR_FP(false, false);
   }
+#undef CTR_FP
   return check_launch("fp_kernel");
 }
 
@@ -2139,6 +2695,32 @@ int launch_fp_ones(const Plan& P, float* out, int vb, int vs, int vc, hipStream_
   return check_launch("fp_ones_kernel");
 }
 
+// Lanes of a packed wave's groups (bp_packed_body), 0 for one view at a time.  A group holds a
+// view's rows and, where they fit half a wave, the voxels of a column that its cone covers at
+// the grid's far edge, DNV l / (S dz) at distance l; a longer window takes a second pass.  The
+// windows at the axis (matched: at the far edge) must fit two groups: 512^2 x 256, 32 rows on
+// windows of 30 voxels, 38 at the far edge, one view at a time and packed: 2.13 ms, 1.92 ms
+// (matched 3.48 ms, 3.65 ms).  The groups' column sums must fit kPackSums floats, a sixth of
+// the LDS with four waves: at that limit (16 rows, 256^2 x 512) 578 us, 459 us (matched 938 us,
+// 866 us).
+int bp_pack_lanes(const Plan& P, bool matched) {
+  const Dims& d = P.d;
+  if (d.DNV > 32 || !bp_row_chunks(d.DNU, d.DNV)) return 0;
+  const double perl = d.DNV / (std::fabs((double)P.bc.S) * d.dz);
+  const double sid = 1.0 / P.bc64.inv_sid, R = 0.5 * std::max(d.XN, d.YN) * (double)d.dx;
+  const double axis = perl * sid + 2.0, edge = perl * (sid + R) + 2.0;
+  if (!((matched ? edge : axis) <= 32.0)) return 0;
+  const int need = std::max({d.DNV, (int)std::min(edge, 32.0), 8});
+  const int G = std::min(64 / need, kPackSums / ((d.ZN + 3) & ~3));
+  return G >= 2 ? 64 / G : 0;
+}
+
+BpShape bp_shape(const Plan& P, bool matched) {
+  const int L = bp_pack_lanes(P, matched), ZN4 = (P.d.ZN + 3) & ~3;
+  if (L) return {kPacked, 64 / L * ZN4};
+  return {bp_row_chunks(P.d.DNU, P.d.DNV), ZN4};
+}
+
 // Row chunks (of 64) a staged wave holds for a detector, 0 for the unstaged form: over 256
 // rows, or 64 frames past the staged loads' 32-bit byte offsets.
 int bp_row_chunks(int DNU, int DNV) {
@@ -2150,14 +2732,18 @@ int launch_bp_ones(const Plan& P, float* vol, int vb, int vs, int vc, hipStream_
   if (P.d.ZN > kWinMaxZ) return fail(CTR_ERR_ARG, "bp of ones: columns over the LDS limit");
   const BpArgs<float> A = bp_args<float>(P, nullptr, vol, vb, vs, vc, nullptr, nullptr);
   const dim3 wgrid((P.d.XN * P.d.YN + kWaves - 1) / kWaves);
-  const int rc = bp_row_chunks(P.d.DNU, P.d.DNV);
-  const size_t lds = (size_t)kWaves * bp_win_floats(rc, P.d.ZN) * sizeof(float);
-  switch (rc) {
-    case 1: hipLaunchKernelGGL(bp_win_ones_kernel<1>, wgrid, dim3(kBlock), lds, st, A); break;
-    case 2: hipLaunchKernelGGL(bp_win_ones_kernel<2>, wgrid, dim3(kBlock), lds, st, A); break;
-    case 4: hipLaunchKernelGGL(bp_win_ones_kernel<4>, wgrid, dim3(kBlock), lds, st, A); break;
-    default: hipLaunchKernelGGL(bp_win_ones_kernel<0>, wgrid, dim3(kBlock), lds, st, A); break;
+  const BpShape sh = bp_shape(P, false);
+  const size_t lds = (size_t)kWaves * bp_win_floats(sh.rc, sh.sums) * sizeof(float);
+#define CTR_BPO(RC) \
+  hipLaunchKernelGGL(bp_win_ones_kernel<RC>, wgrid, dim3(kBlock), lds, st, A, sh.sums)
+  switch (sh.rc) {
+    case kPacked: CTR_BPO(kPacked); break;
+    case 1: CTR_BPO(1); break;
+    case 2: CTR_BPO(2); break;
+    case 4: CTR_BPO(4); break;
+    default: CTR_BPO(0); break;
   }
+#undef CTR_BPO
   return check_launch("bp_win_ones_kernel");
 }
 
@@ -2170,25 +2756,27 @@ int launch_bp(const Plan& P, const T* prj, float* vol, int vb, int vs, int vc, i
     if constexpr (!std::is_same<T, float>::value) {
       return fail(CTR_ERR_ARG, "the matched back projector reads the FP32 scaled sinogram");
     } else {
-      const int rc = bp_row_chunks(P.d.DNU, P.d.DNV);
-      const size_t slds = (size_t)kWaves * bp_matched_floats(rc, P.d.ZN) * sizeof(float);
-      if (P.d.even_rows && rc > 0 && P.d.ZN <= kWinMaxZ && slds <= 65536) {
+      const BpShape sh = bp_shape(P, true);
+      const size_t slds = (size_t)kWaves * bp_matched_floats(sh.rc, sh.sums) * sizeof(float);
+      if (P.d.even_rows && sh.rc != 0 && P.d.ZN <= kWinMaxZ && slds <= 65536) {
         const dim3 wgrid((P.d.XN * P.d.YN + kWaves - 1) / kWaves);
-#define CTR_BPMS(UPD, RC, IC, SH)                                                              \
-  hipLaunchKernelGGL((bp_matched_staged_kernel<UPD, RC>), wgrid, dim3(kBlock), slds, st, prj,  \
-                     vol, P.views, P.bnd64, P.cols, P.Bz, P.mask, P.d, P.bc, vb, vs, vc, IC, SH)
-        if (accumulate) {
-          switch (rc) {
-            case 1: CTR_BPMS(true, 1, invCol, shadow); break;
-            case 2: CTR_BPMS(true, 2, invCol, shadow); break;
-            default: CTR_BPMS(true, 4, invCol, shadow); break;
-          }
-        } else {
-          switch (rc) {
-            case 1: CTR_BPMS(false, 1, nullptr, nullptr); break;
-            case 2: CTR_BPMS(false, 2, nullptr, nullptr); break;
-            default: CTR_BPMS(false, 4, nullptr, nullptr); break;
-          }
+        const MatchedArgs M{prj, vol, P.views, P.bnd64, P.cols, P.Bz, P.mask, P.d, P.bc, vb, vs,
+                            vc, bp_pack_lanes(P, true), accumulate ? invCol : nullptr,
+                            accumulate ? shadow : nullptr};
+#define CTR_BPMS(RC)                                                                           \
+  do {                                                                                         \
+    if (accumulate)                                                                            \
+      hipLaunchKernelGGL((bp_matched_staged_kernel<true, RC>), wgrid, dim3(kBlock), slds, st,  \
+                         M, sh.sums);                                                          \
+    else                                                                                       \
+      hipLaunchKernelGGL((bp_matched_staged_kernel<false, RC>), wgrid, dim3(kBlock), slds, st, \
+                         M, sh.sums);                                                          \
+  } while (0)
+        switch (sh.rc) {
+          case kPacked: CTR_BPMS(kPacked); break;
+          case 1: CTR_BPMS(1); break;
+          case 2: CTR_BPMS(2); break;
+          default: CTR_BPMS(4); break;
         }
 #undef CTR_BPMS
         return check_launch("bp_matched_staged_kernel");
@@ -2235,16 +2823,19 @@ int launch_bp(const Plan& P, const T* prj, float* vol, int vb, int vs, int vc, i
                                  accumulate ? shadow : nullptr);
   if (P.d.ZN <= kWinMaxZ) {
     const dim3 wgrid((P.d.XN * P.d.YN + kWaves - 1) / kWaves);
-    const int rc = bp_row_chunks(P.d.DNU, P.d.DNV);
-    const size_t lds = (size_t)kWaves * bp_win_floats(rc, P.d.ZN) * sizeof(float);
+    const BpShape sh = bp_shape(P, false);
+    const size_t lds = (size_t)kWaves * bp_win_floats(sh.rc, sh.sums) * sizeof(float);
 #define CTR_BPW(RC)                                                                           \
   do {                                                                                        \
     if (accumulate)                                                                           \
-      hipLaunchKernelGGL((bp_win_kernel<true, T, RC>), wgrid, dim3(kBlock), lds, st, A);      \
+      hipLaunchKernelGGL((bp_win_kernel<true, T, RC>), wgrid, dim3(kBlock), lds, st, A,       \
+                         sh.sums);                                                            \
     else                                                                                      \
-      hipLaunchKernelGGL((bp_win_kernel<false, T, RC>), wgrid, dim3(kBlock), lds, st, A);     \
+      hipLaunchKernelGGL((bp_win_kernel<false, T, RC>), wgrid, dim3(kBlock), lds, st, A,      \
+                         sh.sums);                                                            \
   } while (0)
-    switch (rc) {
+    switch (sh.rc) {
+      case kPacked: CTR_BPW(kPacked); break;
       case 1: CTR_BPW(1); break;
       case 2: CTR_BPW(2); break;
       case 4: CTR_BPW(4); break;
@@ -2317,23 +2908,24 @@ int launch_bp_batch(const BpBatchItem<T>* items, int nscan, int total, int zg, i
 }
 
 template <typename T>
-int launch_bp_batch_win(const BpBatchItem<T>* items, int nscan, int total, int zmax, int rc,
+int launch_bp_batch_win(const BpBatchItem<T>* items, int nscan, int total, int sums, int rc,
                         int grid, int strided, hipStream_t st) {
   if (total <= 0) return CTR_OK;
-  if (zmax < 1 || zmax > kWinMaxZ) return fail(CTR_ERR_ARG, "bp_batch_win: column height");
+  if (sums < 1 || sums > kWinMaxZ) return fail(CTR_ERR_ARG, "bp_batch_win: column height");
   const int sched = grid <= 0 ? 2 : (strided ? 1 : 0);
   grid = grid <= 0 ? total : std::max(1, std::min(grid, total));
-  const size_t lds = (size_t)kWaves * bp_win_floats(rc, zmax) * sizeof(float);
+  const size_t lds = (size_t)kWaves * bp_win_floats(rc, sums) * sizeof(float);
 #define CTR_BPBW(RC)                                                                          \
   do {                                                                                        \
     if (sched == 2)                                                                           \
       hipLaunchKernelGGL((bp_batch_win1_kernel<T, RC>), dim3(grid), dim3(kBlock), lds, st,    \
-                         items, nscan, total, zmax);                                          \
+                         items, nscan, total, sums);                                          \
     else                                                                                      \
       hipLaunchKernelGGL((bp_batch_win_kernel<T, RC>), dim3(grid), dim3(kBlock), lds, st,     \
-                         items, nscan, total, sched, zmax);                                   \
+                         items, nscan, total, sched, sums);                                   \
   } while (0)
   switch (rc) {
+    case kPacked: CTR_BPBW(kPacked); break;
     case 1: CTR_BPBW(1); break;
     case 2: CTR_BPBW(2); break;
     case 4: CTR_BPBW(4); break;
