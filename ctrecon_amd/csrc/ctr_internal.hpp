@@ -309,7 +309,11 @@ int launch_fill(float* p, size_t n, float v, hipStream_t st);
 int launch_copy(float* dst, const float* src, size_t n, hipStream_t st);
 int launch_inv_guard(const float* in, float* out, size_t n, hipStream_t st);
 int launch_axpy(float* y, const float* x, double a, size_t n, hipStream_t st);
-int launch_xpby(float* p, const float* r, double b, size_t n, hipStream_t st);
+// A CG iteration's updates of x, r and p with alpha = *rr / *pAp and beta = *rr1 / *rr, *rr1 the
+// new r.r; all on the device.
+int launch_cg_update(float* x, float* r, float* p, const float* t, size_t n, const double* rr,
+                     const double* pAp, double* rr1, double* partials, int nparts,
+                     hipStream_t st);
 int launch_sub(float* out, const float* a, const float* b, size_t n, hipStream_t st);
 int launch_dot(const float* a, const float* b, size_t n, double* partials, int nparts,
                double* result, hipStream_t st);

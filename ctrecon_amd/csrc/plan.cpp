@@ -1098,36 +1098,34 @@ int ctr_conjgrad(ctr_plan* plan, float* d_x, const float* d_prj, int iterNum, in
     if (e) return e;
     return bp_any<float>(*P, sino.f(), out, 0, 1, d.PN, bp_kind, st, nullptr, 0);
   };
-  auto dot = [&](const float* a, const float* b, double* outv) -> int {
-    int e = launch_dot(a, b, NV, P->partials, nparts, dots, st);
-    if (e) return e;
-    double h[2];
-    if (hipMemcpyAsync(h, dots, sizeof(h), hipMemcpyDeviceToHost, st) != hipSuccess ||
-        hipStreamSynchronize(st) != hipSuccess)
-      return fail(CTR_ERR_HIP, "dot readback failed");
-    *outv = h[0];
-    return CTR_OK;
+  // scalars on the device: p.Ap, and r.r of the last kRing iterations, read back together
+  constexpr int kRing = 32;
+  static_assert(2 + 2 * (kRing + 1) <= kResidualSums, "CG scalars");
+  double* pAp = dots;
+  auto rr = [&](int it) { return dots + 2 + 2 * (it % (kRing + 1)); };
+  auto dot = [&](const float* a, const float* b, double* out) {
+    return launch_dot(a, b, NV, P->partials, nparts, out, st);
   };
   // b = Back(prj); r0 = b - A(x0); p0 = r0 (conjgrad.m:7-9)
   if ((rc = bp_any(*P, d_prj, r.f(), 0, 1, d.PN, bp_kind, st, nullptr, 0))) return rc;
   if ((rc = A(d_x, t.f()))) return rc;
   if ((rc = launch_sub(r.f(), r.f(), t.f(), NV, st))) return rc;
   CTR_HIP(hipMemcpyAsync(pv.p, r.p, NV * sizeof(float), hipMemcpyDeviceToDevice, st));
-  double rr;
-  if ((rc = dot(r.f(), r.f(), &rr))) return rc;
-  for (int it = 0; it < iterNum; ++it) {
+  if ((rc = dot(r.f(), r.f(), rr(0)))) return rc;
+  for (int it = 0, done = 0; it < iterNum; ++it) {
     if ((rc = A(pv.f(), t.f()))) return rc;  // conjgrad.m:14
-    double pAp;
-    if ((rc = dot(pv.f(), t.f(), &pAp))) return rc;
-    const double alpha = rr / pAp;  // conjgrad.m:18
-    if ((rc = launch_axpy(d_x, pv.f(), alpha, NV, st))) return rc;    // :19
-    if ((rc = launch_axpy(r.f(), t.f(), -alpha, NV, st))) return rc;  // :20
-    double r1;
-    if ((rc = dot(r.f(), r.f(), &r1))) return rc;
-    const double beta = r1 / rr;  // :24
-    if ((rc = launch_xpby(pv.f(), r.f(), beta, NV, st))) return rc;  // :25
-    rr = r1;
-    if (resid) resid[it] = std::sqrt(r1);
+    if ((rc = dot(pv.f(), t.f(), pAp))) return rc;
+    // alpha, x, r, beta and p (conjgrad.m:18-25)
+    if ((rc = launch_cg_update(d_x, r.f(), pv.f(), t.f(), NV, rr(it), pAp, rr(it + 1),
+                               P->partials, nparts, st)))
+      return rc;
+    if (resid && (it + 1 == iterNum || it + 1 - done == kRing)) {
+      double h[2 * (kRing + 1)];
+      if (hipMemcpyAsync(h, rr(0), sizeof(h), hipMemcpyDeviceToHost, st) != hipSuccess ||
+          hipStreamSynchronize(st) != hipSuccess)
+        return fail(CTR_ERR_HIP, "dot readback failed");
+      for (; done <= it; ++done) resid[done] = std::sqrt(h[2 * ((done + 1) % (kRing + 1))]);
+    }
   }
   CTR_HIP(hipStreamSynchronize(st));
   return CTR_OK;
