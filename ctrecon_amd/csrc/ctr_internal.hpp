@@ -61,7 +61,7 @@ struct Dims {
   float beta0, dbeta_g;  // fan angle of boundary 0 and mean boundary spacing (adjoint guess)
   float B0, dB;          // row boundary index of row 0 and mean spacing (adjoint guess)
   float dBmin;           // smallest row spacing of the FP32 boundary table
-  float dBmax;           // largest row height (dBz)
+  float dBmax;           // largest row height (bz_(v+1) - bz_v)/dz
   double B0_64, dB_64;   // row boundary 0 and the mean spacing, FP64
   int even_rows;         // 1: every row boundary is B0 + v dB to within the FP32 rounding of
                          // the given row positions
@@ -85,7 +85,6 @@ struct FpArgs {
   const double2* bnd64;
   const float4* cols;
   const float* Bz;
-  const float* dBz;
   const float* h2;
   const float* invdB;
   const float* maskf;
@@ -164,7 +163,7 @@ struct PlanTables {
   float2* bnd;
   double2* bnd64;
   float4* cols;
-  float *Bz, *dBz, *h2, *invdB, *zc, *maskf;
+  float *Bz, *h2, *invdB, *zc, *maskf;
   float2* mext;
 };
 int launch_plan_tables(const PlanTables& T, hipStream_t st);
@@ -183,7 +182,6 @@ struct Plan {
   double2* bnd64 = nullptr;    // [PN][DNU+1]  the same in FP64 (forward projector, transpose)
   float4* cols = nullptr;      // [PN][DNU]    (r0, r1, G, Q)
   float* Bz = nullptr;         // [DNV+1]      (bz_v - z0)/dz
-  float* dBz = nullptr;        // [DNV]        row heights (bz_(v+1) - bz_v)/dz
   float* h2 = nullptr;         // [DNV]        (zds_v - z0)^2
   float* invdB = nullptr;      // [DNV]        1/(Bz[v+1]-Bz[v])
   double2* rot64 = nullptr;    // [PN]         (cos, sin) of the regularised view angle, FP64

@@ -293,7 +293,6 @@ static int build_tables(const ctr_geometry* g, Plan& P, double half = 0.0) {
       (rc = table_alloc((void**)&P.bnd64, lines * sizeof(double2))) ||
       (rc = table_alloc((void**)&P.cols, (size_t)PN * DNU * sizeof(float4))) ||
       (rc = table_alloc((void**)&P.Bz, (DNV + 1) * sizeof(float))) ||
-      (rc = table_alloc((void**)&P.dBz, DNV * sizeof(float))) ||
       (rc = table_alloc((void**)&P.h2, DNV * sizeof(float))) ||
       (rc = table_alloc((void**)&P.invdB, DNV * sizeof(float))) ||
       (rc = table_alloc((void**)&P.zc, DNV * sizeof(float))) ||
@@ -302,7 +301,7 @@ static int build_tables(const ctr_geometry* g, Plan& P, double half = 0.0) {
     return rc;
   T.views = P.views; T.src64 = P.src64; T.rot64 = P.rot64; T.det64 = P.det64; T.mask = P.mask;
   T.bnd = P.bnd; T.bnd64 = P.bnd64; T.cols = P.cols;
-  T.Bz = P.Bz; T.dBz = P.dBz; T.h2 = P.h2; T.invdB = P.invdB; T.zc = P.zc;
+  T.Bz = P.Bz; T.h2 = P.h2; T.invdB = P.invdB; T.zc = P.zc;
   T.maskf = P.maskf; T.mext = P.mext;
   return launch_plan_tables(T, nullptr);
 }
@@ -316,7 +315,6 @@ static void free_plan(Plan* P) {
   (void)hipFree(P->bnd64);
   (void)hipFree(P->cols);
   (void)hipFree(P->Bz);
-  (void)hipFree(P->dBz);
   (void)hipFree(P->h2);
   (void)hipFree(P->invdB);
   (void)hipFree(P->mext);

@@ -86,7 +86,6 @@ __global__ __launch_bounds__(kTB) void plan_tables_kernel(PlanTables T, TableBlo
     T.h2[v] = (float)(h * h);
     T.zc[v] = (float)(h / T.dz);
     T.invdB[v] = (float)(T.dz / step);
-    T.dBz[v] = (float)(step / T.dz);
   }
 }
 
