@@ -192,7 +192,7 @@ __device__ __forceinline__ void z_run(const Buf<uint16_t>&, const uint16_t* vol,
 //
 // Groups (fewer than 64 rows to a column) gather each cell's taps as one load per lane:
 // 64^3, 720 views of 256 x 16, 212 us one thread per ray with its own FP64 footprints,
-// 85 us with four columns per wave.
+// 88 us with four columns per wave.
 //
 // ONES: the projection of a volume of ones (the row sums of OS-SART), read from no volume.
 // A slice wholly inside the volume's z range adds its height times its cells' weights; the
@@ -2668,7 +2668,7 @@ int check_launch(const char* what) {
 // Lanes per item (log2) of the forward projector for a detector of DNV rows: the least
 // lanes spent per column, each weighed by the instructions it issues per slice -- about 20
 // with one column per wave, 25 in groups, and the FP64 evaluation of a slice (about 130)
-// once per L slices.  16 rows: four columns per wave, 85 us against 212 us one thread per
+// once per L slices.  16 rows: four columns per wave, 88 us against 212 us one thread per
 // ray (64^3, 720 views); 40 rows: one column per wave (24 lanes idle), 0.94 ms against
 // 2.19 ms (301^2 x 143, 234 views); 80 rows: groups of 16 without idle lanes.
 int fp_lanes_log2(int DNV) {
