@@ -187,8 +187,8 @@ __device__ __forceinline__ void z_run(const Buf<uint16_t>&, const uint16_t* vol,
 // and every row takes its two or three taps there; the next slice's runs load meanwhile.
 // What bounds it then is VALU issue (0.95 of the chip's rate, about 22 instructions per
 // wave and slice).  512^2 x 256, 197 views of 888 x 64: 4.06 ms with a gather per cell and
-// lane, 3.00 ms with slices in classes, 2.37 ms with runs and the deal of
-// xcd_chunked_block; BF16 4.19 ms, 3.32 ms, 1.99 ms.
+// lane, 3.00 ms with slices in classes, 2.27 ms with runs and the deal of
+// xcd_chunked_block; BF16 4.19 ms, 3.32 ms, 1.97 ms.
 //
 // Groups (fewer than 64 rows to a column) gather each cell's taps as one load per lane:
 // 64^3, 720 views of 256 x 16, 212 us one thread per ray with its own FP64 footprints,
@@ -308,7 +308,7 @@ __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk
             q_e += q_kb;
             q_last = floor_i(fmaf(o.r, Btop, azf)) - q_kb + 2;
             if (q_last > 63) cls |= 2;
-            gen = gen || q_last > 127 || q_e + (o.nj - 1) * cS + 128 > NV;
+            gen = gen || q_last > 127 || q_e + (max(o.nj, 2) - 1) * cS + 128 > NV;
           } else {
             // a run's elements stay inside the array: not on its last column
             gen = gen || e + (o.nj - 1) * cS + d.ZN + 4 > NV;
@@ -326,13 +326,14 @@ __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk
         }
       }
       if (!__any(mj)) continue;
-      // the class as a number: cells * 8 + 0 two taps, 1 three taps, 2 three taps of more than
+      // the class as a number: cells (one counts as two, the second of weight 0: the two are mixed
+      // along a ray, and one class keeps more loads in flight; 512^2 x 256, 2.37 ms with classes of
+      // their own, 2.27 ms) * 8 + 0 two taps, 1 three taps, 2 three taps of more than
       // 64 cells, 3 past the volume's ends; 7 the general form, 0 no footprint
       const int id = cls >= 4 ? 3 : min(cls, 2);
-      const int key = cls >= 8 ? 7 : (mj == 0 ? 0 : id + 8 * (COLW ? mj : max(mj, 2)));
+      const int key = cls >= 8 ? 7 : (mj == 0 ? 0 : id + 8 * max(mj, 2));
       const uint64_t low = ~0ull >> (64 - L);
       using std::integral_constant;
-      using I1 = integral_constant<int, 1>;
       using I2 = integral_constant<int, 2>;
       using I3 = integral_constant<int, 3>;
       using I4 = integral_constant<int, 4>;
@@ -424,7 +425,6 @@ __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk
           run(NJ_, I3{}, T{}, F{}, 2);
           run(NJ_, I3{}, T{}, T{}, 3);
         };
-        cells(I1{});
         cells(I2{});
         cells(I3{});
         cells(I4{});
