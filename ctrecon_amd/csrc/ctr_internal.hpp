@@ -316,7 +316,12 @@ int launch_sub(float* out, const float* a, const float* b, size_t n, hipStream_t
 int launch_dot(const float* a, const float* b, size_t n, double* partials, int nparts,
                double* result, hipStream_t st);
 int launch_reduce_pairs(const double* partials, int nparts, double* result, hipStream_t st);
+// Pairs of partial sums that a fused forward projection of vc views writes with the plan's
+// method: what is reduced.  most: the larger count of the two methods with a fused form, for
+// buffers that outlive a change of the method.
 int fp_partial_blocks(const Plan& P, int vc);
+int fp_partial_most(const Plan& P, int vc);
+int fp_sat_blocks(const Dims& d);
 // pseudo distance-driven pair (pdd.hip), FP32 operands
 int launch_fp_pdd(const Plan& P, const float* vol, float* out, int vb, int vs, int vc,
                   hipStream_t st);

@@ -2692,7 +2692,12 @@ static int fp_blocks_of(const Plan& P, int lg) {
 }
 
 int fp_partial_blocks(const Plan& P, int vc) {
+  if (P.method == CTR_METHOD_SAT) return fp_sat_blocks(P.d) * vc;
   return fp_blocks_of(P, fp_lanes_log2(P.d.DNV)) * vc;
+}
+
+int fp_partial_most(const Plan& P, int vc) {
+  return std::max(fp_sat_blocks(P.d), fp_blocks_of(P, fp_lanes_log2(P.d.DNV))) * vc;
 }
 
 template <typename TV, typename TO>

@@ -478,6 +478,8 @@ struct DBuf {
 
 int residual_chunk(const Plan& P) {
   const int views = std::min(P.d.PN, 256);
+  // (a chunk of the integral-image method builds the volume's tables again)
+  if (P.method == CTR_METHOD_SAT) return views;
   const long long most = (kResidualScratch - kResidualSums) / 2 / fp_partial_blocks(P, 1);
   return (int)std::max<long long>(1, std::min<long long>(views, most));
 }
@@ -794,7 +796,8 @@ int ctr_sart_create(ctr_plan* plan, const float* d_prj, int osNum, int bp_kind, 
     return rc;
   if (S->bf && (rc = S->xs.alloc(NV * sizeof(uint16_t)))) return rc;
   if ((rc = S->sums.alloc(2 * sizeof(double) * osNum))) return rc;
-  if ((rc = S->parts.alloc((2 * (size_t)fp_partial_blocks(*P, S->maxV) + 2) * sizeof(double))))
+  // (the plan's method may change between sweeps)
+  if ((rc = S->parts.alloc((2 * (size_t)fp_partial_most(*P, S->maxV) + 2) * sizeof(double))))
     return rc;
   hipStream_t st = P->stream;
   EventPool ev;

@@ -292,6 +292,9 @@ size_t sat_sino_floats(const Dims& d, int vc) {
   return (size_t)vc * (d.DNU + 1) * (d.DNV + 1);
 }
 
+// Workgroups (and pairs of partial sums) of the forward projector per view.
+int fp_sat_blocks(const Dims& d) { return (d.DNU * d.DNV + kBlock - 1) / kBlock; }
+
 // Volume integral images into sat: ZYX then ZXY texels, each texel (hi, lo).
 template <typename T>
 int launch_volume_sat(const Plan& P, const T* vol, float* sat, hipStream_t st) {
@@ -312,7 +315,7 @@ int launch_fp_sat(const Plan& P, const float* sat, TO* out, int vb, int vs, int 
   const size_t nx = (size_t)d.XN * (d.YN + 1) * (d.ZN + 1);
   const float2* zyx = reinterpret_cast<const float2*>(sat);
   const float2* zxy = zyx + nx;
-  dim3 grid((d.DNU * d.DNV + kBlock - 1) / kBlock, vc);
+  dim3 grid(fp_sat_blocks(d), vc);
   if (b)
     hipLaunchKernelGGL((fp_sat_kernel<true, TO>), grid, dim3(kBlock), 0, st, zyx, zxy, out,
                        P.views, P.bnd, P.cols, P.Bz, P.h2, d, vb, vs, b, invRow, partials);
