@@ -70,15 +70,16 @@ struct ctr_batch {
   Mem sums, zeros;  // sums: [n][osNum][2]; zeros: the largest volume (tuning)
   Mem fpItems, redItems;
   std::vector<int> fpTotal;
-  // back-projection work lists by class: c = 1..4 z groups per lane, c = 0 the windowed
-  // form (one wave per column over all z), c = 5 the windowed form of packed views; the scans
-  // of the class, and per subset step their items (and timing copies with a zero column sum)
-  static constexpr int kClasses = 6, kPackedClass = 5;
+  // back-projection work lists by class: c = 1..4 z groups per lane, c = 0 the windowed form
+  // with staged rows (one wave per column over all z), c = 5 that of packed views, c = 6 that
+  // without staged rows, each scan in the form that its own solver runs; the scans of the
+  // class, and per subset step their items (and timing copies with a zero column sum)
+  static constexpr int kClasses = 7, kPackedClass = 5, kUnstagedClass = 6;
   std::vector<int> clsScans[kClasses];
   Mem bpItems[kClasses], tuneBpItems[kClasses];
   std::vector<int> bpTotal[kClasses];
-  int winZ = 0, packSums = 0;  // most column sums of a wave of classes 0 and 5 (BpShape)
-  int winRC = 0;               // row chunks of the windowed class (bp_row_chunks)
+  // the launch of a windowed class: most row chunks and column sums of its scans (BpShape)
+  BpShape win[kClasses] = {};
   bool colw = false;
   // zg: z groups per lane (1..4; 0 and kZgWindow: each scan's own ceil(ZN / 64)) of the scans
   // with columns taller than kWinMaxZ; every other scan runs the windowed form
@@ -101,10 +102,14 @@ namespace {
 
 constexpr int kZgWindow = 5;
 
+bool windowed(int c) { return c < 1 || c > 4; }
+
 // back-projection class of a scan
 int scan_zg(const ctr_batch& B, const Plan& P) {
-  if (P.d.ZN <= kWinMaxZ)  // a windowed form, whatever zg
-    return bp_shape(P, false).rc == kPacked ? ctr_batch::kPackedClass : 0;
+  if (P.d.ZN <= kWinMaxZ) {  // a windowed form, whatever zg
+    const int rc = bp_shape(P, false).rc;
+    return rc == kPacked ? ctr_batch::kPackedClass : rc == 0 ? ctr_batch::kUnstagedClass : 0;
+  }
   return (B.zg > 0 && B.zg < kZgWindow) ? B.zg : std::min(4, (P.d.ZN + 63) / 64);
 }
 
@@ -118,23 +123,15 @@ int build_tables(ctr_batch& B) {
   for (int c = 0; c < B.kClasses; ++c) {
     B.clsScans[c].clear();
     B.bpTotal[c].assign(S, 0);
+    B.win[c] = {c == B.kPackedClass ? kPacked : 0, 0};
   }
-  B.winZ = B.packSums = 0;
-  bool staged = true;
-  B.winRC = 0;
   for (int i = 0; i < n; ++i) {
     const int c = scan_zg(B, *B.scans[i]->P);
     B.clsScans[c].push_back(i);
     const BpShape sh = bp_shape(*B.scans[i]->P, false);
-    if (c == 0) {
-      B.winZ = std::max(B.winZ, sh.sums);
-      staged = staged && sh.rc > 0;
-      B.winRC = std::max(B.winRC, sh.rc);
-    } else if (c == B.kPackedClass) {
-      B.packSums = std::max(B.packSums, sh.sums);
-    }
+    if (c == 0) B.win[c].rc = std::max(B.win[c].rc, sh.rc);
+    B.win[c].sums = std::max(B.win[c].sums, sh.sums);
   }
-  if (!staged) B.winRC = 0;
   auto up = [&](Mem& m, const void* src, size_t bytes) -> int {
     if (m.p) {
       (void)hipFree(m.p);
@@ -180,8 +177,7 @@ int build_tables(ctr_batch& B) {
                          B.bf ? c.xs.h() : nullptr);
         b.begin = bb;
         b.colBlocks = (P.d.XN * P.d.YN + 3) / 4;
-        const int zblocks =
-            cz == 0 || cz == B.kPackedClass ? 1 : (P.d.ZN + 64 * cz - 1) / (64 * cz);
+        const int zblocks = windowed(cz) ? 1 : (P.d.ZN + 64 * cz - 1) / (64 * cz);
         bb += vc > 0 ? b.colBlocks * zblocks : 0;
         BpBatchItem<T>& t = tbp[(size_t)s * m + j];
         t = b;
@@ -211,11 +207,9 @@ int step_bp(ctr_batch& B, int s, bool tuning) {
     if (!m) continue;
     const Mem& mem = tuning ? B.tuneBpItems[cz] : B.bpItems[cz];
     const BpBatchItem<T>* items = (const BpBatchItem<T>*)mem.p + (size_t)s * m;
-    const bool packed = cz == B.kPackedClass;
-    int rc = cz == 0 || packed
-                 ? launch_bp_batch_win<T>(items, (int)m, B.bpTotal[cz][s],
-                                          packed ? B.packSums : B.winZ, packed ? kPacked : B.winRC,
-                                          B.bpGrid, B.bpStrided, B.st)
+    int rc = windowed(cz)
+                 ? launch_bp_batch_win<T>(items, (int)m, B.bpTotal[cz][s], B.win[cz].sums,
+                                          B.win[cz].rc, B.bpGrid, B.bpStrided, B.st)
                  : launch_bp_batch<T>(items, (int)m, B.bpTotal[cz][s], cz, B.bpGrid, B.bpStrided,
                                       B.st);
     if (rc) return rc;

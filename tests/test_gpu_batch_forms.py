@@ -1,0 +1,53 @@
+"""Batches whose scans run different back projectors: every scan's iterate has the bits of a batch
+of its own with the same launch shapes, whatever the other scans need."""
+
+import numpy as np
+import pytest
+
+from ctrecon_amd import geometry as G
+
+pytestmark = pytest.mark.gpu
+
+SUBSETS = 4
+
+
+def _scan(dnv, nxy=20, nz=24, views=22, seed=0):
+    cfg = G.helical_config(sid=200, sdd=380, DNU=48, DNV=dnv, col_width=1.3, col_height=40.0 / dnv,
+                           views_per_turn=views, turns=1, feed_mm_per_turn=12.0, N_xy=nxy, N_z=nz,
+                           voxel_xy=1.0, voxel_z=1.0)
+    g = G.dd3_geometry(cfg, mask=G.fov_mask(nxy))
+    b = np.random.default_rng(dnv + seed).uniform(0, 10, g.prj_shape).astype(np.float32)
+    return g, b
+
+
+def _run(scans, tuning, storage="f32", sweeps=2):
+    """Iterates of a batch of the scans, and the plans' own buffers kept alive."""
+    from ctrecon_amd.batch import Batch
+    from ctrecon_amd.plan import DeviceArray, Plan
+
+    plans = [Plan(g, 0) for g, _ in scans]
+    for p in plans:
+        p.set_storage(storage)
+    bs = [DeviceArray.from_host(b) for _, b in scans]
+    xs = [DeviceArray(g.vol_shape) for g, _ in scans]
+    B = Batch(plans, xs, bs, SUBSETS)
+    B.set_tuning(*tuning)
+    for x in xs:
+        x.zero()
+    res, _ = B.sweeps(sweeps)
+    out = [x.get() for x in xs]
+    B.close()
+    return out, res
+
+
+@pytest.mark.parametrize("storage", ["f32", "bf16"])
+@pytest.mark.parametrize("grid", [0, 64])
+def test_scans_over_256_rows_leave_the_others(grid, storage, gpu_plan_factory):
+    print(f"[batch with 300 rows] grid={grid} storage={storage}", flush=True)
+    scans = [_scan(64), _scan(300), _scan(16), _scan(100)]
+    tuning = (False, grid, 5, grid)
+    got, res = _run(scans, tuning, storage)
+    for i, s in enumerate(scans):
+        own, own_res = _run([s], tuning, storage)
+        assert np.array_equal(got[i], own[0]), (i, s[0].DNV)
+        assert np.allclose(res[:, i], own_res[:, 0], rtol=1e-12, atol=0)
