@@ -272,11 +272,16 @@ std::string cache_path() {
   return dir + "/batch_tuning.txt";
 }
 
-// The device (architecture, CU count) and every scan's sizes, voxel sizes, source z
-// range and the subset count: what the launch costs depend on.
+// The revision of the launch shapes and kernels that the tuned values were timed on: raised
+// when these change, so that lines of earlier ones are not found.
+constexpr int kTuningRevision = 2;
+
+// The revision, the device (architecture, CU count) and every scan's sizes, voxel sizes, source
+// z range and the subset count: what the launch costs depend on.
 std::string cache_key(const ctr_batch& B) {
   hipDeviceProp_t prop;
   std::ostringstream k;
+  k << "r" << kTuningRevision << "|";
   if (hipGetDeviceProperties(&prop, B.device) == hipSuccess)
     k << prop.gcnArchName << "/" << prop.multiProcessorCount;
   k << "|os" << B.osNum << (B.bf ? "|bf16" : "|f32");

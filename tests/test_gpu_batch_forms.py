@@ -51,3 +51,30 @@ def test_scans_over_256_rows_leave_the_others(grid, storage, gpu_plan_factory):
         own, own_res = _run([s], tuning, storage)
         assert np.array_equal(got[i], own[0]), (i, s[0].DNV)
         assert np.allclose(res[:, i], own_res[:, 0], rtol=1e-12, atol=0)
+
+
+def test_tuning_of_earlier_kernels_is_not_used(tmp_path, monkeypatch, gpu_plan_factory):
+    """A stored line is found again by the same kernels, and not without their revision."""
+    from ctrecon_amd.batch import Batch
+    from ctrecon_amd.plan import DeviceArray, Plan
+
+    print("[tuning revision]", flush=True)
+    cache = tmp_path / "tuning.txt"
+    monkeypatch.setenv("CTRECON_TUNE_CACHE", str(cache))
+    g, b = _scan(40)
+    p, db, x = Plan(g, 0), DeviceArray.from_host(b), DeviceArray(g.vol_shape)
+    x.zero()
+
+    def info():
+        B = Batch([p], [x], [db], SUBSETS)
+        i = B.info()
+        B.close()
+        return i
+
+    assert info()["from_cache"] == 0
+    line = cache.read_text().splitlines()[-1]
+    assert info()["from_cache"] == 1
+    # the line's key starts at the device's name without a revision
+    key, values = line.split("\t")
+    cache.write_text(key[key.index("gfx"):] + "\t" + values + "\n")
+    assert info()["from_cache"] == 0
