@@ -64,7 +64,7 @@ struct Dims {
   float dBmax;           // largest row height (bz_(v+1) - bz_v)/dz
   double B0_64, dB_64;   // row boundary 0 and the mean spacing, FP64
   int even_rows;         // 1: every row boundary is B0 + v dB to within the FP32 rounding of
-                         // the given row positions
+                         // row positions relative to the source
 };
 
 // Host copies used by host-side accounting (cone voxel counts).

@@ -175,7 +175,9 @@ static int build_tables(const ctr_geometry* g, Plan& P, double half = 0.0) {
   {
     double far = 0.0, off = 0.0;
     for (int v = 0; v <= DNV; ++v) {
-      far = std::max(far, std::fabs(bz[v]));
+      // (from the source, as the FP32 boundary table holds them: rows far from z = 0 whose given
+      // positions are rounded more coarsely than that are uneven)
+      far = std::max(far, std::fabs(bz[v] - z0));
       off = std::max(off, std::fabs(bz[v] - (bz[0] + (bz[DNV] - bz[0]) * v / DNV)));
     }
     d.even_rows = off <= 4.0 * 0x1p-24 * far ? 1 : 0;
