@@ -228,12 +228,15 @@ int ensure_bytes(void** p, size_t* have, size_t need, const char* what);
 
 // Relative data residual ||A x - b|| / ||b|| over all views (FP64 sums, added in view
 // order), forward-projecting `chunk` views at a time into prj ([chunk][DNU][DNV]) with
-// partials (2 fp_partial_blocks(P, chunk) doubles) and sums (kResidualSums doubles) as
+// partials (2 fp_partial_blocks(P, chunk) doubles, for the direct method at most
+// 2 kResidualPairs) and sums (kResidualSums doubles) as
 // scratch, on stream st; synchronous.  Allocates nothing for the direct method.
 constexpr int kResidualSums = 128;
 // Views per chunk of both residual entry points (the same chunks give the same sums): at
-// most 256, fewer where their partial sums would exceed kResidualScratch doubles.
+// most 256, fewer where their partial sums would exceed kResidualScratch doubles; where one
+// view's would, it is taken in parts of its columns.
 constexpr long long kResidualScratch = 1ll << 19;
+constexpr long long kResidualPairs = (kResidualScratch - kResidualSums) / 2;
 int residual_chunk(const Plan& P);
 int residual_run(Plan& P, const float* d_x, const float* d_prj, float* prj, int chunk,
                  double* partials, double* sums, hipStream_t st, double* out);
@@ -322,6 +325,11 @@ int launch_reduce_pairs(const double* partials, int nparts, double* result, hipS
 int fp_partial_blocks(const Plan& P, int vc);
 int fp_partial_most(const Plan& P, int vc);
 int fp_sat_blocks(const Dims& d);
+// Parts of a view's columns: workgroups of a part, most columns within a number of them, launch.
+int fp_column_blocks(const Plan& P, int columns);
+int fp_columns_within(const Plan& P, long long blocks);
+int launch_fp_columns(const Plan& P, const float* vol, int p, int u0, int columns, hipStream_t st,
+                      const float* b, double* partials);
 // pseudo distance-driven pair (pdd.hip), FP32 operands
 int launch_fp_pdd(const Plan& P, const float* vol, float* out, int vb, int vs, int vc,
                   hipStream_t st);

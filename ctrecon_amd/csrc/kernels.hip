@@ -2685,10 +2685,21 @@ int fp_lanes_log2(int DNV) {
   return best;
 }
 
-static int fp_blocks_of(const Plan& P, int lg) {
+static int fp_blocks_of(const Plan& P, int lg, int columns) {
   const int L = 1 << lg, per = kWaves << (6 - lg);  // items per workgroup
-  const int items = P.d.DNU * ((P.d.DNV + L - 1) / L);
+  const int items = columns * ((P.d.DNV + L - 1) / L);
   return (items + per - 1) / per;
+}
+static int fp_blocks_of(const Plan& P, int lg) { return fp_blocks_of(P, lg, P.d.DNU); }
+
+int fp_column_blocks(const Plan& P, int columns) {
+  return fp_blocks_of(P, fp_lanes_log2(P.d.DNV), columns);
+}
+
+int fp_columns_within(const Plan& P, long long blocks) {
+  const int lg = fp_lanes_log2(P.d.DNV), L = 1 << lg;
+  const long long items = blocks * (kWaves << (6 - lg));
+  return (int)std::max(1ll, std::min<long long>(P.d.DNU, items / ((P.d.DNV + L - 1) / L)));
 }
 
 int fp_partial_blocks(const Plan& P, int vc) {
@@ -2737,6 +2748,27 @@ int launch_fp(const Plan& P, const TV* vol, TO* out, int vb, int vs, int vc, hip
     else CTR_FP(false, false);
   }
 #undef CTR_FP
+  return check_launch("fp_kernel");
+}
+
+// The fused partial sums of columns u0 ... u0 + columns - 1 of view p alone (no output): the
+// kernel on tables that begin there.
+int launch_fp_columns(const Plan& P, const float* vol, int p, int u0, int columns, hipStream_t st,
+                      const float* b, double* partials) {
+  const size_t at = (size_t)p * P.d.DNU + u0;
+  FpArgs<float, float> A = fp_args<float, float>(P, vol, nullptr, 0, 1, b + at * P.d.DNV, nullptr,
+                                                 partials);
+  A.views += p;
+  A.bnd64 += at + p;
+  A.cols += at;
+  A.d.DNU = columns;
+  const int bpv = fp_blocks_of(P, A.lg, columns);
+  const dim3 grid(xcd_chunked_grid(bpv));
+  if (A.lg == 6)
+    hipLaunchKernelGGL((fp_kernel<true, true, float, float>), grid, dim3(kBlock), 0, st, A, bpv, 1);
+  else
+    hipLaunchKernelGGL((fp_kernel<true, false, float, float>), grid, dim3(kBlock), 0, st, A, bpv,
+                       1);
   return check_launch("fp_kernel");
 }
 

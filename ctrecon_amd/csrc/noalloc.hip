@@ -66,10 +66,8 @@ int ctr_residual_noalloc(ctr_plan* plan, const float* d_x, const float* d_prj, d
                     " doubles of scratch; the maximum is " + std::to_string(kScratchDoubles) +
                     " (4 MiB): use ctr_residual");
   const int chunk = residual_chunk(*P);
-  const size_t parts = 2 * (size_t)fp_partial_blocks(*P, chunk);
-  if (parts + kResidualSums > kScratchDoubles)
-    return fail(CTR_ERR_ARG, "ctr_residual_noalloc: one view's partial sums exceed the 4 MiB "
-                             "scratch: use ctr_residual");
+  const size_t parts =
+      2 * std::min<size_t>(fp_partial_blocks(*P, chunk), (size_t)kResidualPairs);
   double* s = nullptr;
   if (int rc = scratch_on(P->device, &s)) return rc;
   // every partial slot and every total is written before it is read: nothing to clear

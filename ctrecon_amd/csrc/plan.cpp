@@ -482,22 +482,35 @@ int residual_chunk(const Plan& P) {
   const int views = std::min(P.d.PN, 256);
   // (a chunk of the integral-image method builds the volume's tables again)
   if (P.method == CTR_METHOD_SAT) return views;
-  const long long most = (kResidualScratch - kResidualSums) / 2 / fp_partial_blocks(P, 1);
+  const long long most = kResidualPairs / fp_partial_blocks(P, 1);
   return (int)std::max<long long>(1, std::min<long long>(views, most));
 }
 
 int residual_run(Plan& P, const float* d_x, const float* d_prj, float* prj, int chunk,
                  double* partials, double* sums, hipStream_t st, double* out) {
   const int PN = P.d.PN;
-  const int nch = (PN + chunk - 1) / chunk;
+  // (a view whose partial sums exceed the scratch: in parts of its columns, chunk being 1)
+  const int columns = P.method == CTR_METHOD_DIRECT && fp_partial_blocks(P, 1) > kResidualPairs
+                          ? fp_columns_within(P, kResidualPairs)
+                          : P.d.DNU;
+  const int parts = (P.d.DNU + columns - 1) / columns;
+  const int nch = (PN + chunk - 1) / chunk * parts;
   double h[kResidualSums];
   double rr = 0, bb = 0;
   int rc, pending = 0;
   for (int c = 0; c < nch; ++c) {
-    const int v0 = c * chunk, vc = std::min(chunk, PN - v0);
-    if ((rc = fp_any(P, d_x, prj, v0, 1, vc, st, d_prj, nullptr, partials))) return rc;
-    if ((rc = launch_reduce_pairs(partials, fp_partial_blocks(P, vc), sums + 2 * pending, st)))
-      return rc;
+    int blocks;
+    if (parts > 1) {
+      const int u0 = c % parts * columns, nu = std::min(columns, P.d.DNU - u0);
+      rc = launch_fp_columns(P, d_x, c / parts, u0, nu, st, d_prj, partials);
+      blocks = fp_column_blocks(P, nu);
+    } else {
+      const int v0 = c * chunk, vc = std::min(chunk, PN - v0);
+      rc = fp_any(P, d_x, prj, v0, 1, vc, st, d_prj, nullptr, partials);
+      blocks = fp_partial_blocks(P, vc);
+    }
+    if (rc) return rc;
+    if ((rc = launch_reduce_pairs(partials, blocks, sums + 2 * pending, st))) return rc;
     // the chunks' sums are read back kResidualSums / 2 at a time and added in chunk order
     if (++pending == kResidualSums / 2 || c == nch - 1) {
       CTR_HIP(hipMemcpyAsync(h, sums, 2 * pending * sizeof(double), hipMemcpyDeviceToHost, st));
