@@ -81,6 +81,7 @@ struct ctr_batch {
   // the launch of a windowed class: most row chunks and column sums of its scans (BpShape)
   BpShape win[kClasses] = {};
   bool colw = false;
+  bool fine = false;  // the forward projector's form for fine voxels (Dims): a scan needs it
   // zg: z groups per lane (1..4; 0 and kZgWindow: each scan's own ceil(ZN / 64)) of the scans
   // with columns taller than kWinMaxZ; every other scan runs the windowed form
   int fpGrid = 0, zg = 0, bpGrid = 0;  // grids: persistent workgroups, <= 0 one per item
@@ -197,7 +198,7 @@ int build(ctr_batch& B) { return B.bf ? build_tables<uint16_t>(B) : build_tables
 template <typename T>
 int step_fp(ctr_batch& B, int s) {
   return launch_fp_batch<T>((const FpBatchItem<T>*)B.fpItems.p + (size_t)s * B.n, B.n,
-                            B.fpTotal[s], B.colw, B.fpGrid, B.fpStrided, B.st);
+                            B.fpTotal[s], B.colw, B.fine, B.fpGrid, B.fpStrided, B.st);
 }
 
 template <typename T>
@@ -433,7 +434,7 @@ int ctr_batch_create(ctr_plan* const* plans, int nscan, float* const* d_x,
   CTR_HIP(hipEventCreate(&e0));
   CTR_HIP(hipEventCreate(&e1));
   (void)hipEventRecord(e0, B->st);
-  size_t maxNV = 0;
+  size_t maxNV = 0, minNV = ~(size_t)0;
   for (int i = 0; i < nscan; ++i) {
     auto c = std::make_unique<Scan>();
     Plan& P = *plans[i]->impl;
@@ -443,6 +444,8 @@ int ctr_batch_create(ctr_plan* const* plans, int nscan, float* const* d_x,
     c->NV = (size_t)P.d.XN * P.d.YN * P.d.ZN;
     c->frame = (size_t)P.d.DNU * P.d.DNV;
     maxNV = std::max(maxNV, c->NV);
+    B->fine = B->fine || P.d.fine;
+    minNV = std::min(minNV, c->NV);
     const int maxV = vcount(P, 0, osNum);
     const int upv = std::max(fp_blocks_per_view(P, true), fp_blocks_per_view(P, false));
     if ((rc = c->rowInv.alloc(c->frame * P.d.PN * sizeof(float)))) return rc;
@@ -478,6 +481,7 @@ int ctr_batch_create(ctr_plan* const* plans, int nscan, float* const* d_x,
     CTR_HIP(hipStreamSynchronize(B->st));  // before `ones` is freed
     B->scans.push_back(std::move(c));
   }
+  B->fine = B->fine && minNV >= 4;
   (void)hipEventRecord(e1, B->st);
   CTR_HIP(hipEventSynchronize(e1));
   float ms = 0;

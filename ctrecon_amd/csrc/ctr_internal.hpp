@@ -65,6 +65,8 @@ struct Dims {
   double B0_64, dB_64;   // row boundary 0 and the mean spacing, FP64
   int even_rows;         // 1: every row boundary is B0 + v dB to within the FP32 rounding of
                          // row positions relative to the source
+  int fine;              // 1: some footprint can cover more than four cells in-plane or be more
+                         // than two cells high (fp_body's FINE); not for under four voxels
 };
 
 // Host copies used by host-side accounting (cone voxel counts).
@@ -280,8 +282,8 @@ int fp_lanes_log2(int DNV);
 // batched launches: grid = number of persistent workgroups (<= 0: one per work item),
 // strided = interleaved instead of contiguous item ranges
 template <typename T>
-int launch_fp_batch(const FpBatchItem<T>* items, int nscan, int total, bool colw, int grid,
-                    int strided, hipStream_t st);
+int launch_fp_batch(const FpBatchItem<T>* items, int nscan, int total, bool colw, bool fine,
+                    int grid, int strided, hipStream_t st);
 template <typename T>
 int launch_bp_batch(const BpBatchItem<T>* items, int nscan, int total, int zg, int grid,
                     int strided, hipStream_t st);

@@ -168,6 +168,23 @@ __device__ __forceinline__ void z_run(const Buf<uint16_t>&, const uint16_t* vol,
   }
 }
 
+// Four z taps from element e of a volume of n (at least four) elements on; past its end 0.
+__device__ __forceinline__ void z_run4(const Buf<float>& V, const float*, int e, int,
+                                       float (&a)[4]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) a[i] = V[e + i];
+}
+__device__ __forceinline__ void z_run4(const Buf<uint16_t>&, const uint16_t* vol, int e, int n,
+                                       float (&a)[4]) {
+  const int b = min(e, n - 4);
+  const uint64_t q = *(const CTR_GLOBAL u64a2*)((const CTR_GLOBAL char*)vol + (uint32_t)b * 2u) >>
+                     (16 * (e - b));
+  a[0] = __uint_as_float((uint32_t)q << 16);
+  a[1] = __uint_as_float((uint32_t)q & 0xffff0000u);
+  a[2] = __uint_as_float((uint32_t)(q >> 32) << 16);
+  a[3] = __uint_as_float((uint32_t)(q >> 32) & 0xffff0000u);
+}
+
 // Work mapping.  A wave's lanes are 64 / L groups of L = 2^lg lanes (lg = A.lg, 3 .. 6);
 // group g takes item g of the wave, an item being L consecutive detector rows of one
 // (view, column).  COLW: lg = 6, one column per wave, so that everything in-plane is
@@ -194,12 +211,22 @@ __device__ __forceinline__ void z_run(const Buf<uint16_t>&, const uint16_t* vol,
 // 64^3, 720 views of 256 x 16, 212 us one thread per ray with its own FP64 footprints,
 // 88 us with four columns per wave.
 //
+// FINE (Dims::fine, fine voxels or wide detector columns): slices of more than four cells take
+// one pass per four, and those whose rows are more than two cells high four taps to a load,
+// all in the classes' loops over the LDS table.  Without it such slices are rare and take the
+// general form, which evaluates a footprint in every lane; a slice that both forms take rounds
+// the same, so that a batch may run FINE for all of its scans.  128^2 x 64, 100 views of 400 or
+// 888 columns, general form and FINE: 0.3 mm voxels, 64 rows 344 us, 125 us; 0.1 mm slices, 16
+// rows 318 us, 124 us; 64^2 x 64 of 0.1 mm, 64 rows 163 us, 65 us; 4 mm columns, 16 rows 205 us,
+// 83 us.  FINE keeps 5 to 25 more registers (five to eight waves per SIMD) and is slower where
+// no slice needs it.
+//
 // ONES: the projection of a volume of ones (the row sums of OS-SART), read from no volume.
 // A slice wholly inside the volume's z range adds its height times its cells' weights; the
 // others take the weights of the projection itself, so that a ray that grazes the volume by
 // a rounding error has a row sum that matches its projection (no contraction: the
 // instantiations must not round a footprint differently).
-template <bool FUSED, bool COLW, typename TV, typename TO, bool ONES = false>
+template <bool FUSED, bool COLW, typename TV, typename TO, bool FINE, bool ONES = false>
 __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk, double* slot) {
 #pragma clang fp contract(off)
   const Dims& d = A.d;
@@ -253,19 +280,52 @@ __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk
       if (!(t < te)) return;
       const int k0 = min((int)floorf(t), kmax);
       const int nk = min((int)ceilf(te) - 1, kmax) - k0 + 1;
-      const float wf = fminf(te, (float)(k0 + 1)) - t, wl = te - (float)(k0 + nk - 1);
       int e = ii * sS + o.j0 * cS + vp.azi + k0, mo = ii * mS + o.j0 * mC;
-      float s = 0.f;
       for (int ij = 0; ij < o.nj; ++ij) {
-        const float wy = ((ij == 0) ? o.wj0 : (ij == o.nj - 1 ? o.wjl : 1.f)) * maskf[mo];
+        const float wy =
+            o.inv * (((ij == 0) ? o.wj0 : (ij == o.nj - 1 ? o.wjl : 1.f)) * maskf[mo]);
         float g = 0.f;
-        for (int ik = 0; ik < nk; ++ik)
-          g = fmaf((ik == 0) ? wf : (ik == nk - 1 ? wl : 1.f), ONES ? 1.f : (float)V[e + ik], g);
-        s = fmaf(wy, g, s);
+        if constexpr (ONES) g = te - t;
+        else
+          for (int ik = 0; ik < nk; ++ik)
+            g = fmaf(fminf(te, (float)(k0 + ik + 1)) - fmaxf(t, (float)(k0 + ik)),
+                     (float)V[e + ik], g);
+        acc = fmaf(wy, g, acc);
         e += cS;
         mo += mC;
       }
-      acc = fmaf(s, o.inv, acc);
+    };
+    // FINE: the same for all lanes of a slice of up to NJ cells (r, wy, nc cells from element e, z
+    // index azi, on; a cell past a group's own re-reads its last with weight 0), four taps of a
+    // cell to a load (taps past the lane's own have weight 0, past the array's end they are 0)
+    auto tall = [&](auto NJ_, float r, const float(&wy)[4], int e, int nc) {
+      constexpr int NJ = decltype(NJ_)::value;
+      const float t = fmaxf(fmaf(r, Bv, azf), tmin), te = fminf(fmaf(r, Bv1, azf), tmax);
+      if (!(vok && t < te)) return;
+      if constexpr (ONES) {
+#pragma unroll
+        for (int c = 0; c < NJ; ++c) acc = fmaf(wy[c], te - t, acc);
+        return;
+      }
+      const int k0 = min((int)floorf(t), kmax);
+      float g[NJ] = {};
+      for (int k = k0; (float)k < te; k += 4) {
+        float w[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float z = (float)(k + i);
+          w[i] = fmaxf(fminf(te, z + 1.f) - fmaxf(t, z), 0.f);
+        }
+#pragma unroll
+        for (int c = 0; c < NJ; ++c) {
+          float a[4];
+          z_run4(V, A.vol, e + k + min(c, nc - 1) * cS, NV, a);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) g[c] = fmaf(w[i], a[i], g[c]);
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < NJ; ++c) acc = fmaf(wy[c], g[c], acc);
     };
     // per wave: (r, wy0, wy1, wy2) of each slice, and for groups (element, cells, wy3)
     __shared__ float4 s_rec[kWaves * 64];
@@ -275,12 +335,13 @@ __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk
     int4* off = s_off + (COLW ? 0 : wid * 64);
     float* zrun = s_run + (COLW ? wid * 128 : 0);
     const int gbase = lane & ~(L - 1);  // first record of the lane's group
-    for (int ii0 = 0; ii0 < NS; ii0 += L) {
+    // FINE: slices of more than four cells are evaluated again from the next four cells (c0) on
+    for (int ii0 = 0, c0 = 0, next; ii0 < NS; ii0 = next) {
       const int il = ii0 + li;
       float q_r = 0.f, wy0 = 0.f, wy1 = 0.f, wy2 = 0.f, wy3 = 0.f;
       int q_e = 0, q_nj = 0, q_kb = 0, q_last = 0;
       // bits of cls: 1 a third z tap, 2 more than 64 cells of z (COLW), 4 reaches past the
-      // volume's ends, 8 the general form
+      // volume's ends, 8 the general form, 16 more cells
       int cls = 0;
       SliceIP o;
       // clipped to the mask's extent on the slice (inside [-0.5, NI - 0.5]): cells
@@ -288,35 +349,40 @@ __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk
       if (il < NS && uok && fp_inplane(bl, br, ct, gload(me, il), il, NI, o)) {
         // z range of the item's rows; r > 0 beyond the source
         const float tl = fmaf(o.r, Blo, azf), th = fmaf(o.r, Bhi, azf);
-        if (o.r > 0.f && th > tmin && tl < tmax) {
+        const int n = FINE ? o.nj - c0 : o.nj;  // cells from c0 on
+        if (o.r > 0.f && th > tmin && tl < tmax && (!FINE || n > 0)) {
           q_r = o.r;
-          q_nj = o.nj;
+          q_nj = FINE ? min(n, 4) : n;
           const float h = o.r * d.dBmax;
-          const int mo = il * mS + o.j0 * mC;
-          wy0 = o.inv * (o.wj0 * maskf[mo]);
-          if (o.nj >= 2) wy1 = o.inv * ((o.nj == 2 ? o.wjl : 1.f) * maskf[mo + mC]);
-          if (o.nj >= 3) wy2 = o.inv * ((o.nj == 3 ? o.wjl : 1.f) * maskf[mo + 2 * mC]);
-          if (o.nj >= 4) wy3 = o.inv * (o.wjl * maskf[mo + 3 * mC]);
-          const int e = il * sS + o.j0 * cS;
+          const int j0 = FINE ? o.j0 + c0 : o.j0, mo = il * mS + j0 * mC;
+          wy0 = o.inv * ((!FINE || c0 == 0 ? o.wj0 : (n == 1 ? o.wjl : 1.f)) * maskf[mo]);
+          if (n >= 2) wy1 = o.inv * ((n == 2 ? o.wjl : 1.f) * maskf[mo + mC]);
+          if (n >= 3) wy2 = o.inv * ((n == 3 ? o.wjl : 1.f) * maskf[mo + 2 * mC]);
+          if (n >= 4) wy3 = o.inv * ((!FINE || n == 4 ? o.wjl : 1.f) * maskf[mo + 3 * mC]);
+          const int e = il * sS + j0 * cS;
           q_e = e + vp.azi;
-          bool gen = o.nj > 4 || h > 2.f;
+          bool gen = (!FINE && n > 4) || h > 2.f;
           cls = (h > 1.f ? 1 : 0) | (tl < tmin + 0.01f || th > tmax - 0.01f ? 4 : 0);
+          if (FINE && n > 4) cls |= 16;
           if constexpr (COLW) {
             // the z run of the item: cells from the first row's on, read up to the last
             // row's third tap; its 64 or 128 elements stay inside the array
             q_kb = floor_i(tl);
-            q_e += q_kb;
+            if constexpr (!FINE) q_e += q_kb;
             q_last = floor_i(fmaf(o.r, Btop, azf)) - q_kb + 2;
             if (q_last > 63) cls |= 2;
-            gen = gen || q_last > 127 || q_e + (max(o.nj, 2) - 1) * cS + 128 > NV;
+            gen = gen || q_last > 127 ||
+                  q_e + (FINE ? q_kb : 0) + (max(q_nj, 2) - 1) * cS + 128 > NV;
+            if (FINE && !gen) q_e += q_kb;
           } else {
             // a run's elements stay inside the array: not on its last column
-            gen = gen || e + (o.nj - 1) * cS + d.ZN + 4 > NV;
+            gen = gen || e + (q_nj - 1) * cS + d.ZN + 4 > NV;
           }
           cls |= gen ? 8 : 0;
         }
       }
       rec[lane] = make_float4(q_r, wy0, wy1, wy2);
+      next = ii0 + L;
       int mj = q_nj;  // most cells of the slice over the wave's groups
       if constexpr (!COLW) {
         off[lane] = make_int4(q_e, q_nj, __float_as_int(wy3), 0);
@@ -324,6 +390,12 @@ __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk
           cls |= __shfl_xor(cls, x, 64);
           mj = max(mj, __shfl_xor(mj, x, 64));
         }
+      }
+      if constexpr (FINE) {
+        const bool more = __any(cls & 16);
+        cls &= 15;
+        next = more ? ii0 : ii0 + L;
+        c0 = more ? c0 + 4 : 0;
       }
       if (!__any(mj)) continue;
       // the class as a number: cells (one counts as two, the second of weight 0: the two are mixed
@@ -484,12 +556,29 @@ __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk
         run(I4{}, I3{}, F{}, 1);
         run(I4{}, I3{}, T{}, 3);
       }
-      uint64_t m = __ballot(key == 7) & low;
-      while (m) {
-        const int j = __builtin_ctzll(m);
-        m &= m - 1;
-        general(ii0 + j);
+      auto generals = [&](auto NJ_) {
+        constexpr int NJ = decltype(NJ_)::value;
+        uint64_t m = __ballot(key == 7 && (!FINE || mj == NJ)) & low;
+        while (m) {
+          const int j = __builtin_ctzll(m);
+          m &= m - 1;
+          if constexpr (!FINE) {
+            general(ii0 + j);
+          } else {
+            const float4 q = rec[gbase + j];
+            const int4 f = off[COLW ? 0 : gbase + j];
+            const float wy[4] = {q.y, q.z, q.w, COLW ? rdl(wy3, j) : __int_as_float(f.z)};
+            tall(NJ_, q.x, wy, COLW ? __builtin_amdgcn_readlane(q_e, j) : f.x,
+                 COLW ? __builtin_amdgcn_readlane(q_nj, j) : f.y);
+          }
+        }
+      };
+      if constexpr (FINE) {
+        generals(integral_constant<int, 1>{});
+        generals(I2{});
+        generals(I3{});
       }
+      generals(I4{});
     }
     if constexpr (!ONES) {
       if (__builtin_expect(__any(vok && not_finite(acc)), 0)) {
@@ -516,23 +605,23 @@ __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk
   if constexpr (FUSED) block_sum2(res, bsq, slot);
 }
 
-template <bool FUSED, bool COLW, typename TV, typename TO>
+template <bool FUSED, bool COLW, typename TV, typename TO, bool FINE>
 __global__ __launch_bounds__(kBlock) void fp_kernel(FpArgs<TV, TO> A, int bpv, int views) {
   const int hw = blockIdx.x;
   const int lb = xcd_chunked_block(hw);
   const int k = lb / bpv;
   if (k >= views) return;
-  fp_body<FUSED, COLW, TV, TO>(A, k, lb - k * bpv, A.partials + 2 * lb);
+  fp_body<FUSED, COLW, TV, TO, FINE>(A, k, lb - k * bpv, A.partials + 2 * lb);
 }
 
 // Forward projection of a volume of ones (A.vol unused).
-template <bool COLW>
+template <bool COLW, bool FINE>
 __global__ __launch_bounds__(kBlock) void fp_ones_kernel(FpArgs<float, float> A, int bpv,
                                                          int views) {
   const int lb = xcd_chunked_block(blockIdx.x);
   const int k = lb / bpv;
   if (k >= views) return;
-  fp_body<false, COLW, float, float, true>(A, k, lb - k * bpv, nullptr);
+  fp_body<false, COLW, float, float, FINE, true>(A, k, lb - k * bpv, nullptr);
 }
 
 // Batched persistent forward projection: each workgroup takes one contiguous range of
@@ -574,7 +663,7 @@ __device__ __forceinline__ void batch_range(const Item* __restrict__ D, int nsca
   }
 }
 
-template <bool FUSED, bool COLW, typename T>
+template <bool FUSED, bool COLW, typename T, bool FINE>
 __global__ __launch_bounds__(kBlock) void fp_batch_kernel(const FpBatchItem<T>* __restrict__ D,
                                                           int nscan, int total, int sched) {
   int i0, step, i1;
@@ -586,13 +675,13 @@ __global__ __launch_bounds__(kBlock) void fp_batch_kernel(const FpBatchItem<T>* 
     const FpBatchItem<T>& B = D[s];
     const int local = item - B.begin;
     const int k = local / B.upv;
-    fp_body<FUSED, COLW, T, T>(B.a, k, local - k * B.upv, B.a.partials + 2 * local);
+    fp_body<FUSED, COLW, T, T, FINE>(B.a, k, local - k * B.upv, B.a.partials + 2 * local);
   }
 }
 
 
 // fp_batch_kernel for the one-workgroup-per-item schedule (grid = total): no item loop.
-template <bool FUSED, bool COLW, typename T>
+template <bool FUSED, bool COLW, typename T, bool FINE>
 __global__ __launch_bounds__(kBlock) void fp_batch1_kernel(const FpBatchItem<T>* __restrict__ D,
                                                            int nscan, int total) {
   int i0, step, i1;
@@ -602,7 +691,7 @@ __global__ __launch_bounds__(kBlock) void fp_batch1_kernel(const FpBatchItem<T>*
   const FpBatchItem<T>& B = D[s];
   const int local = i0 - B.begin;
   const int k = local / B.upv;
-  fp_body<FUSED, COLW, T, T>(B.a, k, local - k * B.upv, B.a.partials + 2 * local);
+  fp_body<FUSED, COLW, T, T, FINE>(B.a, k, local - k * B.upv, B.a.partials + 2 * local);
 }
 
 // ---------------------------------------------------------------------------
@@ -2730,6 +2819,18 @@ int fp_blocks_per_view(const Plan& P, bool colw) {
   return fp_blocks_of(P, colw ? 6 : fp_lanes_log2(P.d.DNV));
 }
 
+// f(one column per wave, FINE) with a launch's choices as integral constants.
+template <typename F>
+static void fp_variant(const Plan& P, F f) {
+  using Y = std::true_type;
+  using N = std::false_type;
+  const bool colw = fp_lanes_log2(P.d.DNV) == 6;
+  if (colw && P.d.fine) f(Y{}, Y{});
+  else if (colw) f(Y{}, N{});
+  else if (P.d.fine) f(N{}, Y{});
+  else f(N{}, N{});
+}
+
 template <typename TV, typename TO>
 int launch_fp(const Plan& P, const TV* vol, TO* out, int vb, int vs, int vc, hipStream_t st,
               const float* b, const float* invRow, double* partials) {
@@ -2737,17 +2838,13 @@ int launch_fp(const Plan& P, const TV* vol, TO* out, int vb, int vs, int vc, hip
   const FpArgs<TV, TO> A = fp_args<TV, TO>(P, vol, out, vb, vs, b, invRow, partials);
   const int bpv = fp_blocks_of(P, A.lg);
   const dim3 grid(xcd_chunked_grid((long long)bpv * vc));
-  const bool colw = A.lg == 6;
-#define CTR_FP(FUSED, COLW)                                                                   \
-  hipLaunchKernelGGL((fp_kernel<FUSED, COLW, TV, TO>), grid, dim3(kBlock), 0, st, A, bpv, vc)
-  if (b) {
-    if (colw) CTR_FP(true, true);
-    else CTR_FP(true, false);
-  } else {
-    if (colw) CTR_FP(false, true);
-    else CTR_FP(false, false);
-  }
-#undef CTR_FP
+  fp_variant(P, [&](auto C, auto F) {
+    constexpr bool c = decltype(C)::value, f = decltype(F)::value;
+    if (b)
+      hipLaunchKernelGGL((fp_kernel<true, c, TV, TO, f>), grid, dim3(kBlock), 0, st, A, bpv, vc);
+    else
+      hipLaunchKernelGGL((fp_kernel<false, c, TV, TO, f>), grid, dim3(kBlock), 0, st, A, bpv, vc);
+  });
   return check_launch("fp_kernel");
 }
 
@@ -2764,11 +2861,10 @@ int launch_fp_columns(const Plan& P, const float* vol, int p, int u0, int column
   A.d.DNU = columns;
   const int bpv = fp_blocks_of(P, A.lg, columns);
   const dim3 grid(xcd_chunked_grid(bpv));
-  if (A.lg == 6)
-    hipLaunchKernelGGL((fp_kernel<true, true, float, float>), grid, dim3(kBlock), 0, st, A, bpv, 1);
-  else
-    hipLaunchKernelGGL((fp_kernel<true, false, float, float>), grid, dim3(kBlock), 0, st, A, bpv,
-                       1);
+  fp_variant(P, [&](auto C, auto F) {
+    hipLaunchKernelGGL((fp_kernel<true, decltype(C)::value, float, float, decltype(F)::value>),
+                       grid, dim3(kBlock), 0, st, A, bpv, 1);
+  });
   return check_launch("fp_kernel");
 }
 
@@ -2778,10 +2874,10 @@ int launch_fp_ones(const Plan& P, float* out, int vb, int vs, int vc, hipStream_
       fp_args<float, float>(P, nullptr, out, vb, vs, nullptr, nullptr, nullptr);
   const int bpv = fp_blocks_of(P, A.lg);
   const dim3 grid(xcd_chunked_grid((long long)bpv * vc));
-  if (A.lg == 6)
-    hipLaunchKernelGGL((fp_ones_kernel<true>), grid, dim3(kBlock), 0, st, A, bpv, vc);
-  else
-    hipLaunchKernelGGL((fp_ones_kernel<false>), grid, dim3(kBlock), 0, st, A, bpv, vc);
+  fp_variant(P, [&](auto C, auto F) {
+    hipLaunchKernelGGL((fp_ones_kernel<decltype(C)::value, decltype(F)::value>), grid,
+                       dim3(kBlock), 0, st, A, bpv, vc);
+  });
   return check_launch("fp_ones_kernel");
 }
 
@@ -2957,23 +3053,26 @@ int launch_bp(const Plan& P, const T* prj, float* vol, int vb, int vs, int vc, i
 
 // grid <= 0: one workgroup per item (hardware scheduling, per-scan XCD map)
 template <typename T>
-int launch_fp_batch(const FpBatchItem<T>* items, int nscan, int total, bool colw, int grid,
-                    int strided, hipStream_t st) {
+int launch_fp_batch(const FpBatchItem<T>* items, int nscan, int total, bool colw, bool fine,
+                    int grid, int strided, hipStream_t st) {
   if (total <= 0) return CTR_OK;
   const int sched = grid <= 0 ? 2 : (strided ? 1 : 0);
   grid = grid <= 0 ? total : std::max(1, std::min(grid, total));
-  if (sched == 2 && colw)
-    hipLaunchKernelGGL((fp_batch1_kernel<true, true, T>), dim3(grid), dim3(kBlock), 0, st,
-                       items, nscan, total);
-  else if (sched == 2)
-    hipLaunchKernelGGL((fp_batch1_kernel<true, false, T>), dim3(grid), dim3(kBlock), 0, st,
-                       items, nscan, total);
-  else if (colw)
-    hipLaunchKernelGGL((fp_batch_kernel<true, true, T>), dim3(grid), dim3(kBlock), 0, st, items,
-                       nscan, total, sched);
-  else
-    hipLaunchKernelGGL((fp_batch_kernel<true, false, T>), dim3(grid), dim3(kBlock), 0, st, items,
-                       nscan, total, sched);
+  auto launch = [&](auto C, auto F) {
+    constexpr bool c = decltype(C)::value, f = decltype(F)::value;
+    if (sched == 2)
+      hipLaunchKernelGGL((fp_batch1_kernel<true, c, T, f>), dim3(grid), dim3(kBlock), 0, st,
+                         items, nscan, total);
+    else
+      hipLaunchKernelGGL((fp_batch_kernel<true, c, T, f>), dim3(grid), dim3(kBlock), 0, st, items,
+                         nscan, total, sched);
+  };
+  using Y = std::true_type;
+  using N = std::false_type;
+  if (colw && fine) launch(Y{}, Y{});
+  else if (colw) launch(Y{}, N{});
+  else if (fine) launch(N{}, Y{});
+  else launch(N{}, N{});
   return check_launch("fp_batch_kernel");
 }
 
@@ -3060,9 +3159,9 @@ template BpArgs<float> bp_args<float>(const Plan&, const float*, float*, int, in
                                       const float*, uint16_t*);
 template BpArgs<uint16_t> bp_args<uint16_t>(const Plan&, const uint16_t*, float*, int, int, int,
                                             const float*, uint16_t*);
-template int launch_fp_batch<float>(const FpBatchItem<float>*, int, int, bool, int, int,
+template int launch_fp_batch<float>(const FpBatchItem<float>*, int, int, bool, bool, int, int,
                                     hipStream_t);
-template int launch_fp_batch<uint16_t>(const FpBatchItem<uint16_t>*, int, int, bool, int, int,
+template int launch_fp_batch<uint16_t>(const FpBatchItem<uint16_t>*, int, int, bool, bool, int, int,
                                        hipStream_t);
 template int launch_bp_batch<float>(const BpBatchItem<float>*, int, int, int, int, int,
                                     hipStream_t);

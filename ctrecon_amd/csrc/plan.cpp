@@ -211,6 +211,12 @@ static int build_tables(const ctr_geometry* g, Plan& P, double half = 0.0) {
     const double minBeta = std::asin(dirx * ly - diry * lx);
     const double cU = -minBeta / dbeta - 0.5;
     const double S2D = std::hypot((double)g->xds[0] - x0, (double)g->yds[0] - y0);
+    // footprints at the grid's far side: rows of more than two cells of z, or columns (seen at
+    // 45 degrees) that can cover more than four cells, being over three wide
+    const double far = 1.0 + 0.5 * std::max(g->XN, g->YN) * dx / sid;
+    const bool fine = d.dBmax * (sid / S2D) * far > 2.0 ||
+                      std::fabs(dbeta) * sid / dx * std::sqrt(2.0) * far > 3.0;
+    d.fine = fine && (long long)g->XN * g->YN * g->ZN >= 4 ? 1 : 0;
     P.bc.S = (float)(S2D / ddv);
     P.bc.ib = (float)(1.0 / dbeta);
     P.bc.hz = (float)(dz * 0.5);
