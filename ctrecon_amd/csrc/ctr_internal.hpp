@@ -60,6 +60,7 @@ struct Dims {
   float dx, dz;
   float beta0, dbeta_g;  // fan angle of boundary 0 and mean boundary spacing (adjoint guess)
   float B0, dB;          // row boundary index of row 0 and mean spacing (adjoint guess)
+  float idz;             // 1 / dz
   float dBmin;           // smallest row spacing of the FP32 boundary table
   float dBmax;           // largest row height (bz_(v+1) - bz_v)/dz
   double B0_64, dB_64;   // row boundary 0 and the mean spacing, FP64

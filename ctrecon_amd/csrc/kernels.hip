@@ -26,6 +26,22 @@ __device__ __forceinline__ float rdl(float v, int lane) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
+// A wave-uniform value in scalar registers that the compiler takes for a new one: what is computed
+// or loaded from it in a loop is not hoisted out of the loop into registers.
+template <typename V>
+__device__ __forceinline__ V held(V v) {
+  constexpr int N = sizeof(V) / 4;
+  uint32_t w[N];
+  __builtin_memcpy(w, &v, sizeof(V));
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    w[i] = __builtin_amdgcn_readfirstlane(w[i]);
+    asm volatile("" : "+s"(w[i]));
+  }
+  __builtin_memcpy(&v, w, sizeof(V));
+  return v;
+}
+
 // Block-wide sum of two doubles into slot[0], slot[1].
 __device__ __forceinline__ void block_sum2(double a, double b, double* slot) {
   __shared__ double red[2][kWaves];
@@ -719,24 +735,29 @@ struct BpView {
 };
 
 template <typename T>
-__device__ __forceinline__ BpView bp_view(const BpArgs<T>& A, int p, double Px, double Py,
-                                          float Pxf, float Pyf) {
+__device__ __forceinline__ BpView bp_view(const BpArgs<T>& A, int p, double Px_, double Py_) {
   const Dims& d = A.d;
   const BpConsts& c = A.c;
-  const BpConsts64& c64 = A.c64;
+  // (constants in scalar registers: hoisted out of a wave's loop over its views they would stand
+  // in vector registers, which spilled)
+  BpConsts64 c64 = A.c64;
+  c64.inv_sid = held(c64.inv_sid);
+  c64.dx = held(c64.dx);
+  c64.ib = held(c64.ib);
+  c64.cU = held(c64.cU);
+  c64.S = held(c64.S);
+  const double Px = held(Px_), Py = held(Py_);
   BpView r{};
   const ViewP vp = gload(A.views, p);
-  // row shadow, FP32 (DD3_GPU.cu:1446-1450): t = (dZ +- hz) * S / l + cV
-  const float dXf = Pxf - vp.sx, dYf = Pyf - vp.sy;
-  const float l2f = dXf * dXf + dYf * dYf;
-  const float rlS = __builtin_amdgcn_rsqf(l2f) * c.S;
-  const bool rneg = rlS < 0.f;  // rows then run backwards: swap the bounds
   // fan-angle shadow, FP64 (DD3_GPU.cu:1447-1464); sy*dX - sx*dY == sy*Px - sx*Py
   const double2 s64 = gload(A.src64, p);
   const double dX = Px - s64.x, dY = Py - s64.y;
   const double l2 = dX * dX + dY * dY;
   const double rl = rsqrt(l2);
   r.rl = rl;
+  // row shadow (DD3_GPU.cu:1446-1450): t = (dZ +- hz) * S / l + cV
+  const float rlS = (float)(rl * c64.S);
+  const bool rneg = rlS < 0.f;  // rows then run backwards: swap the bounds
   const double alpha = asin_fan((s64.y * Px - s64.x * Py) * c64.inv_sid * rl);
   const double w = vp.wx ? dX : dY;
   const double dA = w * (rl * rl) * (c64.dx * 0.5);
@@ -764,7 +785,7 @@ __device__ __forceinline__ BpView bp_view(const BpArgs<T>& A, int p, double Px, 
   r.cB = rneg ? cDp : cUp;  // upper row bound
   r.rlS = rlS;
   r.sz = vp.sz;
-  r.l2 = l2f;
+  r.l2 = (float)l2;
   return r;
 }
 
@@ -806,10 +827,10 @@ __device__ __forceinline__ float bp_cells(const Buf<T>& pp, int o, int DNV, int 
   return s;
 }
 
-// The voxel's shadow [vlo, vhi] (rows) x cells u0 .. u0 + nu - 1 integrated over the
+// The voxel's shadow [vlo, vhi] (rows) x nu columns from offset o0 on integrated over the
 // piecewise-constant view pp (first / last column weights wu0, fh).
 template <typename T>
-__device__ __forceinline__ float bp_cell_sum(const Buf<T>& pp, int u0, int nu, float wu0,
+__device__ __forceinline__ float bp_cell_sum(const Buf<T>& pp, int o0, int nu, float wu0,
                                              float fh, float vlo, float vhi, int DNV) {
 #pragma clang fp contract(off)
   // first row v0 = floor(vlo + .5) and its upper edge e; with d = vhi - e the overlaps of
@@ -826,7 +847,7 @@ __device__ __forceinline__ float bp_cell_sum(const Buf<T>& pp, int u0, int nu, f
     const float wv2 = __builtin_amdgcn_fmed3f(d - 1.f, 0.f, 1.f);
     // taps of zero weight re-read the first row (never a row outside the shadow)
     const int t1 = d > 0.f ? 1 : 0, t2 = d > 1.f ? 2 : 0;
-    const int o = u0 * DNV + v0;
+    const int o = o0 + v0;
     if (!__any(d > 1.f)) {  // at most two rows in every lane's shadow
       switch (nu) {  // uniform over the wave
         case 1: s = bp_cells<1, 2>(pp, o, DNV, t1, t2, wv0, wv1, wv2, wu0, fh); break;
@@ -848,7 +869,7 @@ __device__ __forceinline__ float bp_cell_sum(const Buf<T>& pp, int u0, int nu, f
     edge_weights(vlo, vhi, v0, nv, wv0, wvl);
     for (int iv = 0; iv < nv; ++iv) {
       const float wv = (iv == 0) ? wv0 : (iv == nv - 1 ? wvl : 1.f);
-      const int o = u0 * DNV + v0 + iv;
+      const int o = o0 + v0 + iv;
       float R = wu0 * pp[o];
       for (int iu = 1; iu < nu; ++iu) R = fmaf((iu == nu - 1) ? fh : 1.f, pp[o + iu * DNV], R);
       s = fmaf(wv, R, s);
@@ -890,9 +911,8 @@ __device__ __forceinline__ void bp_ref_body(const BpArgs<T>& A, int col, int zbl
     }
     return;
   }
-  const double Px = ((double)x - c64.ocx) * c64.dx;
-  const double Py = ((double)y - c64.ocy) * c64.dx;
-  const float Pxf = (float)Px, Pyf = (float)Py;
+  const double Px = held(((double)x - c64.ocx) * c64.dx);
+  const double Py = held(((double)y - c64.ocy) * c64.dx);
   // z extent of the wave's voxel centres (uniform), for the whole-column view test
   const float Zlo = ((float)zb0 - d.ocz) * d.dz;
   const float Zhi = ((float)min(zb0 + 64 * ZG, d.ZN) - 1.f - d.ocz) * d.dz;
@@ -911,7 +931,7 @@ __device__ __forceinline__ void bp_ref_body(const BpArgs<T>& A, int col, int zbl
     BpView q{};
     bool vis = false;
     if (kl < A.vc) {
-      q = bp_view(A, A.vb + kl * A.vs, Px, Py, Pxf, Pyf);
+      q = bp_view(A, A.vb + kl * A.vs, Px, Py);
       // the whole group range of rows, to skip views the wave's voxels do not meet
       const float ta = fmaf(Zlo - q.sz, q.rlS, q.cA), tb = fmaf(Zhi - q.sz, q.rlS, q.cB);
       vis = q.uvis && fmaxf(ta, tb) > -0.5f && fminf(ta, tb) < DNVh;
@@ -937,7 +957,7 @@ __device__ __forceinline__ void bp_ref_body(const BpArgs<T>& A, int col, int zbl
         if (!__any(vok)) continue;
         if (!vok) continue;
         const float cosVal = cws * __builtin_amdgcn_sqrtf(fmaf(dZ, dZ, l2f));
-        acc[g] = fmaf(cosVal, bp_cell_sum(pp, u0, nu, wu0, fh, vlo, vhi, DNV), acc[g]);
+        acc[g] = fmaf(cosVal, bp_cell_sum(pp, u0 * DNV, nu, wu0, fh, vlo, vhi, DNV), acc[g]);
       }
     }
   }
@@ -953,10 +973,11 @@ __device__ __forceinline__ void bp_ref_body(const BpArgs<T>& A, int col, int zbl
 // voxel indices whose FP32 ends are within ~1e-4 of it, so the integers inside it widened
 // by 1e-2 include every one of them.
 __device__ __forceinline__ void bp_window(const Dims& d, const BpView& q, int& z0, int& z1) {
-  const float DNVh = (float)d.DNV - 0.5f, ZNf = (float)d.ZN, idz = 1.f / d.dz;
+  const float DNVh = (float)held(d.DNV) - 0.5f, ZNf = (float)held(d.ZN), idz = held(d.idz);
+  const float ocz = held(d.ocz);
   const float ea = (-0.5f - q.cB) / q.rlS, eb = (DNVh - q.cA) / q.rlS;
-  const float za = fminf(fmaxf((fminf(ea, eb) + q.sz) * idz + d.ocz, -4.f), ZNf + 4.f);
-  const float zb = fminf(fmaxf((fmaxf(ea, eb) + q.sz) * idz + d.ocz, -4.f), ZNf + 4.f);
+  const float za = fminf(fmaxf((fminf(ea, eb) + q.sz) * idz + ocz, -4.f), ZNf + 4.f);
+  const float zb = fminf(fmaxf((fmaxf(ea, eb) + q.sz) * idz + ocz, -4.f), ZNf + 4.f);
   z0 = max((int)floorf(za - 1e-2f) + 1, 0);
   z1 = min((int)ceilf(zb + 1e-2f) - 1, d.ZN - 1);
 }
@@ -1056,13 +1077,16 @@ struct BpRecord {
 };
 template <typename T>
 __device__ __forceinline__ BpRecord bp_record(const BpArgs<T>& A, int kl, double Px, double Py,
-                                              float Pxf, float Pyf, int lanes, bool exact) {
+                                              int lanes, bool exact) {
 #pragma clang fp contract(off)
   const Dims& d = A.d;
-  const BpConsts64& c64 = A.c64;
+  BpConsts64 c64 = A.c64;
+  c64.S = held(c64.S);
+  c64.cV = held(c64.cV);
+  c64.ocz = held(c64.ocz);
   BpRecord v{};
   v.z1 = -1;
-  const BpView q = bp_view(A, A.vb + kl * A.vs, Px, Py, Pxf, Pyf);
+  const BpView q = bp_view(A, A.vb + kl * A.vs, Px, Py);
   bp_window(d, q, v.z0, v.z1);
   if (q.uvis && v.z0 <= v.z1) {
     // row shadow of the window's first voxel and its step, dZ of that voxel
@@ -1193,16 +1217,15 @@ __device__ __forceinline__ void bp_staged_body(const BpArgs<T>& A, int col, floa
   const int DNV = d.DNV;
   int row[RC], slot[RC];
   stage_rows<RC>(rows, DNV, lane, row, slot);
-  const double Px = ((double)x - c64.ocx) * c64.dx;
-  const double Py = ((double)y - c64.ocy) * c64.dx;
-  const float Pxf = (float)Px, Pyf = (float)Py;
+  const double Px = held(((double)x - c64.ocx) * c64.dx);
+  const double Py = held(((double)y - c64.ocy) * c64.dx);
   const int frame = d.DNU * DNV;
   const float lanef = (float)lane;
   bool rest = false;
   for (int k0 = 0; k0 < A.vc; k0 += 64) {
     const int kl = k0 + lane;
     BpRecord v{};
-    if (kl < A.vc) v = bp_record(A, kl, Px, Py, Pxf, Pyf, 64, false);
+    if (kl < A.vc) v = bp_record(A, kl, Px, Py, 64, false);
     const int z0 = v.z0, z1 = v.z1, q_o = lane * frame + v.o, key = v.key;
     if (!__any(key)) continue;
     rest = rest || __any(key == 1);
@@ -1263,7 +1286,7 @@ __device__ __forceinline__ void bp_staged_body(const BpArgs<T>& A, int col, floa
     for (int k0 = 0; k0 < A.vc; k0 += 64) {
       const int kl = k0 + lane;
       BpRecord v{};
-      if (kl < A.vc) v = bp_record(A, kl, Px, Py, Pxf, Pyf, 64, exact);
+      if (kl < A.vc) v = bp_record(A, kl, Px, Py, 64, exact);
       const uint64_t m = __ballot(v.key == 1);
       if (!m) continue;
       rec[2 * lane] = v.r;
@@ -1393,9 +1416,8 @@ __device__ __forceinline__ void bp_packed_body(const BpArgs<T>& A, int col, floa
   g.zero_pads(lds, DNV);
   float* rows = lds + g.rows;
   float* gacc = lacc + g.sums;
-  const double Px = ((double)x - c64.ocx) * c64.dx;
-  const double Py = ((double)y - c64.ocy) * c64.dx;
-  const float Pxf = (float)Px, Pyf = (float)Py;
+  const double Px = held(((double)x - c64.ocx) * c64.dx);
+  const double Py = held(((double)y - c64.ocy) * c64.dx);
   const int frame = d.DNU * DNV;
   const float glf = (float)g.gl;
   bool rest = false;
@@ -1407,7 +1429,7 @@ __device__ __forceinline__ void bp_packed_body(const BpArgs<T>& A, int col, floa
   for (int k0 = 0; k0 < A.vc; k0 += 64) {
     const int kl = k0 + lane;
     BpRecord v{};
-    if (kl < A.vc) v = bp_record(A, kl, Px, Py, Pxf, Pyf, g.L, false);
+    if (kl < A.vc) v = bp_record(A, kl, Px, Py, g.L, false);
     if (!__any(v.key)) continue;
     rest = rest || __any(v.key == 1);
     int first[11];
@@ -1466,7 +1488,7 @@ __device__ __forceinline__ void bp_packed_body(const BpArgs<T>& A, int col, floa
     for (int k0 = 0; k0 < A.vc; k0 += 64) {
       const int kl = k0 + lane;
       BpRecord v{};
-      if (kl < A.vc) v = bp_record(A, kl, Px, Py, Pxf, Pyf, g.L, exact);
+      if (kl < A.vc) v = bp_record(A, kl, Px, Py, g.L, exact);
       int first[11];
       const int pos = sort_classes(v.key, first), n = first[2];
       if (!n) continue;
@@ -1550,9 +1572,8 @@ __device__ __forceinline__ void bp_win_body(const BpArgs<T>& A, int col, float* 
     return;
   }
   for (int z = lane; z < d.ZN; z += 64) lacc[z] = 0.f;
-  const double Px = ((double)x - c64.ocx) * c64.dx;
-  const double Py = ((double)y - c64.ocy) * c64.dx;
-  const float Pxf = (float)Px, Pyf = (float)Py;
+  const double Px = held(((double)x - c64.ocx) * c64.dx);
+  const double Py = held(((double)y - c64.ocy) * c64.dx);
   const float DNVh = (float)d.DNV - 0.5f;
   const int DNV = d.DNV;
   const uint32_t frame = (uint32_t)(d.DNU * d.DNV);
@@ -1561,7 +1582,7 @@ __device__ __forceinline__ void bp_win_body(const BpArgs<T>& A, int col, float* 
     BpView q{};
     int q_z0 = 0, q_z1 = -1;
     if (kl < A.vc) {
-      q = bp_view(A, A.vb + kl * A.vs, Px, Py, Pxf, Pyf);
+      q = bp_view(A, A.vb + kl * A.vs, Px, Py);
       bp_window(d, q, q_z0, q_z1);
     }
     uint64_t live = __ballot(q.uvis && q_z0 <= q_z1);
@@ -1587,7 +1608,7 @@ __device__ __forceinline__ void bp_win_body(const BpArgs<T>& A, int col, float* 
           const float Wu = nu == 1 ? wu0 : wu0 + (float)(nu - 2) + fh;
           lacc[z] = fmaf(cosVal, Wu * (vhi - vlo), lacc[z]);
         } else {
-          lacc[z] = fmaf(cosVal, bp_cell_sum(pp, u0, nu, wu0, fh, vlo, vhi, DNV), lacc[z]);
+          lacc[z] = fmaf(cosVal, bp_cell_sum(pp, u0 * DNV, nu, wu0, fh, vlo, vhi, DNV), lacc[z]);
         }
       }
     }
@@ -1605,8 +1626,13 @@ __host__ __device__ constexpr int bp_win_floats(int RC, int sums) {
                         : 0) +
          ((sums + 3) & ~3);
 }
-// Waves per SIMD that the registers of a body leave room for.
-constexpr int bp_waves(int RC) { return RC == 4 ? 5 : RC == 2 || RC == kPacked ? 6 : 7; }
+// Waves per SIMD that a body is compiled for.  One row chunk takes one more in its own kernel (8
+// waves, 64 registers, 8 values spilled; 512^2 x 256: 2.40 ms, 2.47 ms with 7 waves and none);
+// two chunks spill up to 4 values, four 12.  While the FP64 constants of a view's evaluation stood
+// in vector registers (held) they spilled 26, 12 and 24: 2.44 ms.
+constexpr int bp_waves(int RC) {
+  return RC == 4 ? 5 : RC == 2 || RC == kPacked ? 6 : 7;
+}
 template <bool UPDATE, typename T, int RC, bool ONES = false>
 __device__ __forceinline__ void bp_any_win_body(const BpArgs<T>& A, int col, float* lds) {
   if constexpr (RC == kPacked) bp_packed_body<UPDATE, T, ONES>(A, col, lds);

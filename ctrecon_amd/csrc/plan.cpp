@@ -159,6 +159,7 @@ static int build_tables(const ctr_geometry* g, Plan& P, double half = 0.0) {
   const double ocz = (g->ZN - 1.0) * 0.5 - g->imgZCenter / dz;
   d.ocx = (float)ocx; d.ocy = (float)ocy; d.ocz = (float)ocz;
   d.dx = (float)dx; d.dz = (float)dz;
+  d.idz = 1.f / d.dz;
   const std::vector<double> bx = boundaries(g->xds, DNU), by = boundaries(g->yds, DNU),
                             bz = boundaries(g->zds, DNV);
 
