@@ -72,9 +72,9 @@ struct ctr_batch {
   std::vector<int> fpTotal;
   // back-projection work lists by class: c = 1..4 z groups per lane, c = 0 the windowed form
   // with staged rows (one wave per column over all z), c = 5 that of packed views, c = 6 that
-  // without staged rows, each scan in the form that its own solver runs; the scans of the
-  // class, and per subset step their items (and timing copies with a zero column sum)
-  static constexpr int kClasses = 7, kPackedClass = 5, kUnstagedClass = 6;
+  // without staged rows, c = 7 that of rows staged view by view, each scan in the form that its
+  // own solver runs; the scans of the class, and per subset step their items (and timing copies with a zero column sum)
+  static constexpr int kClasses = 8, kPackedClass = 5, kUnstagedClass = 6, kPlainClass = 7;
   std::vector<int> clsScans[kClasses];
   Mem bpItems[kClasses], tuneBpItems[kClasses];
   std::vector<int> bpTotal[kClasses];
@@ -109,7 +109,10 @@ bool windowed(int c) { return c < 1 || c > 4; }
 int scan_zg(const ctr_batch& B, const Plan& P) {
   if (P.d.ZN <= kWinMaxZ) {  // a windowed form, whatever zg
     const int rc = bp_shape(P, false).rc;
-    return rc == kPacked ? ctr_batch::kPackedClass : rc == 0 ? ctr_batch::kUnstagedClass : 0;
+    return rc == kPacked  ? ctr_batch::kPackedClass
+           : rc == kPlain ? ctr_batch::kPlainClass
+           : rc == 0      ? ctr_batch::kUnstagedClass
+                          : 0;
   }
   return (B.zg > 0 && B.zg < kZgWindow) ? B.zg : std::min(4, (P.d.ZN + 63) / 64);
 }
@@ -124,7 +127,7 @@ int build_tables(ctr_batch& B) {
   for (int c = 0; c < B.kClasses; ++c) {
     B.clsScans[c].clear();
     B.bpTotal[c].assign(S, 0);
-    B.win[c] = {c == B.kPackedClass ? kPacked : 0, 0};
+    B.win[c] = {c == B.kPackedClass ? kPacked : c == B.kPlainClass ? kPlain : 0, 0};
   }
   for (int i = 0; i < n; ++i) {
     const int c = scan_zg(B, *B.scans[i]->P);

@@ -66,6 +66,8 @@ struct Dims {
   double B0_64, dB_64;   // row boundary 0 and the mean spacing, FP64
   int even_rows;         // 1: every row boundary is B0 + v dB to within the FP32 rounding of
                          // row positions relative to the source
+  int coarse;            // 1: about half of the voxels' shadows or more are over two rows high
+                         // or over four columns wide (bp_shape)
   int fine;              // 1: some footprint can cover more than four cells in-plane or be more
                          // than two cells high (fp_body's FINE); not for under four voxels
 };
@@ -293,9 +295,10 @@ int launch_bp_batch(const BpBatchItem<T>* items, int nscan, int total, int zg, i
 // when a scan needs the unstaged form; kPacked for a list of packed scans)
 int bp_row_chunks(int DNU, int DNV);
 int bp_pack_lanes(const Plan& P, bool matched);
-constexpr int kPacked = -1, kPackSums = 1536;
+constexpr int kPlain = -2, kPacked = -1, kPackSums = 1536;
 static_assert(kPackSums <= kWinMaxZ, "a packed wave's sums");
-// A windowed back projector of a plan: rc and sums as above (ZN <= kWinMaxZ).
+// A windowed back projector of a plan: rc and sums as above, kPlain for rows staged view by view
+// (ZN <= kWinMaxZ).
 struct BpShape {
   int rc, sums;
 };

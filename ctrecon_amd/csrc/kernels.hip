@@ -1347,6 +1347,118 @@ __device__ __forceinline__ void bp_staged_body(const BpArgs<T>& A, int col, floa
   for (int z = lane; z < d.ZN; z += 64) bp_store<UPDATE>(A, vcol, col, z, lacc[z]);
 }
 
+// Staged rows view by view, in one loop for any number of columns and rows: short, for where the
+// classes do not pay (bp_shape).  Otherwise as bp_staged_body; rows that are not finite are read
+// only by the shadows that they lie in.
+template <bool UPDATE, typename T, int RC, bool ONES = false>
+__device__ __forceinline__ void bp_plain_body(const BpArgs<T>& A, int col, float* lds) {
+#pragma clang fp contract(off)
+  const Dims& d = A.d;
+  const BpConsts64& c64 = A.c64;
+  const int lane = threadIdx.x & 63;
+  if (col >= d.XN * d.YN) return;
+  const int y = col / d.XN, x = col - y * d.XN;
+  CTR_GLOBAL float* vcol = gp(A.vol) + (size_t)col * d.ZN;
+  if (gp(A.mask)[col] != 1) {
+    if constexpr (!UPDATE) {
+      for (int z = lane; z < d.ZN; z += 64) vcol[z] = 0.f;
+    }
+    return;
+  }
+  float* rows = lds;
+  float4* rec = reinterpret_cast<float4*>(lds + kRowsLds<RC>);  // [64][2]
+  float* lacc = lds + kStagedF<RC>;
+  for (int z = lane; z < d.ZN; z += 64) lacc[z] = 0.f;
+  const int DNV = d.DNV;
+  int row[RC], slot[RC];
+  stage_rows<RC>(rows, DNV, lane, row, slot);
+  const double Px = held(((double)x - c64.ocx) * c64.dx);
+  const double Py = held(((double)y - c64.ocy) * c64.dx);
+  const int frame = d.DNU * DNV;
+  for (int k0 = 0; k0 < A.vc; k0 += 64) {
+    const int kl = k0 + lane;
+    BpRecord v{};
+    if (kl < A.vc) v = bp_record(A, kl, Px, Py, 64, true);
+    const uint64_t m = __ballot(v.key != 0);
+    if (!m) continue;
+    const int nu = __float_as_int(v.w.w);
+    const float wx = v.w.x, wl = v.w.x * v.w.z;
+    if (v.key) {
+      rec[2 * lane] = v.r;
+      rec[2 * lane + 1] = make_float4(v.w.x * v.w.y, nu > 1 ? (nu == 2 ? wl : wx) : 0.f,
+                                      nu > 2 ? (nu == 3 ? wl : wx) : 0.f,
+                                      nu > 3 ? (nu == 4 ? wl : wx) : 0.f);
+    }
+    const int q_o = lane * frame + v.o;
+    const Buf<T> P(A.prj + (size_t)k0 * frame, (uint32_t)min(64, A.vc - k0) * (uint32_t)frame);
+    struct Set {
+      uint32_t y[4][RC];
+    };
+    auto fetch = [&](int j, Set& f) {
+      if constexpr (ONES) return;
+      const int o = __builtin_amdgcn_readlane(q_o, j), n = __builtin_amdgcn_readlane(nu, j);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int c = 0; c < RC; ++c) f.y[i][c] = P.at_bits(row[c], o + min(i, n - 1) * DNV);
+    };
+    auto use = [&](int j, const Set& f) {
+      const float4 r = rec[2 * j], w = rec[2 * j + 1];
+      const int n = __builtin_amdgcn_readlane(nu, j);
+      const float wu[4] = {w.x, w.y, w.z, w.w};
+      float R[RC];
+#pragma unroll
+      for (int c = 0; c < RC; ++c) {
+        R[c] = wu[0] * (ONES ? 1.f : Buf<T>::widen(f.y[0][c]));
+#pragma unroll
+        for (int i = 1; i < 4; ++i)
+          R[c] = fmaf(wu[i], ONES ? 1.f : Buf<T>::widen(f.y[i][c]), R[c]);
+      }
+      if (n > 4) {
+        const int o = __builtin_amdgcn_readlane(q_o, j);
+        const float wj = rdl(wx, j), lj = rdl(wl, j);
+#pragma unroll 4
+        for (int i = 4; i < n; ++i)
+#pragma unroll
+          for (int c = 0; c < RC; ++c)
+            R[c] = fmaf(i == n - 1 ? lj : wj,
+                        ONES ? 1.f : Buf<T>::widen(P.at_bits(row[c], o + i * DNV)), R[c]);
+      }
+      bool bad = false;
+#pragma unroll
+      for (int c = 0; c < RC; ++c) {
+        rows[slot[c]] = R[c];
+        bad = bad || not_finite(R[c]);
+      }
+      const float s = rdl(v.r.y, j);
+      const int zf = __builtin_amdgcn_readlane(v.z0, j);
+      const int zn = __builtin_amdgcn_readlane(v.z1, j) - zf;
+      const float* R0 = rows + kPadRows;
+      float* a = lacc + zf;
+      if (s > kTaps5 || __any(bad)) {
+        for (int zz = lane; zz <= zn; zz += 64) {
+          if constexpr (ONES) {
+            // every row of the shadow holds R
+            const float t = fmaf((float)zz, r.y, r.x), dZ = fmaf((float)zz, d.dz, r.z);
+            const float h = fmaxf(fminf(t + r.y, (float)DNV) - fmaxf(t, 0.f), 0.f);
+            a[zz] = fmaf(__builtin_amdgcn_sqrtf(fmaf(dZ, dZ, r.w)), R[0] * h, a[zz]);
+          } else {
+            a[zz] = bp_voxel<0>(d, r, (float)zz, R0, a[zz]);
+          }
+        }
+      } else if (s > 2.f) {
+        for (int zz = lane; zz <= zn; zz += 64)
+          a[zz] = bp_voxel<5>(d, r, (float)zz, R0, a[zz]);
+      } else {
+        for (int zz = lane; zz <= zn; zz += 64)
+          a[zz] = bp_voxel<3>(d, r, (float)zz, R0, a[zz]);
+      }
+    };
+    pipelined<Set>(m, fetch, use);
+  }
+  for (int z = lane; z < d.ZN; z += 64) bp_store<UPDATE>(A, vcol, col, z, lacc[z]);
+}
+
 // Staged rows with several views at a time, for detectors of few rows (bp_pack_lanes): the wave
 // is split into G = 64 / L groups of L lanes, as many as a view's rows and its window of a
 // column take, and each group takes its own view of a class, with its own rows and column sums
@@ -1616,11 +1728,12 @@ __device__ __forceinline__ void bp_win_body(const BpArgs<T>& A, int col, float* 
   for (int z = lane; z < d.ZN; z += 64) bp_store<UPDATE>(A, vcol, col, z, lacc[z]);
 }
 
-// The windowed body with staged rows (RC = 1, 2, 4), of packed views (kPacked) or without
-// either (0); lds: bp_win_floats of this wave, sums = the floats of its column sums.
+// The windowed body with staged rows (RC = 1, 2, 4), of packed views (kPacked), of rows staged
+// view by view (kPlain: one row chunk) or without any (0);
+// lds: bp_win_floats of this wave, sums = the floats of its column sums.
 __host__ __device__ constexpr int bp_win_floats(int RC, int sums) {
   return (RC == kPacked ? kPackF
-          : RC == 1     ? kStagedF<1>
+          : RC == 1 || RC == kPlain ? kStagedF<1>
           : RC == 2     ? kStagedF<2>
           : RC == 4     ? kStagedF<4>
                         : 0) +
@@ -1635,7 +1748,8 @@ constexpr int bp_waves(int RC) {
 }
 template <bool UPDATE, typename T, int RC, bool ONES = false>
 __device__ __forceinline__ void bp_any_win_body(const BpArgs<T>& A, int col, float* lds) {
-  if constexpr (RC == kPacked) bp_packed_body<UPDATE, T, ONES>(A, col, lds);
+  if constexpr (RC == kPlain) bp_plain_body<UPDATE, T, 1, ONES>(A, col, lds);
+  else if constexpr (RC == kPacked) bp_packed_body<UPDATE, T, ONES>(A, col, lds);
   else if constexpr (RC > 0) bp_staged_body<UPDATE, T, RC, ONES>(A, col, lds);
   else bp_win_body<UPDATE, T, ONES>(A, col, lds);
 }
@@ -2927,10 +3041,17 @@ int bp_pack_lanes(const Plan& P, bool matched) {
   return G >= 2 ? 64 / G : 0;
 }
 
+// The classes' second loop does not pay where it takes about half of the views or more
+// (Dims::coarse): 128^2 x 64, 100 views of 888 x 64, 2.8 mm voxels 323 us, 272 us view by view;
+// 1.4 mm 192 us, 159 us; 1 mm (not coarse) 93 us, 152 us; more rows gain nothing.
 BpShape bp_shape(const Plan& P, bool matched) {
-  const int L = bp_pack_lanes(P, matched), ZN4 = (P.d.ZN + 3) & ~3;
+  const int ZN4 = (P.d.ZN + 3) & ~3, rc = bp_row_chunks(P.d.DNU, P.d.DNV);
+  const BpShape staged{rc, ZN4};
+  const int L = bp_pack_lanes(P, matched);
   if (L) return {kPacked, 64 / L * ZN4};
-  return {bp_row_chunks(P.d.DNU, P.d.DNV), ZN4};
+  if (matched || !rc) return staged;
+  if (rc == 1 && P.d.coarse) return {kPlain, ZN4};
+  return staged;
 }
 
 // Row chunks (of 64) a staged wave holds for a detector, 0 for the unstaged form: over 256
@@ -2950,6 +3071,7 @@ int launch_bp_ones(const Plan& P, float* vol, int vb, int vs, int vc, hipStream_
   hipLaunchKernelGGL(bp_win_ones_kernel<RC>, wgrid, dim3(kBlock), lds, st, A, sh.sums)
   switch (sh.rc) {
     case kPacked: CTR_BPO(kPacked); break;
+    case kPlain: CTR_BPO(kPlain); break;
     case 1: CTR_BPO(1); break;
     case 2: CTR_BPO(2); break;
     case 4: CTR_BPO(4); break;
@@ -3048,6 +3170,7 @@ int launch_bp(const Plan& P, const T* prj, float* vol, int vb, int vs, int vc, i
   } while (0)
     switch (sh.rc) {
       case kPacked: CTR_BPW(kPacked); break;
+    case kPlain: CTR_BPW(kPlain); break;
       case 1: CTR_BPW(1); break;
       case 2: CTR_BPW(2); break;
       case 4: CTR_BPW(4); break;
@@ -3141,6 +3264,7 @@ int launch_bp_batch_win(const BpBatchItem<T>* items, int nscan, int total, int s
   } while (0)
   switch (rc) {
     case kPacked: CTR_BPBW(kPacked); break;
+    case kPlain: CTR_BPBW(kPlain); break;
     case 1: CTR_BPBW(1); break;
     case 2: CTR_BPBW(2); break;
     case 4: CTR_BPBW(4); break;
