@@ -72,8 +72,10 @@ struct ctr_batch {
   std::vector<int> fpTotal;
   // back-projection work lists by class: c = 1..4 z groups per lane, c = 0 the windowed form
   // with staged rows (one wave per column over all z), c = 5 that of packed views, c = 6 that
-  // without staged rows, c = 7 that of rows staged view by view, each scan in the form that its
-  // own solver runs; the scans of the class, and per subset step their items (and timing copies with a zero column sum)
+  // without staged rows, c = 7 that of rows staged view by view: in each subset step a scan runs
+  // the form that its own solver runs for as many views; the scans of the class, and per subset
+  // step their items, empty where the step's form is another (and timing copies with a zero
+  // column sum)
   static constexpr int kClasses = 8, kPackedClass = 5, kUnstagedClass = 6, kPlainClass = 7;
   std::vector<int> clsScans[kClasses];
   Mem bpItems[kClasses], tuneBpItems[kClasses];
@@ -105,12 +107,12 @@ constexpr int kZgWindow = 5;
 
 bool windowed(int c) { return c < 1 || c > 4; }
 
-// back-projection class of a scan
-int scan_zg(const ctr_batch& B, const Plan& P) {
+// back-projection class of a scan in a subset of vc views
+int scan_class(const ctr_batch& B, const Plan& P, int vc) {
   if (P.d.ZN <= kWinMaxZ) {  // a windowed form, whatever zg
-    const int rc = bp_shape(P, false).rc;
+    const int rc = bp_shape(P, false, vc).rc;
     return rc == kPacked  ? ctr_batch::kPackedClass
-           : rc == kPlain ? ctr_batch::kPlainClass
+           : rc <= kPlain ? ctr_batch::kPlainClass
            : rc == 0      ? ctr_batch::kUnstagedClass
                           : 0;
   }
@@ -129,13 +131,16 @@ int build_tables(ctr_batch& B) {
     B.bpTotal[c].assign(S, 0);
     B.win[c] = {c == B.kPackedClass ? kPacked : c == B.kPlainClass ? kPlain : 0, 0};
   }
-  for (int i = 0; i < n; ++i) {
-    const int c = scan_zg(B, *B.scans[i]->P);
-    B.clsScans[c].push_back(i);
-    const BpShape sh = bp_shape(*B.scans[i]->P, false);
-    if (c == 0) B.win[c].rc = std::max(B.win[c].rc, sh.rc);
-    B.win[c].sums = std::max(B.win[c].sums, sh.sums);
-  }
+  for (int i = 0; i < n; ++i)
+    for (int s = 0; s < S; ++s) {
+      const Plan& P = *B.scans[i]->P;
+      const int vc = vcount(P, s, S), c = scan_class(B, P, vc);
+      if (B.clsScans[c].empty() || B.clsScans[c].back() != i) B.clsScans[c].push_back(i);
+      const BpShape sh = bp_shape(P, false, vc);
+      if (c == 0) B.win[c].rc = std::max(B.win[c].rc, sh.rc);
+      else if (c == B.kPlainClass) B.win[c].rc = std::min(B.win[c].rc, sh.rc);
+      B.win[c].sums = std::max(B.win[c].sums, sh.sums);
+    }
   auto up = [&](Mem& m, const void* src, size_t bytes) -> int {
     if (m.p) {
       (void)hipFree(m.p);
@@ -182,7 +187,7 @@ int build_tables(ctr_batch& B) {
         b.begin = bb;
         b.colBlocks = (P.d.XN * P.d.YN + 3) / 4;
         const int zblocks = windowed(cz) ? 1 : (P.d.ZN + 64 * cz - 1) / (64 * cz);
-        bb += vc > 0 ? b.colBlocks * zblocks : 0;
+        bb += vc > 0 && scan_class(B, P, vc) == cz ? b.colBlocks * zblocks : 0;
         BpBatchItem<T>& t = tbp[(size_t)s * m + j];
         t = b;
         t.a.invCol = B.zeros.f();  // x += acc * 0: timing runs leave the iterate unchanged

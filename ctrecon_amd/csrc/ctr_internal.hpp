@@ -297,12 +297,12 @@ int bp_row_chunks(int DNU, int DNV);
 int bp_pack_lanes(const Plan& P, bool matched);
 constexpr int kPlain = -2, kPacked = -1, kPackSums = 1536;
 static_assert(kPackSums <= kWinMaxZ, "a packed wave's sums");
-// A windowed back projector of a plan: rc and sums as above, kPlain for rows staged view by view
-// (ZN <= kWinMaxZ).
+// The windowed back projector of vc views: rc and sums as above; rc kPlain, kPlain - 1, kPlain - 2
+// for one, two or four chunks of rows staged view by view (ZN <= kWinMaxZ).
 struct BpShape {
   int rc, sums;
 };
-BpShape bp_shape(const Plan& P, bool matched);
+BpShape bp_shape(const Plan& P, bool matched, int vc);
 template <typename T>
 int launch_bp_batch_win(const BpBatchItem<T>* items, int nscan, int total, int sums, int rc,
                         int grid, int strided, hipStream_t st);

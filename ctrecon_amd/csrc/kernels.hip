@@ -982,6 +982,17 @@ __device__ __forceinline__ void bp_window(const Dims& d, const BpView& q, int& z
   z1 = min((int)ceilf(zb + 1e-2f) - 1, d.ZN - 1);
 }
 
+// fetch(j, set), use(j, set) over the set bits j of m, one after the other.
+template <typename Set, typename Fetch, typename Use>
+__device__ __forceinline__ void in_turn(uint64_t m, Fetch fetch, Use use) {
+  for (; m; m &= m - 1) {
+    const int j = __builtin_ctzll(m);
+    Set x;
+    fetch(j, x);
+    use(j, x);
+  }
+}
+
 // Runs f(slot, j) ... over the set bits j of m with the fetches of the next bit in flight:
 // fetch(j, set) loads into one of two register sets, use(j, set) consumes it.
 template <typename Set, typename Fetch, typename Use>
@@ -1454,7 +1465,9 @@ __device__ __forceinline__ void bp_plain_body(const BpArgs<T>& A, int col, float
           a[zz] = bp_voxel<3>(d, r, (float)zz, R0, a[zz]);
       }
     };
-    pipelined<Set>(m, fetch, use);
+    // (more row chunks run for a view or two only, and take the registers of one set)
+    if constexpr (RC == 1) pipelined<Set>(m, fetch, use);
+    else in_turn<Set>(m, fetch, use);
   }
   for (int z = lane; z < d.ZN; z += 64) bp_store<UPDATE>(A, vcol, col, z, lacc[z]);
 }
@@ -1729,26 +1742,29 @@ __device__ __forceinline__ void bp_win_body(const BpArgs<T>& A, int col, float* 
 }
 
 // The windowed body with staged rows (RC = 1, 2, 4), of packed views (kPacked), of rows staged
-// view by view (kPlain: one row chunk) or without any (0);
+// view by view (kPlain, kPlain - 1, kPlain - 2: 1, 2, 4 row chunks) or without any (0);
 // lds: bp_win_floats of this wave, sums = the floats of its column sums.
 __host__ __device__ constexpr int bp_win_floats(int RC, int sums) {
   return (RC == kPacked ? kPackF
-          : RC == 1 || RC == kPlain ? kStagedF<1>
-          : RC == 2     ? kStagedF<2>
-          : RC == 4     ? kStagedF<4>
+          : RC == 1 || RC == kPlain     ? kStagedF<1>
+          : RC == 2 || RC == kPlain - 1 ? kStagedF<2>
+          : RC == 4 || RC == kPlain - 2 ? kStagedF<4>
                         : 0) +
          ((sums + 3) & ~3);
 }
 // Waves per SIMD that a body is compiled for.  One row chunk takes one more in its own kernel (8
 // waves, 64 registers, 8 values spilled; 512^2 x 256: 2.40 ms, 2.47 ms with 7 waves and none);
 // two chunks spill up to 4 values, four 12.  While the FP64 constants of a view's evaluation stood
-// in vector registers (held) they spilled 26, 12 and 24: 2.44 ms.
+// in vector registers (held) they spilled 26, 12 and 24: 2.44 ms, and 14 us for 11 us where one
+// view of 128^2 x 64 is projected.
 constexpr int bp_waves(int RC) {
   return RC == 4 ? 5 : RC == 2 || RC == kPacked ? 6 : 7;
 }
 template <bool UPDATE, typename T, int RC, bool ONES = false>
 __device__ __forceinline__ void bp_any_win_body(const BpArgs<T>& A, int col, float* lds) {
   if constexpr (RC == kPlain) bp_plain_body<UPDATE, T, 1, ONES>(A, col, lds);
+  else if constexpr (RC == kPlain - 1) bp_plain_body<UPDATE, T, 2, ONES>(A, col, lds);
+  else if constexpr (RC == kPlain - 2) bp_plain_body<UPDATE, T, 4, ONES>(A, col, lds);
   else if constexpr (RC == kPacked) bp_packed_body<UPDATE, T, ONES>(A, col, lds);
   else if constexpr (RC > 0) bp_staged_body<UPDATE, T, RC, ONES>(A, col, lds);
   else bp_win_body<UPDATE, T, ONES>(A, col, lds);
@@ -3041,16 +3057,20 @@ int bp_pack_lanes(const Plan& P, bool matched) {
   return G >= 2 ? 64 / G : 0;
 }
 
-// The classes' second loop does not pay where it takes about half of the views or more
-// (Dims::coarse): 128^2 x 64, 100 views of 888 x 64, 2.8 mm voxels 323 us, 272 us view by view;
-// 1.4 mm 192 us, 159 us; 1 mm (not coarse) 93 us, 152 us; more rows gain nothing.
-BpShape bp_shape(const Plan& P, bool matched) {
+// Packed views need enough of them to pay for a group's own sums: 512^2 x 128, 16 rows, 8 views
+// 223 us, 173 us one view at a time, 16 views 249 us, 255 us (64^3 7.9 us, 7.1 us; 8.4 us, 9.2 us);
+// matched 330 us, 273 us; 381 us, 384 us.  One or two views do not pay for the classes' longer
+// code: 512^2 x 128, 64 rows, one view 123 us, 114 us view by view (160 rows 158 us, 123 us;
+// 64^3 6.7 us, 4.9 us), four views 150 us, 168 us.  Nor do the second loop's views where they are
+// about half of all or more (Dims::coarse): 128^2 x 64, 100 views of 888 x 64, 2.8 mm voxels
+// 323 us, 272 us; 1.4 mm 192 us, 159 us; 1 mm (not coarse) 93 us, 152 us; more rows gain nothing.
+BpShape bp_shape(const Plan& P, bool matched, int vc) {
   const int ZN4 = (P.d.ZN + 3) & ~3, rc = bp_row_chunks(P.d.DNU, P.d.DNV);
   const BpShape staged{rc, ZN4};
-  const int L = bp_pack_lanes(P, matched);
+  const int L = vc >= 16 ? bp_pack_lanes(P, matched) : 0;
   if (L) return {kPacked, 64 / L * ZN4};
   if (matched || !rc) return staged;
-  if (rc == 1 && P.d.coarse) return {kPlain, ZN4};
+  if (vc <= 2 || (rc == 1 && P.d.coarse)) return {kPlain - rc / 2, ZN4};
   return staged;
 }
 
@@ -3065,13 +3085,15 @@ int launch_bp_ones(const Plan& P, float* vol, int vb, int vs, int vc, hipStream_
   if (P.d.ZN > kWinMaxZ) return fail(CTR_ERR_ARG, "bp of ones: columns over the LDS limit");
   const BpArgs<float> A = bp_args<float>(P, nullptr, vol, vb, vs, vc, nullptr, nullptr);
   const dim3 wgrid((P.d.XN * P.d.YN + kWaves - 1) / kWaves);
-  const BpShape sh = bp_shape(P, false);
+  const BpShape sh = bp_shape(P, false, vc);
   const size_t lds = (size_t)kWaves * bp_win_floats(sh.rc, sh.sums) * sizeof(float);
 #define CTR_BPO(RC) \
   hipLaunchKernelGGL(bp_win_ones_kernel<RC>, wgrid, dim3(kBlock), lds, st, A, sh.sums)
   switch (sh.rc) {
     case kPacked: CTR_BPO(kPacked); break;
     case kPlain: CTR_BPO(kPlain); break;
+    case kPlain - 1: CTR_BPO(kPlain - 1); break;
+    case kPlain - 2: CTR_BPO(kPlain - 2); break;
     case 1: CTR_BPO(1); break;
     case 2: CTR_BPO(2); break;
     case 4: CTR_BPO(4); break;
@@ -3090,7 +3112,7 @@ int launch_bp(const Plan& P, const T* prj, float* vol, int vb, int vs, int vc, i
     if constexpr (!std::is_same<T, float>::value) {
       return fail(CTR_ERR_ARG, "the matched back projector reads the FP32 scaled sinogram");
     } else {
-      const BpShape sh = bp_shape(P, true);
+      const BpShape sh = bp_shape(P, true, vc);
       const size_t slds = (size_t)kWaves * bp_matched_floats(sh.rc, sh.sums) * sizeof(float);
       if (P.d.even_rows && sh.rc != 0 && P.d.ZN <= kWinMaxZ && slds <= 65536) {
         const dim3 wgrid((P.d.XN * P.d.YN + kWaves - 1) / kWaves);
@@ -3157,7 +3179,7 @@ int launch_bp(const Plan& P, const T* prj, float* vol, int vb, int vs, int vc, i
                                  accumulate ? shadow : nullptr);
   if (P.d.ZN <= kWinMaxZ) {
     const dim3 wgrid((P.d.XN * P.d.YN + kWaves - 1) / kWaves);
-    const BpShape sh = bp_shape(P, false);
+    const BpShape sh = bp_shape(P, false, vc);
     const size_t lds = (size_t)kWaves * bp_win_floats(sh.rc, sh.sums) * sizeof(float);
 #define CTR_BPW(RC)                                                                           \
   do {                                                                                        \
@@ -3171,6 +3193,8 @@ int launch_bp(const Plan& P, const T* prj, float* vol, int vb, int vs, int vc, i
     switch (sh.rc) {
       case kPacked: CTR_BPW(kPacked); break;
     case kPlain: CTR_BPW(kPlain); break;
+    case kPlain - 1: CTR_BPW(kPlain - 1); break;
+    case kPlain - 2: CTR_BPW(kPlain - 2); break;
       case 1: CTR_BPW(1); break;
       case 2: CTR_BPW(2); break;
       case 4: CTR_BPW(4); break;
@@ -3265,6 +3289,8 @@ int launch_bp_batch_win(const BpBatchItem<T>* items, int nscan, int total, int s
   switch (rc) {
     case kPacked: CTR_BPBW(kPacked); break;
     case kPlain: CTR_BPBW(kPlain); break;
+    case kPlain - 1: CTR_BPBW(kPlain - 1); break;
+    case kPlain - 2: CTR_BPBW(kPlain - 2); break;
     case 1: CTR_BPBW(1); break;
     case 2: CTR_BPBW(2); break;
     case 4: CTR_BPBW(4); break;
