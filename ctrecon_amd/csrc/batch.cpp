@@ -489,7 +489,7 @@ int ctr_batch_create(ctr_plan* const* plans, int nscan, float* const* d_x,
     CTR_HIP(hipStreamSynchronize(B->st));  // before `ones` is freed
     B->scans.push_back(std::move(c));
   }
-  B->fine = B->fine && minNV >= 4;
+  B->fine = B->fine && fine_volume(minNV) && fine_volume(maxNV);
   (void)hipEventRecord(e1, B->st);
   CTR_HIP(hipEventSynchronize(e1));
   float ms = 0;

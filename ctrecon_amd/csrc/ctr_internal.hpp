@@ -69,8 +69,16 @@ struct Dims {
   int coarse;            // 1: about half of the voxels' shadows or more are over two rows high
                          // or over four columns wide (bp_shape)
   int fine;              // 1: some footprint can cover more than four cells in-plane or be more
-                         // than two cells high (fp_body's FINE); not for under four voxels
+                         // than two cells high (fp_body's FINE); only where fine_volume
 };
+
+// Elements that the forward projector's buffer loads may lie before a volume's first.
+constexpr unsigned kFarRun = 256;
+// Volumes that its form for fine voxels takes: at least one run of four voxels, and in either type
+// within 32-bit byte offsets.
+inline bool fine_volume(long long voxels) {
+  return voxels >= 4 && voxels <= 0xffffffffll / 4 - kFarRun;
+}
 
 // Host copies used by host-side accounting (cone voxel counts).
 struct HostGeo {

@@ -184,6 +184,9 @@ __device__ __forceinline__ void z_run(const Buf<uint16_t>&, const uint16_t* vol,
   }
 }
 
+__device__ __forceinline__ float widened(float v) { return v; }
+__device__ __forceinline__ float widened(uint16_t v) { return __uint_as_float((uint32_t)v << 16); }
+
 // Four z taps from element e of a volume of n (at least four) elements on; past its end 0.
 __device__ __forceinline__ void z_run4(const Buf<float>& V, const float*, int e, int,
                                        float (&a)[4]) {
@@ -284,6 +287,11 @@ __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk
     const float2* me = A.mext + (vp.xmarch ? 0 : d.XN);
     const int NV = d.XN * d.YN * d.ZN;
     const Buf<TV> V(A.vol, (uint32_t)NV);
+    // a volume past the buffer loads' 32-bit byte offsets (with room for a run before its first
+    // element, which their range check has to reject): the general form throughout, by address
+    // (as rows of infinite height)
+    const bool far = !FINE && (uint32_t)NV > 0xffffffffu / (uint32_t)sizeof(TV) - kFarRun;
+    const float dBmax = far ? __builtin_inff() : d.dBmax;
     const CTR_GLOBAL float* maskf = gp(A.maskf);
     float acc = 0.f;
     // one slice in the general form (any number of cells and taps; reads the footprint's cells
@@ -305,7 +313,7 @@ __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk
         else
           for (int ik = 0; ik < nk; ++ik)
             g = fmaf(fminf(te, (float)(k0 + ik + 1)) - fmaxf(t, (float)(k0 + ik)),
-                     (float)V[e + ik], g);
+                     widened(gp(A.vol)[e + ik]), g);
         acc = fmaf(wy, g, acc);
         e += cS;
         mo += mC;
@@ -369,7 +377,7 @@ __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk
         if (o.r > 0.f && th > tmin && tl < tmax && (!FINE || n > 0)) {
           q_r = o.r;
           q_nj = FINE ? min(n, 4) : n;
-          const float h = o.r * d.dBmax;
+          const float h = o.r * dBmax;
           const int j0 = FINE ? o.j0 + c0 : o.j0, mo = il * mS + j0 * mC;
           wy0 = o.inv * ((!FINE || c0 == 0 ? o.wj0 : (n == 1 ? o.wjl : 1.f)) * maskf[mo]);
           if (n >= 2) wy1 = o.inv * ((n == 2 ? o.wjl : 1.f) * maskf[mo + mC]);
@@ -388,11 +396,11 @@ __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk
             q_last = floor_i(fmaf(o.r, Btop, azf)) - q_kb + 2;
             if (q_last > 63) cls |= 2;
             gen = gen || q_last > 127 ||
-                  q_e + (FINE ? q_kb : 0) + (max(q_nj, 2) - 1) * cS + 128 > NV;
+                  q_e + (FINE ? q_kb : 0) > NV - 128 - (max(q_nj, 2) - 1) * cS;
             if (FINE && !gen) q_e += q_kb;
           } else {
             // a run's elements stay inside the array: not on its last column
-            gen = gen || e + (q_nj - 1) * cS + d.ZN + 4 > NV;
+            gen = gen || e > NV - (d.ZN + 4) - (q_nj - 1) * cS;
           }
           cls |= gen ? 8 : 0;
         }

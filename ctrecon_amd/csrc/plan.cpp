@@ -217,7 +217,7 @@ static int build_tables(const ctr_geometry* g, Plan& P, double half = 0.0) {
     const double far = 1.0 + 0.5 * std::max(g->XN, g->YN) * dx / sid;
     const bool fine = d.dBmax * (sid / S2D) * far > 2.0 ||
                       std::fabs(dbeta) * sid / dx * std::sqrt(2.0) * far > 3.0;
-    d.fine = fine && (long long)g->XN * g->YN * g->ZN >= 4 ? 1 : 0;
+    d.fine = fine && fine_volume((long long)g->XN * g->YN * g->ZN) ? 1 : 0;
     // shadows at the axis: rows high, and columns wide at right angles (0.9 of it on average)
     d.coarse = dz * S2D / (ddv * sid) > 2.0 || dx / (sid * std::fabs(dbeta)) > 4.0 ? 1 : 0;
     P.bc.S = (float)(S2D / ddv);
