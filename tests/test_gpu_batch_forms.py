@@ -78,3 +78,36 @@ def test_tuning_of_earlier_kernels_is_not_used(tmp_path, monkeypatch, gpu_plan_f
     key, values = line.split("\t")
     cache.write_text(key[key.index("gfx"):] + "\t" + values + "\n")
     assert info()["from_cache"] == 0
+
+
+@pytest.mark.parametrize("storage", ["f32", "bf16"])
+def test_tall_columns_in_z_groups(storage, gpu_plan_factory):
+    """Columns over 2048 voxels: every number of z groups per lane adds a voxel's views in the same
+    order as the scan's own solver (equal bits), beside a scan of short columns."""
+    from ctrecon_amd.batch import Batch
+    from ctrecon_amd.plan import DeviceArray, Plan
+
+    print(f"[batch, tall columns] {storage}", flush=True)
+    scans = [_scan(64, nxy=4, nz=2100), _scan(64), _scan(64, nxy=3, nz=2309, views=17)]
+    ref = []
+    for g, b in scans:
+        p, x = Plan(g, 0), DeviceArray(g.vol_shape)
+        p.set_storage(storage)
+        x.zero()
+        p.os_sart(x, DeviceArray.from_host(b), SUBSETS, 2)
+        ref.append(x.get())
+    plans = [Plan(g, 0) for g, _ in scans]
+    for p in plans:
+        p.set_storage(storage)
+    bs = [DeviceArray.from_host(b) for _, b in scans]
+    xs = [DeviceArray(g.vol_shape) for g, _ in scans]
+    B = Batch(plans, xs, bs, SUBSETS)
+    for zg in (0, 1, 2, 3, 4, 5):
+        for grid, strided in ((0, False), (64, False), (64, True)):
+            B.set_tuning(True, grid, zg, grid, strided, strided)
+            for x in xs:
+                x.zero()
+            B.sweeps(2)
+            for i, x in enumerate(xs):
+                assert np.array_equal(x.get(), ref[i]), (zg, grid, strided, i)
+    B.close()
