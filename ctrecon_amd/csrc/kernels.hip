@@ -221,14 +221,14 @@ __device__ __forceinline__ void z_run4(const Buf<uint16_t>&, const uint16_t* vol
 // neighbouring elements costs the texture unit about a quarter of a 2- or 3-dword gather per
 // lane, which bound this kernel at 97% of that unit), combines the cells per z into LDS,
 // and every row takes its two or three taps there; the next slice's runs load meanwhile.
-// What bounds it then is VALU issue (0.95 of the chip's rate, about 22 instructions per
+// What bounds it then is VALU issue (0.97 of the chip's rate, about 22 instructions per
 // wave and slice).  512^2 x 256, 197 views of 888 x 64: 4.06 ms with a gather per cell and
-// lane, 3.00 ms with slices in classes, 2.27 ms with runs and the deal of
-// xcd_chunked_block; BF16 4.19 ms, 3.32 ms, 1.97 ms.
+// lane, 3.00 ms with slices in classes, 2.28 ms with runs and the deal of
+// xcd_chunked_block; BF16 4.19 ms, 3.32 ms, 1.99 ms.
 //
 // Groups (fewer than 64 rows to a column) gather each cell's taps as one load per lane:
 // 64^3, 720 views of 256 x 16, 212 us one thread per ray with its own FP64 footprints,
-// 88 us with four columns per wave.
+// 87 us with four columns per wave.
 //
 // FINE (Dims::fine, fine voxels or wide detector columns): slices of more than four cells take
 // one pass per four, and those whose rows are more than two cells high four taps to a load,
@@ -1062,11 +1062,11 @@ __device__ __forceinline__ void pipelined_n(int n, Fetch fetch, Use use) {
 // takes the three rows that its shadow [T, T + s] can overlap, without clamps.
 // Views of more than four columns, or whose shadows are taller than two rows (key 1), follow in
 // a second loop: any number of columns, five rows, or the shadow's own rows.
-// Bound by VALU issue (0.96 of the chip's rate).  512^2 x 256, 197 views of 888 x 64:
-// 3.76 ms with the views in order, four column loads and two-row clamps for each, 2.46 ms
-// (BF16 sinogram 3.85 ms, 2.46 ms); 256^2 x 128 of 1.4 mm, where most views are of the second
-// kind, 1.17 ms, 1.06 ms, of 1 mm 1.09 ms, 0.89 ms; 277^2 x 165, 164 views of 611 x 80 in BF16,
-// without staged rows 1.78 ms, with two chunks of rows 0.69 ms.
+// Bound by VALU issue (0.98 of the chip's rate).  512^2 x 256, 197 views of 888 x 64:
+// 3.76 ms with the views in order, four column loads and two-row clamps for each, 2.40 ms
+// (BF16 sinogram 3.85 ms, 2.43 ms); 256^2 x 128 of 1 mm 0.92 ms, 0.61 ms; 277^2 x 165, 164 views
+// of 611 x 80 in BF16, without staged rows 1.78 ms, with two chunks of rows 0.67 ms.  Grids where
+// most views are of the second kind run view by view (bp_plain_body, bp_shape).
 constexpr int kPadRows = 4, kPadEnd = 5;
 template <int RC>
 constexpr int kRowsLds = 64 * RC + 12;  // zeros, rows, zeros, a slot for idle lanes
@@ -2365,9 +2365,9 @@ struct MatchedCols {
 // the forward projector's weight: w_t = overlap dB / (tr - tl), r cancelling.  Lane l
 // evaluates view k0 + l (columns, T0 and s in FP64); the row sets hold w_t y[u + t][v].
 // Views of more than four columns take further records for the rest.
-// Bound by VALU issue (0.73 of the chip's rate) and the texture unit's row loads.  256^2 x
+// Bound by VALU issue (0.75 of the chip's rate) and the texture unit's row loads.  256^2 x
 // 128, 197 views of 888 x 64: 3.94 ms with a search and a gather of the rows per voxel
-// (bp_matched_win_kernel), 0.90 ms; 512^2 x 256: 18.0 ms, 4.1 ms; 256^2 x 128 of 1.4 mm 5.7 ms,
+// (bp_matched_win_kernel), 0.91 ms; 512^2 x 256: 18.0 ms, 4.1 ms; 256^2 x 128 of 1.4 mm 5.7 ms,
 // 2.2 ms.
 //
 // RC = kPacked: several views at a time, as bp_packed_body.
@@ -2923,7 +2923,7 @@ int check_launch(const char* what) {
 // Lanes per item (log2) of the forward projector for a detector of DNV rows: the least
 // lanes spent per column, each weighed by the instructions it issues per slice -- about 20
 // with one column per wave, 25 in groups, and the FP64 evaluation of a slice (about 130)
-// once per L slices.  16 rows: four columns per wave, 88 us against 212 us one thread per
+// once per L slices.  16 rows: four columns per wave, 87 us against 212 us one thread per
 // ray (64^3, 720 views); 40 rows: one column per wave (24 lanes idle), 0.94 ms against
 // 2.19 ms (301^2 x 143, 234 views); 80 rows: groups of 16 without idle lanes.
 int fp_lanes_log2(int DNV) {
