@@ -244,7 +244,9 @@ __device__ __forceinline__ void z_run4(const Buf<uint16_t>&, const uint16_t* vol
 // A slice wholly inside the volume's z range adds its height times its cells' weights; the
 // others take the weights of the projection itself, so that a ray that grazes the volume by
 // a rounding error has a row sum that matches its projection (no contraction: the
-// instantiations must not round a footprint differently).
+// instantiations must not round a footprint differently).  FINE adds up a slice's weights first,
+// in one pass: sums of 20 x 20 views of 888 x 64, 128^2 x 64 of 0.1 mm, with the columns' sums
+// 7.7 ms in the general form, 1.5 ms with a pass per four cells, 1.05 ms.
 template <bool FUSED, bool COLW, typename TV, typename TO, bool FINE, bool ONES = false>
 __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk, double* slot) {
 #pragma clang fp contract(off)
@@ -376,18 +378,24 @@ __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk
         const int n = FINE ? o.nj - c0 : o.nj;  // cells from c0 on
         if (o.r > 0.f && th > tmin && tl < tmax && (!FINE || n > 0)) {
           q_r = o.r;
-          q_nj = FINE ? min(n, 4) : n;
+          q_nj = FINE ? (ONES ? 1 : min(n, 4)) : n;
           const float h = o.r * dBmax;
           const int j0 = FINE ? o.j0 + c0 : o.j0, mo = il * mS + j0 * mC;
-          wy0 = o.inv * ((!FINE || c0 == 0 ? o.wj0 : (n == 1 ? o.wjl : 1.f)) * maskf[mo]);
-          if (n >= 2) wy1 = o.inv * ((n == 2 ? o.wjl : 1.f) * maskf[mo + mC]);
-          if (n >= 3) wy2 = o.inv * ((n == 3 ? o.wjl : 1.f) * maskf[mo + 2 * mC]);
-          if (n >= 4) wy3 = o.inv * ((!FINE || n == 4 ? o.wjl : 1.f) * maskf[mo + 3 * mC]);
+          if constexpr (ONES && FINE) {  // all of the slice's cells as one
+            float W = o.wj0 * maskf[mo];
+            for (int j = 1; j < n; ++j) W += (j == n - 1 ? o.wjl : 1.f) * maskf[mo + j * mC];
+            wy0 = o.inv * W;
+          } else {
+            wy0 = o.inv * ((!FINE || c0 == 0 ? o.wj0 : (n == 1 ? o.wjl : 1.f)) * maskf[mo]);
+            if (n >= 2) wy1 = o.inv * ((n == 2 ? o.wjl : 1.f) * maskf[mo + mC]);
+            if (n >= 3) wy2 = o.inv * ((n == 3 ? o.wjl : 1.f) * maskf[mo + 2 * mC]);
+            if (n >= 4) wy3 = o.inv * ((!FINE || n == 4 ? o.wjl : 1.f) * maskf[mo + 3 * mC]);
+          }
           const int e = il * sS + j0 * cS;
           q_e = e + vp.azi;
           bool gen = (!FINE && n > 4) || h > 2.f;
           cls = (h > 1.f ? 1 : 0) | (tl < tmin + 0.01f || th > tmax - 0.01f ? 4 : 0);
-          if (FINE && n > 4) cls |= 16;
+          if (FINE && !ONES && n > 4) cls |= 16;
           if constexpr (COLW) {
             // the z run of the item: cells from the first row's on, read up to the last
             // row's third tap; its 64 or 128 elements stay inside the array
@@ -402,6 +410,8 @@ __device__ __forceinline__ void fp_body(const FpArgs<TV, TO>& A, int k, int ublk
             // a run's elements stay inside the array: not on its last column
             gen = gen || e > NV - (d.ZN + 4) - (q_nj - 1) * cS;
           }
+          // ones inside the volume's z range read nothing and take no taps
+          if (ONES && FINE && !(cls & 4)) gen = false;
           cls |= gen ? 8 : 0;
         }
       }
